@@ -46,7 +46,10 @@ extern "C" {
  *                 members have finished). Best for large batches.
  *   PHASES_FIXED  as PHASES, but enqueues exactly max_iters iterations (finished members' blocks exit at once)
  *                 and never reads back: asynchronous and capturable in a HIP graph.
- *   AUTO          PERSISTENT below 256 (member, tile) units, PHASES from there. */
+ *   AUTO          with block_threads = grid_blocks = 0, tiles of 90 x 90 with OL = 4, at most 16 tiles and a stream
+ *                 that is not being captured: resident, one cooperative launch in which a workgroup per tile keeps a
+ *                 member's vectors on chip and members are taken from a queue; asynchronous. Otherwise PERSISTENT
+ *                 below 256 (member, tile) units, PHASES from there. */
 #define MJ_CG_LAUNCH_AUTO 0
 #define MJ_CG_LAUNCH_PERSISTENT 1
 #define MJ_CG_LAUNCH_PHASES 2
@@ -101,8 +104,7 @@ int mj_halo_exchange_adjoint(const mj_halo_plan* plan, const double* ubar_out, c
  * cg2dNorm and 1/max|b|, exchange the first guess, PCG with the 5-point operator aW2d/aS2d/aC2d and the
  * 5-point preconditioner pW/pS/pC in the Fortran update order, stop when err_sq < tol^2 or after max_iters
  * iterations, un-normalise. The halos of x are left as cg2d.F leaves them: the exchanged normalised first guess
- * where the T map writes, the first guess itself elsewhere. Runs all members of a batch in one persistent launch
- * with per-member convergence masks. */
+ * where the T map writes, the first guess itself elsewhere. Every member of a batch converges on its own. */
 typedef struct {
     double firstResidual;  /* sqrt(err_sq) before the first iteration */
     double lastResidual;   /* sqrt(err_sq) at exit */
@@ -112,7 +114,7 @@ typedef struct {
     int32_t converged;     /* 1 if err_sq < tol^2 at exit */
     int32_t outerIters;    /* FP64 residual replacements (mixed precision), 0 for the plain solve */
     int32_t launches;      /* kernel launches of the iteration loop (PHASES modes; the same value in every member's
-                              record, written when the loop ends); 0 for the persistent launch */
+                              record, written when the loop ends); 0 for the persistent and resident launches */
 } mj_cg2d_diag;
 
 typedef struct {

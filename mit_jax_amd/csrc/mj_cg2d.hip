@@ -36,6 +36,7 @@
 #include "mj_cg_sweep.h"
 #include "mj_common.h"
 #include "mj_internal.h"
+#include "mj_resident.h"
 
 namespace mj {
 
@@ -483,7 +484,9 @@ int ensure_cg_tables(mj_halo_plan* P, int sNx, int sNy, int OL) {
         }
         cring[k] = make_int4(csrc, s, lds | (rsg[k] < 0 ? 1 << 30 : 0), 0);
     }
-    if ((rc = up(cring.data(), cring.size() * sizeof(int4), (void**)&P->cg_cring))) return rc;
+    if ((rc = up(cring.data(), cring.size() * sizeof(int4), (void**)&P->cg_cring)) ||
+        (rc = ensure_resident_tables(P, roff, rdst, rsrc, rsg)))
+        return rc;
     P->cg_sNx = sNx;
     P->cg_sNy = sNy;
     P->cg_OL = OL;
@@ -654,6 +657,17 @@ int solve_impl(const mj_halo_plan* plan_T, const mj_cg2d_ops* ops, const double*
     const int mode = launch_mode_of(cfg);
     const int threads = block_threads_of(cfg, mode);
     if (threads < 0) return threads;
+    hipStream_t st = as_stream(stream);
+    if (cfg->launch_mode == MJ_CG_LAUNCH_AUTO && cfg->block_threads == 0 && cfg->grid_blocks == 0 &&
+        resident_fits(P, cfg)) {
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        MJ_HIP(hipStreamIsCapturing(st, &cap));
+        bool done = false;
+        if (cap == hipStreamCaptureStatusNone &&
+            (rc = resident_solve(P, ops, b, x0, x, cg2dNorm, cfg, workspace, workspace_bytes, diag, st, &done)))
+            return rc;
+        if (done) return MJ_OK;
+    }
 
     char* w = (char*)workspace;
     CgDev a{};
@@ -708,7 +722,6 @@ int solve_impl(const mj_halo_plan* plan_T, const mj_cg2d_ops* ops, const double*
     a.grp = (int32_t*)(w + L.grp);
     a.diag = diag;
 
-    hipStream_t st = as_stream(stream);
     hipLaunchKernelGGL(cg2d_init_kernel, dim3(1), dim3(64), 0, st, counter, error, a.nactive, a.B);
     MJ_HIP(hipGetLastError());
     hipLaunchKernelGGL(build_groups_kernel, dim3(1), dim3(1024), 0, st, a.op_index, a.oms, a.B, a.grp, a.ngroups);

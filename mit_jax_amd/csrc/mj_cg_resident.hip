@@ -1,0 +1,837 @@
+// CG2D on gfx950, resident form: the whole solve of a member runs in 13 workgroups (one per tile) that keep every
+// vector of the recurrence on chip, for 90 x 90 tiles.
+//
+// What bounds the other launch shapes: the phase launches stream 11 FP64 vectors per iteration through HBM, and the
+// grid barriers of the persistent launch cost about 10 us each (device-scope fences write back and invalidate the L2s).
+// Here a workgroup of 512 threads owns a (member, tile): x, r, s and z / q are registers (18 points per thread, 256
+// registers at two waves per SIMD), the stencil operand is an LDS tile, aW sits in LDS and the other coefficients
+// stream from L2. What the tiles of a member tell each other per phase is small: the ring values their neighbours read
+// and one or two partial sums. These go through device memory as tagged 8-byte words, {tag, half of a double} (the tag
+// is the number of the exchange): a reader polls a word until its tag arrives, so no fence, no barrier and no separate
+// flag is needed. A round (publish, poll, workgroup barrier) takes 1.5-2.0 us for 1 to 19 members in flight.
+//
+// Members are taken from a queue by groups of workgroups (one per tile), as many groups as fit the device at one
+// workgroup per CU: a member's tiles never wait for another member. Launched cooperatively (all workgroups resident).
+//
+// Arithmetic, operation order and the sums are those of mj_cg2d.hip, bit for bit (see unit_I1, group_phase_B / _C).
+//
+// Thread mapping: lane l of a half-wave holds columns l, l + 32 and l + 64 of six consecutive rows, so the first two
+// steps of the row tree (v[l] + v[l + 64], then + v[l + 32]) are within the thread and 94 % of the lanes work (column
+// pairs on a wave: 70 %). Lanes whose third column would be 90..95 repeat column 89, and the 16th half-wave repeats the
+// 15th's rows: same loads, same values, the same values written to the same places, and counted once in the sums.
+#include <algorithm>
+#include <type_traits>
+
+#include "mj_cg_sweep.h"
+#include "mj_common.h"
+#include "mj_internal.h"
+#include "mj_resident.h"
+
+namespace mj {
+namespace {
+
+constexpr int kN = 90;                    // tile side
+constexpr int kOL = 4, kNX = kN + 2 * kOL, kPlane = kNX * kNX;  // the arrays' padded tiles
+constexpr int kPitch = kN + 2;            // LDS tile: rows and columns -1..90
+constexpr int kTile = kPitch * kPitch;    // doubles
+constexpr int kWaves = 8, kThreads = 64 * kWaves;
+constexpr int kRows = 6, kPts = 3 * kRows;   // rows of a half-wave, points of a thread
+constexpr int kRingLanes = 4 * kN / kWaves;  // ring points per wave, in its first lanes
+constexpr int kPartA = 32, kPartB = 48;      // lanes that poll the partial sums of tile lane - kPartA / - kPartB
+static_assert(kRingLanes <= 64 && kPartB - kPartA >= kResMaxTiles && 64 - kPartB >= kResMaxTiles, "poll lanes");
+static_assert(15 * kRows == kN && 2 * kWaves == 16, "rows");
+struct ResDev {
+    int B, T, G, nslots;
+    int64_t ms, oms;
+    const double *aW, *aS, *aC, *pW, *pS, *pC;
+    const double *b, *x0;
+    double* x;
+    const double* norm;
+    double tol_sq;
+    int max_iters;
+    const int32_t *full_off, *full_dst, *full_src;
+    const int8_t* full_sign;
+    const int32_t* op_index;
+    const int4* ring;     // [T][360] {slot, LDS offset | neg << 30, padded source or -1, padded destination}
+    const int32_t* pub;   // [T][4][90] slots of the tile's south and north rows and west and east columns, -1: not read
+    uint64_t* ring_ll;    // per group: [2][nslots][2] ring values, [2][T][4] partial sums, by parity of the exchange
+    size_t group_words;
+    uint64_t* next_ll;    // [G]
+    int* queue;
+    int* error;
+    unsigned long long limit;  // ticks a wait may take
+    mj_cg2d_diag* diag;
+};
+
+// ---------------------------------------------------------------------------------------------------- tagged words
+__device__ __forceinline__ void put_word(uint64_t* p, uint64_t v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ uint64_t get_word(const uint64_t* p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void put_double(uint64_t* p, double v, unsigned tag) {
+    const uint64_t hi = (uint64_t)tag << 32;
+    put_word(p, hi | (unsigned)__double2loint(v));
+    put_word(p + 1, hi | (unsigned)__double2hiint(v));
+}
+// Whether a wait that began at t0 (0: now) is to end: it took too long, or another workgroup gave up.
+__device__ __forceinline__ bool gave_up(const ResDev& a, unsigned long long& t0) {
+    const unsigned long long now = wall_clock64();
+    if (t0 == 0) t0 = now;
+    if (__hip_atomic_load(a.error, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0 && now - t0 <= a.limit) return false;
+    __hip_atomic_store(a.error, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return true;
+}
+// The doubles published with this tag at p (lanes with need_p) and q (lanes with need_q); the whole wave waits together.
+// False when the wait timed out or another workgroup gave up.
+__device__ __forceinline__ bool wait_doubles(const ResDev& a, const uint64_t* p, bool need_p, double& vp,
+                                             const uint64_t* q, bool need_q, double& vq, unsigned tag) {
+    uint64_t p0 = 0, p1 = 0, q0 = 0, q1 = 0;
+    unsigned spins = 0;
+    unsigned long long t0 = 0;
+    bool wp = need_p, wq = need_q;
+    for (;;) {
+        if (wp) {
+            p0 = get_word(p);
+            p1 = get_word(p + 1);
+        }
+        if (wq) {
+            q0 = get_word(q);
+            q1 = get_word(q + 1);
+        }
+        if (wp) wp = (unsigned)(p0 >> 32) != tag || (unsigned)(p1 >> 32) != tag;
+        if (wq) wq = (unsigned)(q0 >> 32) != tag || (unsigned)(q1 >> 32) != tag;
+        if (!__any(wp || wq)) break;
+        if ((++spins & 1023u) == 0 && gave_up(a, t0)) return false;
+    }
+    if (need_p) vp = __hiloint2double((int)(unsigned)p1, (int)(unsigned)p0);
+    if (need_q) vq = __hiloint2double((int)(unsigned)q1, (int)(unsigned)q0);
+    return true;
+}
+__device__ __forceinline__ double lane_double(double v, int lane) {
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
+                            __builtin_amdgcn_readlane(__double2loint(v), lane));
+}
+// p[off / 8 + k]: a uniform base, a lane's byte offset and a constant, the form of one load's address.
+__device__ __forceinline__ double at(const double* p, unsigned off, int k) {
+    return *reinterpret_cast<const double*>(reinterpret_cast<const char*>(p + k) + off);
+}
+__device__ __forceinline__ void put_at(double* p, unsigned off, int k, double v) {
+    *reinterpret_cast<double*>(reinterpret_cast<char*>(p + k) + off) = v;
+}
+
+// ---------------------------------------------------------------------------------------------------- row trees
+// a: the even rows of 16 lanes from a, the odd ones from b's even; b: a's odd rows, b's odd rows.
+__device__ __forceinline__ void swap16(double& a, double& b) {
+    const auto lo = __builtin_amdgcn_permlane16_swap((unsigned)__double2loint(a), (unsigned)__double2loint(b), false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap((unsigned)__double2hiint(a), (unsigned)__double2hiint(b), false, false);
+    a = __hiloint2double((int)hi[0], (int)lo[0]);
+    b = __hiloint2double((int)hi[1], (int)lo[1]);
+}
+template <int CTRL, int BANKS>
+__device__ __forceinline__ double dpp(double old, double v) {
+    const int lo = __builtin_amdgcn_update_dpp(__double2loint(old), __double2loint(v), CTRL, 0xf, BANKS, false);
+    const int hi = __builtin_amdgcn_update_dpp(__double2hiint(old), __double2hiint(v), CTRL, 0xf, BANKS, false);
+    return __hiloint2double(hi, lo);
+}
+// The row trees of a half-wave's six rows, both halves at once: w[i] is lane l's v[l] (+ v[l + 64]) + v[l + 32] of row
+// i. The steps 16, 8 and 4 run on two rows at a time in the lanes they leave idle; the sums end in the lanes of
+// row_of_lane.
+__device__ __forceinline__ double row_trees(double (&w)[kRows]) {
+    swap16(w[0], w[1]);
+    swap16(w[2], w[3]);
+    swap16(w[4], w[5]);
+    const double a = w[0] + w[1], b = w[2] + w[3], c = w[4] + w[5];
+    // step 8: lanes 0..7 of a row of 16 go on with a, lanes 8..15 with b
+    const double ab = dpp<0x118, 0xc>(a, b) + dpp<0x108, 0x3>(b, a), c8 = c + dpp<0x108, 0xf>(c, c);
+    // step 4: c goes on in lanes 4..7
+    double s = dpp<0x114, 0x2>(ab, c8) + dpp<0x104, 0x5>(c8, ab);
+    s = s + dpp<0x102, 0xf>(s, s);
+    return s + dpp<0x101, 0xf>(s, s);
+}
+// Which of its half's six rows a lane ends with, -1: none.
+__device__ __forceinline__ int row_of_lane(int lane) {
+    const int l = lane & 15, pair = l == 0 ? 0 : l == 8 ? 1 : l == 4 ? 2 : -1;
+    return pair < 0 ? -1 : 2 * pair + (lane >> 4 & 1);
+}
+
+// s = s + v[0], s + v[1], ... over the 16 lanes of the lane's row of 16; fma(v, 1, s) is the addition (one rounding),
+// and its operand can be broadcast within the instruction.
+__device__ __forceinline__ double add16(double s, double v) {
+    double one = 1.0;
+#define MJ_ADD1(i) "v_fmac_f64_dpp %0, %1, %2 row_newbcast:" #i " row_mask:0xf bank_mask:0xf\n"
+    asm volatile("s_nop 1\n" MJ_ADD1(0) MJ_ADD1(1) MJ_ADD1(2) MJ_ADD1(3) MJ_ADD1(4) MJ_ADD1(5) MJ_ADD1(6) MJ_ADD1(7)
+                     MJ_ADD1(8) MJ_ADD1(9) MJ_ADD1(10) MJ_ADD1(11) MJ_ADD1(12) MJ_ADD1(13) MJ_ADD1(14) MJ_ADD1(15)
+                 : "+v"(s)
+                 : "v"(v), "v"(one));
+#undef MJ_ADD1
+    return s;
+}
+// Tile-order sums of the partials in lanes kPartA.. and kPartB.. (rows 2 and 3 of 16 lanes; -0.0 in those of no tile:
+// s + -0.0 is s).
+__device__ __forceinline__ void part_sums(double v, double& A, double& B) {
+    const double s = add16(0.0, v);
+    A = lane_double(s, kPartA);
+    B = lane_double(s, kPartB);
+}
+
+// ---------------------------------------------------------------------------------------------------- Fortran order
+// Two chains of 16 additions at a time (their additions alternate: each hides the other's latency).
+__device__ __forceinline__ void add16x2(double& s, double v, double& t, double w) {
+    const double one = 1.0;
+#define MJ_ADD2(i)                                                                    \
+    "v_fmac_f64_dpp %0, %2, %4 row_newbcast:" #i " row_mask:0xf bank_mask:0xf\n"     \
+    "v_fmac_f64_dpp %1, %3, %4 row_newbcast:" #i " row_mask:0xf bank_mask:0xf\n"
+    asm volatile("s_nop 1\n" MJ_ADD2(0) MJ_ADD2(1) MJ_ADD2(2) MJ_ADD2(3) MJ_ADD2(4) MJ_ADD2(5) MJ_ADD2(6) MJ_ADD2(7)
+                     MJ_ADD2(8) MJ_ADD2(9) MJ_ADD2(10) MJ_ADD2(11) MJ_ADD2(12) MJ_ADD2(13) MJ_ADD2(14) MJ_ADD2(15)
+                 : "+v"(s), "+v"(t)
+                 : "v"(v), "v"(w), "v"(one));
+#undef MJ_ADD2
+}
+
+// The strictly sequential sums ((0 + v[0]) + v[1]) + ... of NS staged arrays of kN * kN values, bitwise.
+//
+// A chain of 8,100 dependent additions is bound by the latency of an FP64 addition (8.5 cycles: 29 us a sum; 12-16
+// cycles with operands from LDS, 45 us). So the chain is cut into chunks that run at the same time, two to a wave: a
+// chunk needs the running sum it starts from, which is only known approximately (the tree sums of the chunks before
+// it), up to the rounding of the chain so far, a few units in the last place. Its 64 lanes therefore run the chunk from
+// the 64 consecutive doubles around that estimate; then the chunks are put together by looking up, chunk after chunk,
+// the lane that started from the true running sum. Where no lane did, the chunks from there on run again around better
+// estimates: the first of them around its true start, the others moved by the same distance. Every pass settles at
+// least one chunk, so the result is always the chain's, whatever the data; it rarely takes more than two passes.
+// All threads call it; sum[q] is valid in every thread.
+struct ChainLds {
+    double ends[2 * kWaves][64], center[2 * kWaves], sum[2];
+    int from[2];  // first chunk of a sum that has to run (again); all of them: done
+};
+template <int NS>
+__device__ __forceinline__ void tile_chain(const double* st0, const double* st1, ChainLds& C) {
+    constexpr int NC = 2 * kWaves / NS, n = kN * kN;  // chunks of a sum
+    constexpr int len = (n + NC - 1) / NC, steps = (len + 15) / 16;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15;
+    const int q = NS == 2 && wave >= kWaves / 2 ? 1 : 0, c = 2 * wave - q * NC;  // this wave's chunks: c, c + 1
+    const double* const v = (q ? st1 : st0) + c * len;
+    const int n1 = min(len, n - (c + 1) * len);  // values of chunk c + 1 (chunk c has len)
+    auto val = [&](int h, int k) { return k < (h ? n1 : len) ? v[h * len + k] : -0.0; };  // s + -0.0 is s
+    {
+        double t0 = 0.0, t1 = 0.0;
+        for (int k = lane; k < len; k += 64) {
+            t0 = t0 + val(0, k);
+            t1 = t1 + val(1, k);
+        }
+        t0 = wave_tree(t0, 0.0, false);
+        t1 = wave_tree(t1, 0.0, false);
+        if (lane == 0) {
+            C.center[2 * wave] = t0;
+            C.center[2 * wave + 1] = t1;
+        }
+    }
+    if (tid < NS) C.from[tid] = 0;
+    __syncthreads();
+    if (tid < NS) {
+        double g = 0.0, d[NC];
+#pragma unroll
+        for (int k = 0; k < NC; ++k) d[k] = C.center[tid * NC + k];
+#pragma unroll
+        for (int k = 0; k < NC; ++k) {
+            C.center[tid * NC + k] = g;
+            g = g + d[k];
+        }
+    }
+    __syncthreads();
+    for (;;) {
+        const int from = C.from[q];
+        if (c + 1 >= from) {
+            double s = __longlong_as_double(__double_as_longlong(C.center[2 * wave]) + (lane - 32));
+            double t = __longlong_as_double(__double_as_longlong(C.center[2 * wave + 1]) + (lane - 32));
+            if (c == 0) s = 0.0;
+            double v0 = val(0, l16), v1 = val(1, l16);
+            for (int k = 0; k < steps; ++k) {
+                const double a = v0, b = v1;
+                v0 = val(0, 16 * (k + 1) + l16);
+                v1 = val(1, 16 * (k + 1) + l16);
+                add16x2(s, a, t, b);
+            }
+            C.ends[2 * wave][lane] = s;
+            C.ends[2 * wave + 1][lane] = t;
+        }
+        __syncthreads();
+        const int w = NS == 2 && tid >= 64 ? 1 : 0;  // the sum that this thread puts together
+        if (tid == 0 || (NS == 2 && tid == 64)) {
+            int k = C.from[w];
+            double s = k < NC ? C.center[w * NC + k] : 0.0;  // the true start of the first chunk that ran
+            while (k < NC) {
+                const long long at = __double_as_longlong(s) - __double_as_longlong(C.center[w * NC + k]) + 32;
+                if (at < 0 || at > 63) break;
+                s = C.ends[w * NC + k][at];
+                ++k;
+            }
+            if (k < NC) {  // chunk k starts from s: move its estimate there and the later ones along
+                double g = s;
+                for (int i = k; i < NC; ++i) {
+                    const double old = C.center[w * NC + i], e = C.ends[w * NC + i][32];
+                    C.center[w * NC + i] = g;
+                    g = e + (g - old);
+                }
+                C.from[w] = k;
+            } else if (C.from[w] < NC) {
+                C.from[w] = NC;
+                C.sum[w] = s;
+            }
+        }
+        __syncthreads();
+        if (C.from[0] >= NC && (NS == 1 || C.from[1] >= NC)) return;
+    }
+}
+
+// ---------------------------------------------------------------------------------------------------- the kernel
+// A thread's points, k = 3 i + c: row row0 + i, column l + 32 c (the third clamped to 89); in the padded arrays at
+// go[c > 1] bytes + gk(k), in the LDS tile at lo[c > 1] + lk(k). Derived anew wherever it is used (the thread number
+// passes through an empty asm statement), so that no derived address stays in registers across the phases.
+struct Pos {
+    int tid, l, row0, col2;
+    unsigned go[2];
+    int lo[2];
+    __device__ __forceinline__ explicit Pos(int tid_) : tid(tid_) {
+        asm volatile("" : "+v"(tid));
+        l = tid & 31;
+        row0 = kRows * min(tid >> 5, 14);
+        col2 = min(l + 64, kN - 1);
+        const int cols[2] = {l, col2};
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            go[c] = 8u * (unsigned)(row0 * kNX + cols[c]);
+            lo[c] = (row0 + 1) * kPitch + 1 + cols[c];
+        }
+    }
+    static __device__ __forceinline__ constexpr int gk(int k) { return k / 3 * kNX + (k % 3 == 1 ? 32 : 0); }
+    static __device__ __forceinline__ constexpr int lk(int k) { return k / 3 * kPitch + (k % 3 == 1 ? 32 : 0); }
+    __device__ __forceinline__ bool third() const { return l + 64 < kN; }
+    __device__ __forceinline__ int col(int k) const { return k % 3 == 2 ? col2 : l + 32 * (k % 3); }
+    // p: column 0 of the tile's first interior row
+    __device__ __forceinline__ double ld(const double* p, int k, int d = 0) const {
+        return at(p, go[k % 3 == 2], gk(k) + d);
+    }
+    __device__ __forceinline__ void st(double* p, int k, double v) const { put_at(p, go[k % 3 == 2], gk(k), v); }
+};
+
+// The coefficients of one row of a thread's points: W here and at the next column, S of the next row, C.
+struct Coef {
+    double w[3], e[3], n[3], c[3];
+};
+
+// LDS. Tree order: the tile, then aW of the tile's rows (columns 0..90). Fortran order: the tile, over which one sum's
+// values are staged, then a second sum's.
+constexpr int kWPitch = kN + 1;
+constexpr int kLdsTree = kTile + kN * kWPitch, kLdsFort = kTile + kN * kN;
+
+template <int MODE>
+__global__ void __launch_bounds__(kThreads, 2) cg2d_resident_kernel(ResDev a) {
+    constexpr bool kFort = MODE == MJ_SUM_FORTRAN;
+    extern __shared__ __align__(16) double lds[];
+    double* const tile = lds;
+    double* const cacheW = lds + kTile;
+    __shared__ double rows[2][128], edge[4][kN];
+    __shared__ typename std::conditional<kFort, ChainLds, int>::type chain;
+    __shared__ int s_bad, s_next;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    // unit of this block: the blocks of an XCD (b % 8) take consecutive units, tile-major, so that few tiles'
+    // coefficients pass through an L2
+    int g, t;
+    {
+        const int n = gridDim.x, xcd = blockIdx.x % kXcds;
+        const int u = xcd * (n / kXcds) + min(xcd, n % kXcds) + blockIdx.x / kXcds;
+        t = u / a.G;
+        g = u - t * a.G;
+    }
+    const int tbase = t * kPlane + kOL * kNX + kOL;
+    // this lane's ring point (lanes below kRingLanes): where its value comes from and goes
+    const int epos = wave * kRingLanes + lane;
+    const int4 re = lane < kRingLanes ? a.ring[t * 4 * kN + epos] : make_int4(0, 0, -1, 0);
+    const bool rneed = lane < kRingLanes && re.z >= 0;
+    const int rlds = re.y;
+    const int eslot = lane < kRingLanes ? a.pub[t * 4 * kN + epos] : -1;
+    uint64_t* const words = a.ring_ll + (size_t)g * a.group_words;  // [2][nslots][2] ring values, [2][T][4] sums
+    const unsigned ring_words = 4u * (unsigned)a.nslots;
+    const bool pA = lane >= kPartA && lane < kPartA + a.T, pB = lane >= kPartB && lane < kPartB + a.T;
+    const unsigned ring_src = 2u * (unsigned)re.x;
+    const unsigned part_src = ring_words + (pB ? 4u * (unsigned)(lane - kPartB) + 2u : pA ? 4u * (unsigned)(lane - kPartA) : 0u);
+    unsigned seq = 0;  // number of the last exchange
+    unsigned members = 0;
+
+    if (tid == 0) s_bad = 0;
+    // the last exchange's words: ring value (lanes below kRingLanes) and partial sums A, B of every tile
+    auto receive = [&](bool ring, bool A, bool B, double& v, double& part) {
+        v = 0.0;
+        part = -0.0;
+        const unsigned odd = seq & 1;
+        if (!wait_doubles(a, words + (ring_src + odd * (ring_words >> 1)), ring && rneed, v,
+                          words + (part_src + odd * 4u * (unsigned)a.T), (A && pA) || (B && pB), part, seq) &&
+            lane == 0)
+            s_bad = 1;
+    };
+    auto publish_part = [&](int q, double v) {
+        put_double(words + (ring_words + ((seq & 1) * (unsigned)a.T + (unsigned)t) * 4 + 2 * q), v, seq);
+    };
+    // the tile's outermost rows and columns of v, for send_edges to publish after a barrier
+    auto keep_edges = [&](const double (&v)[kPts]) {
+        const Pos P(tid);
+        if (P.row0 == 0) {
+#pragma unroll
+            for (int c = 0; c < 3; ++c) edge[0][P.col(c)] = v[c];
+        }
+        if (P.row0 == kN - kRows) {
+#pragma unroll
+            for (int c = 0; c < 3; ++c) edge[1][P.col(c)] = v[kPts - 3 + c];
+        }
+        if (P.l == 0) {
+#pragma unroll
+            for (int i = 0; i < kRows; ++i) edge[2][P.row0 + i] = v[3 * i];
+        }
+        if (P.l == kN - 65) {
+#pragma unroll
+            for (int i = 0; i < kRows; ++i) edge[3][P.row0 + i] = v[3 * i + 2];
+        }
+    };
+    auto send_edges = [&]() {
+        if (eslot >= 0)
+            put_double(words + ((seq & 1) * (ring_words >> 1) + 2u * (unsigned)eslot), edge[0][epos], seq);
+    };
+    // the products f(k) of the thread's points into the row sums q, or into a staging area (Fortran order)
+    auto row_sums = [&](int q, auto&& f) {
+        const Pos P(tid);
+        const bool third = P.third();
+        double w[kRows];
+#pragma unroll
+        for (int i = 0; i < kRows; ++i) {
+            const double v0 = f(3 * i), v1 = f(3 * i + 1), v2 = f(3 * i + 2);
+            w[i] = (third ? v0 + v2 : v0) + v1;
+        }
+        const double s = row_trees(w);
+        const int i = row_of_lane(lane);
+        if (i >= 0) rows[q][P.row0 + i] = s;
+    };
+    auto stage = [&](double* st, auto&& f) {
+        const Pos P(tid);
+#pragma unroll
+        for (int k = 0; k < kPts; ++k) st[(P.row0 + k / 3) * kN + P.col(k)] = f(k);
+    };
+    // exchange seq: the edges of v, and the tile's sum of f as part q; every thread calls it
+    auto send_sum = [&](const double (&v)[kPts], int q, auto&& f) {
+        keep_edges(v);
+        if constexpr (kFort) {
+            __syncthreads();  // the staging area lies over the tile: every wave has read it
+            send_edges();
+            stage(tile, f);
+            __syncthreads();
+            tile_chain<1>(tile, nullptr, chain);
+            if (tid == 0) publish_part(q, chain.sum[0]);
+        } else {
+            row_sums(0, f);
+            __syncthreads();
+            send_edges();
+            if (wave == 0) {
+                const bool h = lane + 64 < kN;
+                const double s = wave_tree(rows[0][lane], h ? rows[0][lane + 64] : 0.0, h);
+                if (lane == 0) publish_part(q, s);
+            }
+        }
+    };
+    // the edges of v, and the tile's sums of f0 and f1 as parts 0 and 1
+    auto send_sums = [&](const double (&v)[kPts], auto&& f0, auto&& f1) {
+        keep_edges(v);
+        if constexpr (kFort) {
+            __syncthreads();
+            send_edges();
+            stage(tile, f0);
+            stage(lds + kTile, f1);
+            __syncthreads();
+            tile_chain<2>(tile, lds + kTile, chain);
+            if (tid < 2) publish_part(tid, chain.sum[tid]);
+        } else {
+            row_sums(0, f0);
+            row_sums(1, f1);
+            __syncthreads();
+            send_edges();
+            if (wave < 2) {
+                const bool h = lane + 64 < kN;
+                const double s = wave_tree(rows[wave][lane], h ? rows[wave][lane + 64] : 0.0, h);
+                if (lane == 0) publish_part(wave, s);
+            }
+        }
+    };
+    auto put_tile = [&](const double (&v)[kPts], double ring) {
+        const Pos P(tid);
+#pragma unroll
+        for (int k = 0; k < kPts; ++k) tile[P.lo[k % 3 == 2] + P.lk(k)] = v[k];
+        if (lane < kRingLanes) tile[rlds & ((1 << 30) - 1)] = (rlds >> 30) & 1 ? -ring : ring;
+    };
+    // o = A v (isA) or M v of the LDS tile at the thread's points, v its own values; W, S, C the slot's coefficients.
+    // The next row's coefficients are loaded while a row is computed; the first row's come from the caller (first_row),
+    // loaded before the wait for the other tiles.
+    auto row_coef = [&](const Pos& P, auto isA, const double* W, const double* S, const double* C, int i) {
+        constexpr bool kCached = decltype(isA)::value && !kFort;
+        Coef r;
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+            const int k = 3 * i + c;
+            r.w[c] = kCached ? 0.0 : P.ld(W, k);
+            r.e[c] = kCached ? 0.0 : P.ld(W, k, 1);
+            r.n[c] = P.ld(S, k, kNX);
+            r.c[c] = P.ld(C, k);
+        }
+        return r;
+    };
+    struct First {
+        Coef r;
+        double s[3];
+    };
+    auto first_row = [&](auto isA, const double* W, const double* S, const double* C) {
+        const Pos P(tid);
+        First f;
+        f.r = row_coef(P, isA, W, S, C, 0);
+#pragma unroll
+        for (int c = 0; c < 3; ++c) f.s[c] = P.ld(S, c);
+        return f;
+    };
+    auto stencil = [&](auto isA, const double* W, const double* S, const double* C, const First& f,
+                       const double (&v)[kPts], double (&o)[kPts]) {
+        constexpr bool kA = decltype(isA)::value, kCached = kA && !kFort;
+        const Pos P(tid);
+        Coef r = f.r;
+        double sn[3] = {f.s[0], f.s[1], f.s[2]};
+#pragma unroll
+        for (int i = 0; i < kRows; ++i) {
+            Coef nx;
+            if (i + 1 < kRows) nx = row_coef(P, isA, W, S, C, i + 1);
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                const int k = 3 * i + c, lq = P.lo[c == 2] + P.lk(k);
+                const double* cw = cacheW + (P.row0 + i) * kWPitch + P.col(c);
+                const double w = kCached ? cw[0] : r.w[c], e = kCached ? cw[1] : r.e[c];
+                const double s0 = sn[c], s1 = r.n[c], cc = r.c[c];
+                const double vm = i > 0 ? v[k - 3] : tile[lq - kPitch];
+                const double vp = i + 1 < kRows ? v[k + 3] : tile[lq + kPitch];
+                const double vl = tile[lq - 1], vr = tile[lq + 1], vc = v[k];
+                sn[c] = s1;
+                o[k] = kA ? w * vl + e * vr + s0 * vm + s1 * vp + cc * vc
+                          : cc * vc + w * vl + e * vr + s0 * vm + s1 * vp;
+            }
+            // the row is computed here: the compiler would otherwise move the arithmetic to its first use, behind
+            // every row's loads, and spill what they return
+            asm volatile("" : "+v"(o[3 * i]), "+v"(o[3 * i + 1]), "+v"(o[3 * i + 2]));
+            r = nx;
+        }
+    };
+
+    for (;;) {
+        // ---- the next member of the queue
+        ++members;
+        if (tid == 0) {
+            uint64_t* w = a.next_ll + g;
+            if (t == 0) {
+                s_next = atomicAdd(a.queue, 1);
+                put_word(w, (uint64_t)members << 32 | (unsigned)s_next);
+            } else {
+                unsigned spins = 0;
+                unsigned long long t0 = 0;
+                for (;;) {
+                    const uint64_t v = get_word(w);
+                    if ((unsigned)(v >> 32) == members) {
+                        s_next = (int)(unsigned)v;
+                        break;
+                    }
+                    if ((++spins & 1023u) == 0 && gave_up(a, t0)) {
+                        s_bad = 1;
+                        break;
+                    }
+                }
+            }
+        }
+        __syncthreads();
+        if (s_bad) break;
+        const int m = s_next;
+        if (m >= a.B) return;
+        const double* const x0 = a.x0 + m * a.ms;
+        const double* const b = a.b + m * a.ms + tbase;
+        double* const xg = a.x + m * a.ms;
+        const int64_t ob = (int64_t)(a.op_index ? a.op_index[m] : m) * a.oms + tbase;
+        const double nm = a.norm[m];
+        double x[kPts], r[kPts], s[kPts], zq[kPts];
+        const double *const aW = a.aW + ob, *const aS = a.aS + ob, *const aC = a.aC + ob;
+        const double *const pW = a.pW + ob, *const pS = a.pS + ob, *const pC = a.pC + ob;
+        const std::true_type A{};
+        const std::false_type M{};
+        double rring = 0.0, sring = 0.0;
+
+        // ---- I0: max |b cg2dNorm|
+        {
+            const Pos P(tid);
+            double mx = 0.0;
+#pragma unroll
+            for (int k = 0; k < kPts; ++k) mx = fmax(mx, fabs(P.ld(b, k) * nm));
+            for (int o = 32; o >= 1; o >>= 1) mx = fmax(mx, __shfl_xor(mx, o, 64));
+            if (lane == 0) rows[0][wave] = mx;
+            if constexpr (!kFort) {
+                for (int q = tid; q < kN * kWPitch; q += kThreads) {
+                    const int j = q / kWPitch;
+                    cacheW[q] = aW[j * kNX + q - j * kWPitch];
+                }
+            }
+        }
+        __syncthreads();
+        ++seq;
+        if (wave == 0) {
+            double mx = lane < kWaves ? rows[0][lane] : 0.0;
+            for (int o = 8; o >= 1; o >>= 1) mx = fmax(mx, __shfl_xor(mx, o, 64));
+            if (lane == 0) publish_part(0, mx);
+        }
+        // ---- I1: x = the normalised first guess with its exchanged halo, r = b - A x
+        double rhsMax = 0.0, v, part;
+        receive(false, true, false, v, part);
+        for (int k = 0; k < a.T; ++k) rhsMax = fmax(rhsMax, lane_double(part, kPartA + k));
+        const double rhsNorm = rhsMax != 0.0 ? 1.0 / rhsMax : 1.0;
+        First f = first_row(A, aW, aS, aC);
+        {
+            const Pos P(tid);
+#pragma unroll
+            for (int k = 0; k < kPts; ++k) x[k] = P.ld(x0 + tbase, k) * rhsNorm;
+            double xr = 0.0;
+            if (lane < kRingLanes) xr = re.z >= 0 ? x0[re.z] * rhsNorm : x0[re.w];
+            put_tile(x, xr);
+        }
+        // halo of x: the first guess, then the exchanged points
+        for (int q = tid; q < kPlane; q += kThreads) {
+            const int j = q / kNX, i = q - j * kNX;
+            if (j < kOL || j >= kOL + kN || i < kOL || i >= kOL + kN) xg[t * kPlane + q] = x0[t * kPlane + q];
+        }
+        __syncthreads();
+        if (s_bad) break;
+        for (int k = a.full_off[t] + tid; k < a.full_off[t + 1]; k += kThreads) {
+            const int sp = a.full_src[k], sq = sp % kPlane, sj = sq / kNX, si = sq - sj * kNX;
+            const bool inner = sj >= kOL && sj < kOL + kN && si >= kOL && si < kOL + kN;
+            const double v = inner ? x0[sp] * rhsNorm : x0[sp];
+            xg[a.full_dst[k]] = a.full_sign[k] < 0 ? -v : v;
+        }
+        ++seq;
+        stencil(A, aW, aS, aC, f, x, zq);
+        {
+            const Pos P(tid);
+#pragma unroll
+            for (int k = 0; k < kPts; ++k) {
+                s[k] = P.ld(b, k) * nm * rhsNorm;
+                r[k] = s[k] - zq[k];
+            }
+        }
+        send_sums(r, [&](int k) { return r[k] * r[k]; }, [&](int k) { return s[k]; });
+        // ---- I2: z = M r, eta(1)
+        double err, eta, sumRHS, etaP = 1.0;
+        f = first_row(M, pW, pS, pC);
+        receive(true, true, true, rring, part);
+        part_sums(part, err, sumRHS);
+        put_tile(r, rring);
+        __syncthreads();
+        if (s_bad) break;
+        ++seq;
+        stencil(M, pW, pS, pC, f, r, zq);
+        send_sum(zq, 1, [&](int k) { return zq[k] * r[k]; });
+#pragma unroll
+        for (int k = 0; k < kPts; ++k) s[k] = 0.0;
+        if (t == 0 && tid == 0) {
+            a.diag[m].firstResidual = sqrt(err);
+            a.diag[m].sumRHS = sumRHS;
+            a.diag[m].rhsMax = rhsMax;
+            a.diag[m].outerIters = 0;
+            a.diag[m].launches = 0;
+        }
+        bool bad = false;
+        int n = 1;
+        for (;; ++n) {
+            // ---- B(n): stopping rule on err(n-1); s = z + beta s, q = A s, sigma
+            f = first_row(A, aW, aS, aC);
+            receive(true, n > 1, true, v, part);
+            {
+                double e;
+                part_sums(part, e, eta);
+                if (n > 1) err = e;
+            }
+            if (!(n - 1 < a.max_iters) || err < a.tol_sq) break;
+            const double beta = eta / etaP;
+#pragma unroll
+            for (int k = 0; k < kPts; ++k) s[k] = zq[k] + beta * s[k];
+            sring = rneed ? v + beta * sring : 0.0;
+            put_tile(s, sring);
+            __syncthreads();
+            if ((bad = s_bad)) break;
+            ++seq;
+            stencil(A, aW, aS, aC, f, s, zq);
+            send_sum(zq, 0, [&](int k) { return s[k] * zq[k]; });
+            // ---- C(n): x += alpha s, r -= alpha q, z = M r, err, eta
+            f = first_row(M, pW, pS, pC);
+            receive(true, true, false, v, part);
+            double sigma, unused;
+            part_sums(part, sigma, unused);
+            const double alpha = eta / sigma;
+#pragma unroll
+            for (int k = 0; k < kPts; ++k) {
+                x[k] = x[k] + alpha * s[k];
+                r[k] = r[k] - alpha * zq[k];
+            }
+            rring = rneed ? rring - alpha * v : 0.0;
+            put_tile(r, rring);
+            __syncthreads();
+            if ((bad = s_bad)) break;
+            ++seq;
+            stencil(M, pW, pS, pC, f, r, zq);
+            send_sums(zq, [&](int k) { return r[k] * r[k]; }, [&](int k) { return zq[k] * r[k]; });
+            etaP = eta;
+        }
+        if (bad) break;
+        // un-normalise x (cg2d.F:380-395)
+        {
+            const Pos P(tid);
+#pragma unroll
+            for (int k = 0; k < kPts; ++k) P.st(xg + tbase, k, x[k] / rhsNorm);
+        }
+        if (t == 0 && tid == 0) {
+            a.diag[m].lastResidual = sqrt(err);
+            a.diag[m].numIters = n - 1;
+            a.diag[m].converged = err < a.tol_sq ? 1 : 0;
+        }
+    }
+    // a wait timed out: every member's record says so
+    for (int m = blockIdx.x * kThreads + tid; m < a.B; m += gridDim.x * kThreads) a.diag[m].converged = -2;
+}
+
+__global__ void res_init_kernel(uint64_t* words, size_t n, int* queue, int* error) {
+    for (size_t k = (size_t)blockIdx.x * blockDim.x + threadIdx.x; k < n; k += (size_t)gridDim.x * blockDim.x)
+        words[k] = 0;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        *queue = 0;
+        *error = 0;
+    }
+}
+
+// Workspace: the groups' words, the queue's, then the queue and the error flag. The words up to misc are cleared.
+struct ResLayout {
+    size_t group_words, next, misc, total;
+};
+ResLayout res_layout(int G, int T, int nslots) {
+    ResLayout L{};
+    L.group_words = ((size_t)4 * nslots + (size_t)8 * T + 31) / 32 * 32;
+    L.next = (size_t)G * L.group_words * 8;
+    L.misc = (L.next + (size_t)G * 8 + 255) / 256 * 256;
+    L.total = L.misc + 256;
+    return L;
+}
+
+}  // namespace
+
+bool resident_fits(const mj_halo_plan* P, const mj_cg2d_config* c) {
+    return c->sNx == kN && c->sNy == kN && c->OL == kOL && c->ntiles <= kResMaxTiles && P->res_ok;
+}
+
+int resident_solve(mj_halo_plan* P, const mj_cg2d_ops* ops, const double* b, const double* x0, double* x,
+                   const double* cg2dNorm, const mj_cg2d_config* cfg, void* workspace, size_t workspace_bytes,
+                   mj_cg2d_diag* diag, hipStream_t st, bool* done) {
+    *done = false;
+    int dev = 0, ncu = 0, coop = 0, clk_khz = 0, max_lds = 0, per_cu = 0;
+    MJ_HIP(hipGetDevice(&dev));
+    MJ_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
+    MJ_HIP(hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, dev));
+    MJ_HIP(hipDeviceGetAttribute(&clk_khz, hipDeviceAttributeWallClockRate, dev));
+    MJ_HIP(hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
+    const void* kfn = cfg->sum_order == MJ_SUM_FORTRAN ? (const void*)cg2d_resident_kernel<MJ_SUM_FORTRAN>
+                                                       : (const void*)cg2d_resident_kernel<MJ_SUM_TREE>;
+    const size_t lds = (cfg->sum_order == MJ_SUM_FORTRAN ? kLdsFort : kLdsTree) * sizeof(double);
+    if (!coop || (size_t)max_lds < lds) return MJ_OK;
+    MJ_HIP(hipFuncSetAttribute(kfn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    MJ_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kfn, kThreads, lds));
+    const int T = cfg->ntiles;
+    int G = std::min(cfg->batch, per_cu * ncu / T);
+    if (G < 1) return MJ_OK;
+    const ResLayout L = res_layout(G, T, P->res_nslots);
+    if (L.total > workspace_bytes) return MJ_OK;
+    char* w = (char*)workspace;
+    ResDev a{};
+    a.B = cfg->batch;
+    a.T = T;
+    a.G = G;
+    a.nslots = P->res_nslots;
+    a.ms = cfg->member_stride;
+    a.oms = ops->member_stride;
+    a.aW = ops->aW2d;
+    a.aS = ops->aS2d;
+    a.aC = ops->aC2d;
+    a.pW = ops->pW;
+    a.pS = ops->pS;
+    a.pC = ops->pC;
+    a.b = b;
+    a.x0 = x0;
+    a.x = x;
+    a.norm = cg2dNorm;
+    a.tol_sq = cfg->tolerance * cfg->tolerance;  // cg2d.F:111
+    a.max_iters = cfg->max_iters;
+    a.full_off = P->cg_full_off;
+    a.full_dst = P->cg_full_dst;
+    a.full_src = P->cg_full_src;
+    a.full_sign = P->cg_full_sign;
+    a.op_index = ops->op_index;
+    a.ring = P->res_ring;
+    a.pub = P->res_pub;
+    a.ring_ll = (uint64_t*)w;
+    a.group_words = L.group_words;
+    a.next_ll = (uint64_t*)(w + L.next);
+    a.queue = (int*)(w + L.misc);
+    a.error = (int*)(w + L.misc + 64);
+    a.limit = (unsigned long long)(clk_khz > 0 ? clk_khz : 100000) * 1000ull * 20ull;  // 20 s
+    a.diag = diag;
+    hipLaunchKernelGGL(res_init_kernel, dim3(64), dim3(256), 0, st, (uint64_t*)w, L.misc / 8, a.queue, a.error);
+    MJ_HIP(hipGetLastError());
+    void* args[] = {(void*)&a};
+    MJ_HIP(hipLaunchCooperativeKernel(kfn, dim3(G * T), dim3(kThreads), args, (unsigned)lds, st));
+    *done = true;
+    return MJ_OK;
+}
+
+// The ring entries and publication slots of the resident solves, from the per-tile ring tables of the plan (held lock).
+int ensure_resident_tables(mj_halo_plan* P, const std::vector<int32_t>& roff, const std::vector<int32_t>& rdst,
+                           const std::vector<int32_t>& rsrc, const std::vector<int8_t>& rsg) {
+    const int nx = P->nx, plane = P->nx * P->ny, T = P->ntiles, OL = kOL;
+    if (nx != kNX || P->ny != kNX || T > kResMaxTiles) return MJ_OK;
+    std::vector<int4> ring((size_t)T * 4 * kN);
+    std::vector<int32_t> pub((size_t)T * 4 * kN, -1);
+    int nslots = 0;
+    for (int t = 0; t < T; ++t) {
+        if (roff[t + 1] - roff[t] != 4 * kN) return MJ_OK;
+        for (int k = 0; k < 4 * kN; ++k) {
+            const int e = roff[t] + k, d = rdst[e] % plane, s = rsrc[e];
+            int slot = 0;
+            if (s >= 0) {
+                const int sq = s % plane, sj = sq / nx - OL, si = sq % nx - OL;
+                // sources lie on the outermost rows and columns (the kernel publishes those)
+                int pos = -1;
+                if (sj == 0) pos = si;
+                else if (sj == kN - 1) pos = kN + si;
+                else if (si == 0) pos = 2 * kN + sj;
+                else if (si == kN - 1) pos = 3 * kN + sj;
+                if (pos < 0) return MJ_OK;
+                int32_t& p = pub[(size_t)(s / plane) * 4 * kN + pos];
+                if (p < 0) p = nslots++;
+                slot = p;
+            }
+            const int lds = (d / nx - OL + 1) * kPitch + (d % nx - OL + 1);
+            ring[(size_t)t * 4 * kN + k] = make_int4(slot, lds | (rsg[e] < 0 ? 1 << 30 : 0), s, rdst[e]);
+        }
+    }
+    MJ_HIP(hipMalloc((void**)&P->res_ring, ring.size() * sizeof(int4)));
+    MJ_HIP(hipMemcpy(P->res_ring, ring.data(), ring.size() * sizeof(int4), hipMemcpyHostToDevice));
+    MJ_HIP(hipMalloc((void**)&P->res_pub, pub.size() * sizeof(int32_t)));
+    MJ_HIP(hipMemcpy(P->res_pub, pub.data(), pub.size() * sizeof(int32_t), hipMemcpyHostToDevice));
+    P->res_nslots = std::max(nslots, 1);
+    P->res_ok = 1;
+    return MJ_OK;
+}
+
+}  // namespace mj

@@ -30,6 +30,11 @@ struct mj_halo_plan {
     // the same ring entries for the compact work vectors of the mixed solve: the LDS offset of the ring point in
     // the stencil tile and the source's compact index within the member (-1: no source)
     int4* cg_cring = nullptr;  // ring entries of the mixed solve: {compact source, padded source, LDS offset | neg << 30, 0}
+    // tables of the resident solves (90 x 90 tiles): per ring point {slot, LDS offset | neg << 30, padded source or -1,
+    // padded destination}, and per point of a tile's outermost rows and columns the slot other tiles read it from
+    int4* res_ring = nullptr;
+    int32_t* res_pub = nullptr;
+    int res_nslots = 0, res_ok = 0;
 
     // Transpose tables (built once, on first use): per input component c (0 = u-like, 1 = v-like) and padded
     // point q, the written points that read q (tr_off[c][q] .. tr_off[c][q+1] into tr_dst/tr_map/tr_sign, sorted by
