@@ -447,11 +447,12 @@ def kernel_times(st, reps=3):
 def roofline_of(precision, cg_ms, d, op_index, members, launch):
     """The `roofline` object of a solve timed alone (cg_ms) with diagnostics d."""
     alg, impl, slot_iters = solve_bytes(precision, d, op_index)
-    launches = int(d["launches"].max())
+    launches = int(d["launches"].max())  # 0: one launch, persistent or resident
     if precision == "fp64":
-        kernel = "cg2d_persistent_kernel" if launch == "persistent" else "cg2d_phase_kernel"
+        kernel = "cg2d_phase_kernel" if launches else \
+            "cg2d_persistent_kernel" if launch == "persistent" else "cg2d_resident_kernel"
     else:
-        kernel = "mx_step_kernel"
+        kernel = "mx_step_kernel" if launches else "mx_resident_kernel"
     achieved = alg / (cg_ms * 1e-3) / 1e9
     tr = measured_traffic(kernel, members)
     return {"bound": "hbm", "kernel": kernel, "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",

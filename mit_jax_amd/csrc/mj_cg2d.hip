@@ -660,10 +660,9 @@ int solve_impl(const mj_halo_plan* plan_T, const mj_cg2d_ops* ops, const double*
     hipStream_t st = as_stream(stream);
     if (cfg->launch_mode == MJ_CG_LAUNCH_AUTO && cfg->block_threads == 0 && cfg->grid_blocks == 0 &&
         resident_fits(P, cfg)) {
-        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-        MJ_HIP(hipStreamIsCapturing(st, &cap));
-        bool done = false;
-        if (cap == hipStreamCaptureStatusNone &&
+        bool capturing = false, done = false;
+        if ((rc = stream_capturing(st, &capturing))) return rc;
+        if (!capturing &&
             (rc = resident_solve(P, ops, b, x0, x, cg2dNorm, cfg, workspace, workspace_bytes, diag, st, &done)))
             return rc;
         if (done) return MJ_OK;

@@ -25,7 +25,7 @@
 #include "mj_cg_sweep.h"
 #include "mj_common.h"
 #include "mj_internal.h"
-#include "mj_resident.h"
+#include "mj_resident_dev.h"
 
 namespace mj {
 namespace {
@@ -37,11 +37,11 @@ constexpr int kTile = kPitch * kPitch;    // doubles
 constexpr int kWaves = 8, kThreads = 64 * kWaves;
 constexpr int kRows = 6, kPts = 3 * kRows;   // rows of a half-wave, points of a thread
 constexpr int kRingLanes = 4 * kN / kWaves;  // ring points per wave, in its first lanes
-constexpr int kPartA = 32, kPartB = 48;      // lanes that poll the partial sums of tile lane - kPartA / - kPartB
-static_assert(kRingLanes <= 64 && kPartB - kPartA >= kResMaxTiles && 64 - kPartB >= kResMaxTiles, "poll lanes");
+static_assert(kRingLanes <= 64, "poll lanes");
 static_assert(15 * kRows == kN && 2 * kWaves == 16, "rows");
+
 struct ResDev {
-    int B, T, G, nslots;
+    int B;
     int64_t ms, oms;
     const double *aW, *aS, *aC, *pW, *pS, *pC;
     const double *b, *x0;
@@ -52,67 +52,12 @@ struct ResDev {
     const int32_t *full_off, *full_dst, *full_src;
     const int8_t* full_sign;
     const int32_t* op_index;
-    const int4* ring;     // [T][360] {slot, LDS offset | neg << 30, padded source or -1, padded destination}
-    const int32_t* pub;   // [T][4][90] slots of the tile's south and north rows and west and east columns, -1: not read
-    uint64_t* ring_ll;    // per group: [2][nslots][2] ring values, [2][T][4] partial sums, by parity of the exchange
-    size_t group_words;
-    uint64_t* next_ll;    // [G]
-    int* queue;
-    int* error;
-    unsigned long long limit;  // ticks a wait may take
+    const int4* ring;    // [T][360] {slot, LDS offset | neg << 30, padded source or -1, padded destination}
+    const int32_t* pub;  // [T][4][90] slots of the tile's south and north rows and west and east columns, -1: not read
+    ResSync y;
     mj_cg2d_diag* diag;
 };
 
-// ---------------------------------------------------------------------------------------------------- tagged words
-__device__ __forceinline__ void put_word(uint64_t* p, uint64_t v) {
-    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ uint64_t get_word(const uint64_t* p) {
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ void put_double(uint64_t* p, double v, unsigned tag) {
-    const uint64_t hi = (uint64_t)tag << 32;
-    put_word(p, hi | (unsigned)__double2loint(v));
-    put_word(p + 1, hi | (unsigned)__double2hiint(v));
-}
-// Whether a wait that began at t0 (0: now) is to end: it took too long, or another workgroup gave up.
-__device__ __forceinline__ bool gave_up(const ResDev& a, unsigned long long& t0) {
-    const unsigned long long now = wall_clock64();
-    if (t0 == 0) t0 = now;
-    if (__hip_atomic_load(a.error, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0 && now - t0 <= a.limit) return false;
-    __hip_atomic_store(a.error, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    return true;
-}
-// The doubles published with this tag at p (lanes with need_p) and q (lanes with need_q); the whole wave waits together.
-// False when the wait timed out or another workgroup gave up.
-__device__ __forceinline__ bool wait_doubles(const ResDev& a, const uint64_t* p, bool need_p, double& vp,
-                                             const uint64_t* q, bool need_q, double& vq, unsigned tag) {
-    uint64_t p0 = 0, p1 = 0, q0 = 0, q1 = 0;
-    unsigned spins = 0;
-    unsigned long long t0 = 0;
-    bool wp = need_p, wq = need_q;
-    for (;;) {
-        if (wp) {
-            p0 = get_word(p);
-            p1 = get_word(p + 1);
-        }
-        if (wq) {
-            q0 = get_word(q);
-            q1 = get_word(q + 1);
-        }
-        if (wp) wp = (unsigned)(p0 >> 32) != tag || (unsigned)(p1 >> 32) != tag;
-        if (wq) wq = (unsigned)(q0 >> 32) != tag || (unsigned)(q1 >> 32) != tag;
-        if (!__any(wp || wq)) break;
-        if ((++spins & 1023u) == 0 && gave_up(a, t0)) return false;
-    }
-    if (need_p) vp = __hiloint2double((int)(unsigned)p1, (int)(unsigned)p0);
-    if (need_q) vq = __hiloint2double((int)(unsigned)q1, (int)(unsigned)q0);
-    return true;
-}
-__device__ __forceinline__ double lane_double(double v, int lane) {
-    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
-                            __builtin_amdgcn_readlane(__double2loint(v), lane));
-}
 // p[off / 8 + k]: a uniform base, a lane's byte offset and a constant, the form of one load's address.
 __device__ __forceinline__ double at(const double* p, unsigned off, int k) {
     return *reinterpret_cast<const double*>(reinterpret_cast<const char*>(p + k) + off);
@@ -122,19 +67,6 @@ __device__ __forceinline__ void put_at(double* p, unsigned off, int k, double v)
 }
 
 // ---------------------------------------------------------------------------------------------------- row trees
-// a: the even rows of 16 lanes from a, the odd ones from b's even; b: a's odd rows, b's odd rows.
-__device__ __forceinline__ void swap16(double& a, double& b) {
-    const auto lo = __builtin_amdgcn_permlane16_swap((unsigned)__double2loint(a), (unsigned)__double2loint(b), false, false);
-    const auto hi = __builtin_amdgcn_permlane16_swap((unsigned)__double2hiint(a), (unsigned)__double2hiint(b), false, false);
-    a = __hiloint2double((int)hi[0], (int)lo[0]);
-    b = __hiloint2double((int)hi[1], (int)lo[1]);
-}
-template <int CTRL, int BANKS>
-__device__ __forceinline__ double dpp(double old, double v) {
-    const int lo = __builtin_amdgcn_update_dpp(__double2loint(old), __double2loint(v), CTRL, 0xf, BANKS, false);
-    const int hi = __builtin_amdgcn_update_dpp(__double2hiint(old), __double2hiint(v), CTRL, 0xf, BANKS, false);
-    return __hiloint2double(hi, lo);
-}
 // The row trees of a half-wave's six rows, both halves at once: w[i] is lane l's v[l] (+ v[l + 64]) + v[l + 32] of row
 // i. The steps 16, 8 and 4 run on two rows at a time in the lanes they leave idle; the sums end in the lanes of
 // row_of_lane.
@@ -185,7 +117,7 @@ __device__ __forceinline__ void add16x2(double& s, double v, double& t, double w
     "v_fmac_f64_dpp %1, %3, %4 row_newbcast:" #i " row_mask:0xf bank_mask:0xf\n"
     asm volatile("s_nop 1\n" MJ_ADD2(0) MJ_ADD2(1) MJ_ADD2(2) MJ_ADD2(3) MJ_ADD2(4) MJ_ADD2(5) MJ_ADD2(6) MJ_ADD2(7)
                      MJ_ADD2(8) MJ_ADD2(9) MJ_ADD2(10) MJ_ADD2(11) MJ_ADD2(12) MJ_ADD2(13) MJ_ADD2(14) MJ_ADD2(15)
-                 : "+v"(s), "+v"(t)
+                 : "+&v"(s), "+&v"(t)
                  : "v"(v), "v"(w), "v"(one));
 #undef MJ_ADD2
 }
@@ -336,15 +268,9 @@ __global__ void __launch_bounds__(kThreads, 2) cg2d_resident_kernel(ResDev a) {
     __shared__ typename std::conditional<kFort, ChainLds, int>::type chain;
     __shared__ int s_bad, s_next;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    // unit of this block: the blocks of an XCD (b % 8) take consecutive units, tile-major, so that few tiles'
-    // coefficients pass through an L2
     int g, t;
-    {
-        const int n = gridDim.x, xcd = blockIdx.x % kXcds;
-        const int u = xcd * (n / kXcds) + min(xcd, n % kXcds) + blockIdx.x / kXcds;
-        t = u / a.G;
-        g = u - t * a.G;
-    }
+    resident_unit(a.y.G, g, t);
+    const int T = a.y.T;
     const int tbase = t * kPlane + kOL * kNX + kOL;
     // this lane's ring point (lanes below kRingLanes): where its value comes from and goes
     const int epos = wave * kRingLanes + lane;
@@ -352,9 +278,9 @@ __global__ void __launch_bounds__(kThreads, 2) cg2d_resident_kernel(ResDev a) {
     const bool rneed = lane < kRingLanes && re.z >= 0;
     const int rlds = re.y;
     const int eslot = lane < kRingLanes ? a.pub[t * 4 * kN + epos] : -1;
-    uint64_t* const words = a.ring_ll + (size_t)g * a.group_words;  // [2][nslots][2] ring values, [2][T][4] sums
-    const unsigned ring_words = 4u * (unsigned)a.nslots;
-    const bool pA = lane >= kPartA && lane < kPartA + a.T, pB = lane >= kPartB && lane < kPartB + a.T;
+    uint64_t* const words = a.y.words + (size_t)g * a.y.group_words;
+    const unsigned ring_words = 4u * (unsigned)a.y.nslots;
+    const bool pA = lane >= kPartA && lane < kPartA + T, pB = lane >= kPartB && lane < kPartB + T;
     const unsigned ring_src = 2u * (unsigned)re.x;
     const unsigned part_src = ring_words + (pB ? 4u * (unsigned)(lane - kPartB) + 2u : pA ? 4u * (unsigned)(lane - kPartA) : 0u);
     unsigned seq = 0;  // number of the last exchange
@@ -363,16 +289,19 @@ __global__ void __launch_bounds__(kThreads, 2) cg2d_resident_kernel(ResDev a) {
     if (tid == 0) s_bad = 0;
     // the last exchange's words: ring value (lanes below kRingLanes) and partial sums A, B of every tile
     auto receive = [&](bool ring, bool A, bool B, double& v, double& part) {
-        v = 0.0;
+        double w[1] = {0.0};
         part = -0.0;
         const unsigned odd = seq & 1;
-        if (!wait_doubles(a, words + (ring_src + odd * (ring_words >> 1)), ring && rneed, v,
-                          words + (part_src + odd * 4u * (unsigned)a.T), (A && pA) || (B && pB), part, seq) &&
+        const uint64_t* const p[1] = {words + (ring_src + odd * (ring_words >> 1))};
+        const bool need[1] = {ring && rneed};
+        if (!wait_words<2, 1>(a.y, p, need, w, words + (part_src + odd * 4u * (unsigned)T), (A && pA) || (B && pB),
+                              part, seq) &&
             lane == 0)
             s_bad = 1;
+        v = w[0];
     };
     auto publish_part = [&](int q, double v) {
-        put_double(words + (ring_words + ((seq & 1) * (unsigned)a.T + (unsigned)t) * 4 + 2 * q), v, seq);
+        put_double(words + (ring_words + ((seq & 1) * (unsigned)T + (unsigned)t) * 4 + 2 * q), v, seq);
     };
     // the tile's outermost rows and columns of v, for send_edges to publish after a barrier
     auto keep_edges = [&](const double (&v)[kPts]) {
@@ -529,25 +458,8 @@ __global__ void __launch_bounds__(kThreads, 2) cg2d_resident_kernel(ResDev a) {
         // ---- the next member of the queue
         ++members;
         if (tid == 0) {
-            uint64_t* w = a.next_ll + g;
-            if (t == 0) {
-                s_next = atomicAdd(a.queue, 1);
-                put_word(w, (uint64_t)members << 32 | (unsigned)s_next);
-            } else {
-                unsigned spins = 0;
-                unsigned long long t0 = 0;
-                for (;;) {
-                    const uint64_t v = get_word(w);
-                    if ((unsigned)(v >> 32) == members) {
-                        s_next = (int)(unsigned)v;
-                        break;
-                    }
-                    if ((++spins & 1023u) == 0 && gave_up(a, t0)) {
-                        s_bad = 1;
-                        break;
-                    }
-                }
-            }
+            s_next = next_member(a.y, g, t, members);
+            if (s_next < 0) s_bad = 1;
         }
         __syncthreads();
         if (s_bad) break;
@@ -590,7 +502,7 @@ __global__ void __launch_bounds__(kThreads, 2) cg2d_resident_kernel(ResDev a) {
         // ---- I1: x = the normalised first guess with its exchanged halo, r = b - A x
         double rhsMax = 0.0, v, part;
         receive(false, true, false, v, part);
-        for (int k = 0; k < a.T; ++k) rhsMax = fmax(rhsMax, lane_double(part, kPartA + k));
+        for (int k = 0; k < T; ++k) rhsMax = fmax(rhsMax, lane_double(part, kPartA + k));
         const double rhsNorm = rhsMax != 0.0 ? 1.0 / rhsMax : 1.0;
         First f = first_row(A, aW, aS, aC);
         {
@@ -713,20 +625,105 @@ __global__ void res_init_kernel(uint64_t* words, size_t n, int* queue, int* erro
     }
 }
 
-// Workspace: the groups' words, the queue's, then the queue and the error flag. The words up to misc are cleared.
-struct ResLayout {
-    size_t group_words, next, misc, total;
-};
-ResLayout res_layout(int G, int T, int nslots) {
-    ResLayout L{};
-    L.group_words = ((size_t)4 * nslots + (size_t)8 * T + 31) / 32 * 32;
-    L.next = (size_t)G * L.group_words * 8;
-    L.misc = (L.next + (size_t)G * 8 + 255) / 256 * 256;
-    L.total = L.misc + 256;
-    return L;
+// The order in which a batch with several operators is taken: the members that need most iterations first, so that the
+// last ones to start are short (a group that starts a long member when the others are done leaves them idle). The number
+// of iterations grows as the diagonal's excess over the face coefficients (the free-surface term) falls; a sample of
+// each member's operator tells (key). It decides nothing but the order.
+constexpr int kOrderMax = 4096, kSampleStep = 8;  // largest batch that is ordered; every 8th row is looked at
+__global__ void __launch_bounds__(256) res_key_kernel(const double* aW, const double* aS, const double* aC, int64_t oms,
+                                                      const int32_t* op_index, int T, unsigned* key) {
+    __shared__ float s_sum[2][4];
+    const int m = blockIdx.x, tid = threadIdx.x;
+    const int64_t ob = (int64_t)(op_index ? op_index[m] : m) * oms;
+    constexpr int rows = (kN + kSampleStep - 1) / kSampleStep;
+    float excess = 0.0f, diag = 0.0f;
+    for (int i = tid; i < T * rows * kN; i += 256) {
+        const int t = i / (rows * kN), r = i - t * rows * kN, j = r / kN;
+        const int64_t p = ob + t * kPlane + (kOL + j * kSampleStep) * kNX + kOL + (r - j * kN);
+        const double c = aC[p];
+        excess += (float)fabs(aW[p] + aW[p + 1] + aS[p] + aS[p + kNX] + c);
+        diag += (float)fabs(c);
+    }
+    for (int o = 32; o >= 1; o >>= 1) {
+        excess += __shfl_xor(excess, o, 64);
+        diag += __shfl_xor(diag, o, 64);
+    }
+    if ((tid & 63) == 0) {
+        s_sum[0][tid >> 6] = excess;
+        s_sum[1][tid >> 6] = diag;
+    }
+    __syncthreads();
+    if (tid == 0) {
+        for (int w = 1; w < 4; ++w) {
+            excess += s_sum[0][w];
+            diag += s_sum[1][w];
+        }
+        key[m] = __float_as_uint(excess / diag);  // >= 0: ordered as its bits (NaN too)
+    }
+}
+__global__ void __launch_bounds__(1024) res_order_kernel(const unsigned* key, int B, int* order) {
+    __shared__ unsigned s_key[kOrderMax];
+    for (int m = threadIdx.x; m < B; m += 1024) s_key[m] = key[m];
+    __syncthreads();
+    for (int m = threadIdx.x; m < B; m += 1024) {
+        int rank = 0;
+        for (int q = 0; q < B; ++q) rank += s_key[q] < s_key[m] || (s_key[q] == s_key[m] && q < m);
+        order[rank] = m;
+    }
 }
 
 }  // namespace
+
+int resident_prepare(const mj_halo_plan* P, const mj_cg2d_ops* ops, const mj_cg2d_config* cfg, const void* kfn,
+                     int threads, size_t lds, void* workspace, size_t workspace_bytes, hipStream_t st, ResSync* y,
+                     bool* ok) {
+    *ok = false;
+    int dev = 0, ncu = 0, coop = 0, clk_khz = 0, max_lds = 0, per_cu = 0;
+    MJ_HIP(hipGetDevice(&dev));
+    MJ_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
+    MJ_HIP(hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, dev));
+    MJ_HIP(hipDeviceGetAttribute(&clk_khz, hipDeviceAttributeWallClockRate, dev));
+    MJ_HIP(hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
+    if (!coop || (size_t)max_lds < lds) return MJ_OK;
+    MJ_HIP(hipFuncSetAttribute(kfn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    MJ_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kfn, threads, lds));
+    y->T = P->ntiles;
+    y->nslots = P->res_nslots;
+    y->B = cfg->batch;
+    y->G = std::min(y->B, per_cu * ncu / y->T);
+    if (y->G < 1) return MJ_OK;
+    y->group_words = ((size_t)4 * y->nslots + (size_t)8 * y->T + 31) / 32 * 32;
+    const size_t next = (size_t)y->G * y->group_words, misc = (next + y->G + 31) / 32 * 32;  // words
+    if ((misc + 32 + y->B) * 8 > workspace_bytes) return MJ_OK;
+    uint64_t* const w = (uint64_t*)workspace;
+    y->words = w;
+    y->next = w + next;
+    y->queue = (int*)(w + misc);
+    y->error = (int*)(w + misc + 8);
+    y->limit = (unsigned long long)(clk_khz > 0 ? clk_khz : 100000) * 1000ull * 20ull;  // 20 s
+    hipLaunchKernelGGL(res_init_kernel, dim3(64), dim3(256), 0, st, w, misc, y->queue, y->error);
+    MJ_HIP(hipGetLastError());
+    y->order = nullptr;
+    if (ops->member_stride != 0 && y->B > y->G && y->B <= kOrderMax) {
+        unsigned* const key = (unsigned*)(w + misc + 32);
+        int* const order = (int*)key + y->B;
+        hipLaunchKernelGGL(res_key_kernel, dim3(y->B), dim3(256), 0, st, ops->aW2d, ops->aS2d, ops->aC2d,
+                           ops->member_stride, ops->op_index, y->T, key);
+        MJ_HIP(hipGetLastError());
+        hipLaunchKernelGGL(res_order_kernel, dim3(1), dim3(1024), 0, st, key, y->B, order);
+        MJ_HIP(hipGetLastError());
+        y->order = order;
+    }
+    *ok = true;
+    return MJ_OK;
+}
+
+int stream_capturing(hipStream_t st, bool* capturing) {
+    hipStreamCaptureStatus s = hipStreamCaptureStatusNone;
+    MJ_HIP(hipStreamIsCapturing(st, &s));
+    *capturing = s != hipStreamCaptureStatusNone;
+    return MJ_OK;
+}
 
 bool resident_fits(const mj_halo_plan* P, const mj_cg2d_config* c) {
     return c->sNx == kN && c->sNy == kN && c->OL == kOL && c->ntiles <= kResMaxTiles && P->res_ok;
@@ -736,29 +733,14 @@ int resident_solve(mj_halo_plan* P, const mj_cg2d_ops* ops, const double* b, con
                    const double* cg2dNorm, const mj_cg2d_config* cfg, void* workspace, size_t workspace_bytes,
                    mj_cg2d_diag* diag, hipStream_t st, bool* done) {
     *done = false;
-    int dev = 0, ncu = 0, coop = 0, clk_khz = 0, max_lds = 0, per_cu = 0;
-    MJ_HIP(hipGetDevice(&dev));
-    MJ_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
-    MJ_HIP(hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, dev));
-    MJ_HIP(hipDeviceGetAttribute(&clk_khz, hipDeviceAttributeWallClockRate, dev));
-    MJ_HIP(hipDeviceGetAttribute(&max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
     const void* kfn = cfg->sum_order == MJ_SUM_FORTRAN ? (const void*)cg2d_resident_kernel<MJ_SUM_FORTRAN>
                                                        : (const void*)cg2d_resident_kernel<MJ_SUM_TREE>;
     const size_t lds = (cfg->sum_order == MJ_SUM_FORTRAN ? kLdsFort : kLdsTree) * sizeof(double);
-    if (!coop || (size_t)max_lds < lds) return MJ_OK;
-    MJ_HIP(hipFuncSetAttribute(kfn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    MJ_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kfn, kThreads, lds));
-    const int T = cfg->ntiles;
-    int G = std::min(cfg->batch, per_cu * ncu / T);
-    if (G < 1) return MJ_OK;
-    const ResLayout L = res_layout(G, T, P->res_nslots);
-    if (L.total > workspace_bytes) return MJ_OK;
-    char* w = (char*)workspace;
     ResDev a{};
+    bool ok = false;
+    const int rc = resident_prepare(P, ops, cfg, kfn, kThreads, lds, workspace, workspace_bytes, st, &a.y, &ok);
+    if (rc || !ok) return rc;
     a.B = cfg->batch;
-    a.T = T;
-    a.G = G;
-    a.nslots = P->res_nslots;
     a.ms = cfg->member_stride;
     a.oms = ops->member_stride;
     a.aW = ops->aW2d;
@@ -780,17 +762,9 @@ int resident_solve(mj_halo_plan* P, const mj_cg2d_ops* ops, const double* b, con
     a.op_index = ops->op_index;
     a.ring = P->res_ring;
     a.pub = P->res_pub;
-    a.ring_ll = (uint64_t*)w;
-    a.group_words = L.group_words;
-    a.next_ll = (uint64_t*)(w + L.next);
-    a.queue = (int*)(w + L.misc);
-    a.error = (int*)(w + L.misc + 64);
-    a.limit = (unsigned long long)(clk_khz > 0 ? clk_khz : 100000) * 1000ull * 20ull;  // 20 s
     a.diag = diag;
-    hipLaunchKernelGGL(res_init_kernel, dim3(64), dim3(256), 0, st, (uint64_t*)w, L.misc / 8, a.queue, a.error);
-    MJ_HIP(hipGetLastError());
     void* args[] = {(void*)&a};
-    MJ_HIP(hipLaunchCooperativeKernel(kfn, dim3(G * T), dim3(kThreads), args, (unsigned)lds, st));
+    MJ_HIP(hipLaunchCooperativeKernel(kfn, dim3(a.y.G * a.y.T), dim3(kThreads), args, (unsigned)lds, st));
     *done = true;
     return MJ_OK;
 }

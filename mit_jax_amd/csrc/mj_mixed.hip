@@ -41,10 +41,12 @@
 // (wave_tree, slot k of the block in lane k), and the block sums are added in block order. The order depends on the
 // tile shape only, not on the launch geometry. The true-residual sums (FP64 refinement) use the "tile" order itself.
 #include <algorithm>
+#include <type_traits>
 
 #include "mj_cg_sweep.h"
 #include "mj_common.h"
 #include "mj_internal.h"
+#include "mj_resident_dev.h"
 
 namespace mj {
 
@@ -284,11 +286,9 @@ __device__ __forceinline__ void ring_fill(const MxDev& a, int t, const MxRing& r
     }
 }
 
-// I1: x = normalised first guess with exchanged halos; r = bn - A x (FP64); partials of err and sumRHS; the
-// member's record starts in RST.
-__device__ __forceinline__ void mx_I1(const MxDev& a, int m, int t) {
+// I1: x = normalised first guess with exchanged halos; r = bn - A x (FP64); row sums of err (0) and sumRHS (1).
+__device__ __forceinline__ void mx_first_rows(const MxDev& a, int m, int t, double rhsNorm) {
     MJ_UNIT_IDS
-    const double rhsNorm = member_rhs_norm(a, m);
     const double nm = a.norm[m];
     const double* b = a.b + m * a.ms;
     double* x = a.x + m * a.ms;
@@ -308,6 +308,11 @@ __device__ __forceinline__ void mx_I1(const MxDev& a, int m, int t) {
         put_row<MJ_SUM_TREE>(0, jl, lane, r_0 * r_0, r_1 * r_1, has1, nullptr, sNx, sNy);
         put_row<MJ_SUM_TREE>(1, jl, lane, bn0, bn1, has1, nullptr, sNx, sNy);
     })
+}
+// I1 with the partials of the two sums; the member's record starts in RST.
+__device__ __forceinline__ void mx_I1(const MxDev& a, int m, int t) {
+    MJ_UNIT_IDS
+    mx_first_rows(a, m, t, member_rhs_norm(a, m));
     store_tile_sums<MJ_SUM_TREE>(a.perr64, a.psum, m * a.T + t, lane, wave, nwaves, nullptr, sNx, sNy);
     if (t == 0 && tid == 0) {
         a.rec[m] = MxRec{MX_RST, 0, 0, 0, 0, 0, 0, 0, 0.0, 0.0, 0.0};
@@ -317,9 +322,8 @@ __device__ __forceinline__ void mx_I1(const MxDev& a, int m, int t) {
 
 // Finish: x /= rhsNorm on the interior; the halo points the true-residual steps used for x's ring get back the
 // exchanged normalised first guess.
-__device__ __forceinline__ void mx_finish(const MxDev& a, int m, int t) {
+__device__ __forceinline__ void mx_finish(const MxDev& a, int m, int t, double rhsNorm) {
     MJ_UNIT_IDS
-    const double rhsNorm = member_rhs_norm(a, m);
     double* x = a.x + m * a.ms;
     MJ_ROWS({
         x[p0] = x[p0] / rhsNorm;
@@ -402,25 +406,16 @@ __device__ __forceinline__ void mx_update(const MxDev& a, int m, int t, int n, d
     }
 }
 
-// True residual: x's ring from its sources (the updated interior of other tiles), r = bn - A x (FP64), partials
-// of err.
-__device__ __forceinline__ void mx_true(const MxDev& a, int m, int t) {
+// True residual of an x whose ring is in place: r = bn - A x (FP64), row sums of err.
+__device__ __forceinline__ void mx_true_rows(const MxDev& a, int m, int t, double rhsNorm) {
     MJ_UNIT_IDS
     MJ_STRIP
-    const double rhsNorm = member_rhs_norm(a, m);
     const double nm = a.norm[m];
     const double* b = a.b + m * a.ms;
     double* x = a.x + m * a.ms;
     double* r = a.r64 + m * a.ms;
     const int64_t ob = (int64_t)slot_of(a, m) * a.oms;
     const double *__restrict__ aW = a.aW + ob, *__restrict__ aS = a.aS + ob, *__restrict__ aC = a.aC + ob;
-    for (int k = a.ring_off[t] + tid; k < a.ring_off[t + 1]; k += blockDim.x) {
-        const int s = a.ring_src[k];
-        if (s < 0) continue;  // no source: x keeps its halo value
-        const double v = x[s];
-        x[a.ring_dst[k]] = a.ring_sign[k] < 0 ? -v : v;
-    }
-    __syncthreads();
     if (j0 < j1) {
         int p = MJ_ROW(j0) + L.c;
         double2 Xm = ld2(x + p - nx), Xc = ld2(x + p), AS0 = ld2(aS + p);
@@ -443,6 +438,19 @@ __device__ __forceinline__ void mx_true(const MxDev& a, int m, int t) {
             AS0 = AS1;
         }
     }
+}
+// The same with x's ring from its sources (the updated interior of other tiles) first, and the partial of err.
+__device__ __forceinline__ void mx_true(const MxDev& a, int m, int t) {
+    MJ_UNIT_IDS
+    double* x = a.x + m * a.ms;
+    for (int k = a.ring_off[t] + tid; k < a.ring_off[t + 1]; k += blockDim.x) {
+        const int s = a.ring_src[k];
+        if (s < 0) continue;  // no source: x keeps its halo value
+        const double v = x[s];
+        x[a.ring_dst[k]] = a.ring_sign[k] < 0 ? -v : v;
+    }
+    __syncthreads();
+    mx_true_rows(a, m, t, member_rhs_norm(a, m));
     store_tile_sums<MJ_SUM_TREE>(a.perr64, nullptr, m * a.T + t, lane, wave, nwaves, nullptr, sNx, sNy);
 }
 
@@ -755,7 +763,7 @@ mx_step_kernel(MxDev a, int k) {
     const int n = (int)g_bcast[2];
     const bool def = g_bcast[5] != 0.0;
     switch (act) {
-        case AX_FINISH: mx_finish(a, m, t); break;
+        case AX_FINISH: mx_finish(a, m, t, member_rhs_norm(a, m)); break;
         case AX_RESTART: mx_restart(a, m, t, sigma, n); break;
         case AX_UPD: mx_update(a, m, t, n, sigma, alpha_prev, def, ap); break;
         case AX_IB: mx_IB(a, m, t, n, c, alpha_prev, true, ap); break;
@@ -782,6 +790,8 @@ __global__ void mx_convert_kernel(const double* aW, const double* aS, const doub
 #pragma unroll
     for (int k = 0; k < 6; ++k) dst[((int64_t)k * nslots + s) * per_slot + q] = inside ? (float)from[k][src] : 0.0f;
 }
+
+#include "mj_mixed_resident.h"
 
 __global__ void mx_reset_kernel(int* nactive, int B) {
     if (threadIdx.x == 0 && blockIdx.x == 0) *nactive = B;
@@ -861,6 +871,34 @@ int check_mixed(const mj_cg2d_config* c, const mj_cg2d_mixed_config* mc) {
     MJ_REQUIRE(mc->inner_tolerance > 0.0 && mc->inner_tolerance < 1.0, "cg2d mixed: inner_tolerance must be in (0, 1)");
     MJ_REQUIRE(mc->inner_max_iters >= 1 && mc->max_outer >= 1, "cg2d mixed: inner_max_iters, max_outer must be >= 1");
     MJ_REQUIRE(mc->op_slots >= 0, "cg2d mixed: op_slots < 0");
+    return MJ_OK;
+}
+
+// The FP32 copies of the operator's coefficients.
+int mx_convert(const MxDev& a, const mj_cg2d_ops* ops, int nslots, hipStream_t st) {
+    const int64_t tp = (int64_t)a.T * a.G.TSc;
+    hipLaunchKernelGGL(mx_convert_kernel, dim3((unsigned)((tp + 255) / 256), (unsigned)nslots), dim3(256), 0, st,
+                       ops->aW2d, ops->aS2d, ops->aC2d, ops->pW, ops->pS, ops->pC, ops->member_stride, nslots, a.T,
+                       a.OL, a.nx, a.plane, a.sNx, a.G, const_cast<float*>(a.aW32));
+    MJ_HIP(hipGetLastError());
+    return MJ_OK;
+}
+
+// The solve as a resident launch of form F (mj_mixed_resident.h); *done false when the device does not allow it.
+template <class F>
+int mx_resident_solve(const MxDev& a, const mj_halo_plan* P, const mj_cg2d_ops* ops, const mj_cg2d_config* cfg, int nslots,
+                      void* words, size_t words_bytes, hipStream_t st, bool* done) {
+    MxRes q{};
+    q.ring = P->res_ring;
+    q.pub = P->res_pub;
+    const void* kfn = (const void*)mx_resident_kernel<F>;
+    const size_t lds = mr_lds<F>();
+    int rc = resident_prepare(P, ops, cfg, kfn, 64 * F::kWaves, lds, words, words_bytes, st, &q.y, done);
+    if (rc || !*done) return rc;
+    if ((rc = mx_convert(a, ops, nslots, st))) return rc;
+    MxDev d = a;
+    void* args[] = {(void*)&d, (void*)&q};
+    MJ_HIP(hipLaunchCooperativeKernel(kfn, dim3(q.y.G * q.y.T), dim3(64 * F::kWaves), args, (unsigned)lds, st));
     return MJ_OK;
 }
 
@@ -968,6 +1006,17 @@ extern "C" int mj_cg2d_solve_mixed(const mj_halo_plan* plan_T, const mj_cg2d_ops
     int dev = 0, ncu = 0;
     MJ_HIP(hipGetDevice(&dev));
     MJ_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
+    if (cfg->launch_mode != MJ_CG_LAUNCH_PHASES_FIXED && cfg->block_threads == 0 && cfg->poll_iters == 0 &&
+        resident_fits(P, cfg)) {
+        bool capturing = false, done = false;
+        if ((rc = stream_capturing(st, &capturing))) return rc;
+        // MrOne up to 2.5 members per place (19 on 256 CUs), MrTwo beyond: on 256 CUs, 13 tiles, mixed level counts, one
+        // / two workgroups per CU take 2.50 / 2.77 ms for 20 members, 3.88 / 3.99 for 39, 5.37 / 4.67 for 57, 10.9 /
+        // 9.2 for 128 (the step launches 6.8, 7.9, 10.0, 18.7)
+        auto* const solve = 2 * (int64_t)a.B * a.T <= 5 * (int64_t)ncu ? mx_resident_solve<MrOne> : mx_resident_solve<MrTwo>;
+        if (!capturing && (rc = solve(a, P, ops, cfg, nslots, w + L.r0, L.coef - L.r0, st, &done))) return rc;
+        if (done) return MJ_OK;
+    }
     const int threads = cfg->block_threads ? cfg->block_threads
                                            : ((int64_t)a.B * a.T <= ncu ? kMxSmallThreads : kMxLargeThreads);
     const int nunits = a.B * a.T;
@@ -978,10 +1027,7 @@ extern "C" int mj_cg2d_solve_mixed(const mj_halo_plan* plan_T, const mj_cg2d_ops
         MJ_HIP(hipFuncSetAttribute((const void*)mx_step_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     hipLaunchKernelGGL(mx_reset_kernel, dim3(1), dim3(64), 0, st, a.nactive, a.B);
     MJ_HIP(hipGetLastError());
-    hipLaunchKernelGGL(mx_convert_kernel, dim3((unsigned)((tp + 255) / 256), (unsigned)nslots), dim3(256), 0, st,
-                       ops->aW2d, ops->aS2d, ops->aC2d, ops->pW, ops->pS, ops->pC, ops->member_stride, nslots, a.T,
-                       a.OL, a.nx, a.plane, a.sNx, a.G, coef);
-    MJ_HIP(hipGetLastError());
+    if ((rc = mx_convert(a, ops, nslots, st))) return rc;
     for (int ph = 0; ph < 2; ++ph) {
         hipLaunchKernelGGL(mx_init_kernel, grid, block, 0, st, a, ph);
         MJ_HIP(hipGetLastError());

@@ -1,0 +1,538 @@
+// The mixed-precision solve as one resident launch (part of mj_mixed.hip; 90 x 90 tiles).
+//
+// As the resident FP64 solve (mj_cg_resident.hip): a workgroup per (member, tile) keeps the FP32 vectors of the
+// recurrence on chip, the tiles of a member exchange ring values and partial sums as tagged words, and groups of
+// workgroups take members from a queue. The step launches stream 9.5 FP32 vectors per iteration through HBM instead.
+// An inner iteration is bound by the latency of its two exchanges and of the sums between them, so there are two forms:
+//   MrOne  one workgroup per CU, 11 waves, 3 slots per thread (r32, s, d and z or q: 48 registers); every coefficient is
+//          on chip (aW, aC and pC in registers, aS, pS and pW in LDS): the faster iteration, for batches that fit
+//   MrTwo  two workgroups per CU, 8 waves, 5 slots per thread (60 registers of r32, s and z or q); d in LDS, the
+//          coefficients from L2: one member's exchanges run under another's arithmetic, for larger batches. (Both
+//          workgroups must be resident whatever SIMDs the waves are placed on: waves in multiples of four are.)
+// The FP64 parts (true residual, solution update) run on the arrays as in the step launches, four or five times a solve.
+//
+// The arithmetic, its order and every sum are those of the step launches (mx_IB, mx_IC, mx_restart, mx_update, mx_true):
+// the same bits. The increment d takes every update when its alpha is known (the step launches apply two at a time, in
+// the same order). Wave w takes the 64-slot blocks w, w + waves, ...; the last valid slot is repeated by the lanes
+// beyond it, which are left out of the sums.
+constexpr int kMrN = 90, kMrNC = 23, kMrNS = kMrN * kMrNC, kMrCPc = 92, kMrW = 96;  // mx_geo(90, 90)
+constexpr int kMrBlocks = (kMrNS + 63) / 64;
+constexpr int kMrTile = (kMrN + 2) * kMrW, kMrS = (kMrN + 1) * kMrW;  // floats
+// A slot's place in the coefficients' LDS copies, rows of kMrW floats, is at = j * kMrW + c4, and in the operand's tile
+// at + kMrAt. The first two floats of a tile row hold no operand: the stencils' results at the row's west and east end.
+constexpr int kMrAt = kMrW + 4;
+struct MrOne {
+    static constexpr int kWaves = 11, kSlots = 3, kPerEu = 3;
+    static constexpr bool kOnChip = true;
+};
+struct MrTwo {
+    static constexpr int kWaves = 8, kSlots = 5, kPerEu = 4;
+    static constexpr bool kOnChip = false;
+};
+template <class F>
+constexpr size_t mr_lds() {
+    return (size_t)(kMrTile + (F::kOnChip ? 3 * kMrS : 4 * 64 * F::kWaves * F::kSlots)) * sizeof(float);
+}
+static_assert(kMrCPc == 4 * kMrNC && kMrBlocks == 33, "slots");
+
+struct MxRes {
+    ResSync y;
+    const int4* ring;    // [T][360] {slot, -, padded source or -1, padded destination}
+    const int32_t* pub;  // [T][4][90] slots of the tile's outermost rows and columns
+};
+
+// v through an empty asm statement: what is derived from it is derived where it is used and not kept in registers.
+__device__ __forceinline__ int anew(int v) {
+    asm volatile("" : "+v"(v));
+    return v;
+}
+// Slot f (clamped to the last): row j, first column c4.
+struct MrSlot {
+    int f, j, c4;
+    bool valid;
+    __device__ __forceinline__ explicit MrSlot(int slot) {
+        f = min(slot, kMrNS - 1);
+        valid = slot < kMrNS;
+        j = f / kMrNC;
+        c4 = 4 * (f - j * kMrNC);
+    }
+};
+
+__device__ __forceinline__ float4 axpy(float a, float4 x, float4 y) {  // y + a x
+    return make_float4(y.x + a * x.x, y.y + a * x.y, y.z + a * x.z, y.w + a * x.w);
+}
+__device__ __forceinline__ float4 axmy(float a, float4 x, float4 y) {  // y - a x
+    return make_float4(y.x - a * x.x, y.y - a * x.y, y.z - a * x.z, y.w - a * x.w);
+}
+
+// The sums over 64 lanes of six values, in the order of wave_tree, in the lanes of mr_lane.
+__device__ __forceinline__ double mr_trees(double v0, double v1, double v2, double v3, double v4, double v5) {
+    swap32(v0, v1);
+    swap32(v2, v3);
+    swap32(v4, v5);
+    double a = v0 + v1, b = v2 + v3, c = v4 + v5;  // halves: 0 | 1, 2 | 3, 4 | 5
+    swap16(a, b);
+    const double d = a + b;           // rows of 16: 0, 2, 1, 3
+    const double e = c + lane_up16(c);  // rows 0 and 2: 4, 5
+    // step 8: lanes 0..7 of a row go on with d, lanes 8..15 with e
+    double s = dpp<0x118, 0xc>(d, e) + dpp<0x108, 0x3>(e, d);
+    s = s + dpp<0x104, 0xf>(s, s);
+    s = s + dpp<0x102, 0xf>(s, s);
+    return s + dpp<0x101, 0xf>(s, s);
+}
+// Which of the six sums a lane holds, -1: none.
+__device__ __forceinline__ int mr_lane(int lane) {
+    return lane == 0 ? 0 : lane == 32 ? 1 : lane == 16 ? 2 : lane == 48 ? 3 : lane == 8 ? 4 : lane == 40 ? 5 : -1;
+}
+
+template <class F>
+__global__ void __launch_bounds__(64 * F::kWaves, F::kPerEu) mx_resident_kernel(MxDev a, MxRes q) {
+    constexpr int kMrWaves = F::kWaves, kMrThreads = 64 * kMrWaves, kMrSlots = F::kSlots;
+    constexpr int kRing = (4 * kMrN + kMrThreads - 1) / kMrThreads;  // ring points of a thread: tid, tid + kMrThreads
+    static_assert(kMrBlocks > (kMrSlots - 1) * kMrWaves && kMrBlocks <= kMrSlots * kMrWaves, "slots");
+    float* const tile = reinterpret_cast<float*>(mj_lds);
+    float *const ldsW = tile + kMrTile, *const ldsA = ldsW + kMrS, *const ldsM = ldsA + kMrS;  // pW, aS, pS
+    float4* const ldsD = reinterpret_cast<float4*>(tile + kMrTile);  // MrTwo: d
+    __shared__ float edge[2 * kMrN];
+    __shared__ int s_bad, s_next;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, T = q.y.T;
+    int g, t;
+    resident_unit(q.y.G, g, t);
+    // this thread's ring points: slot of the source, LDS offset and sign; and its points of the tile's edge: slot
+    int rslot[kRing], rlds[kRing], eslot[kRing];
+    bool rlane[kRing], rneed[kRing];
+#pragma unroll
+    for (int i = 0; i < kRing; ++i) {
+        const int e = tid + i * kMrThreads;
+        rlane[i] = e < 4 * kMrN;
+        const int4 re = rlane[i] ? q.ring[t * 4 * kMrN + e] : make_int4(0, 0, -1, 0);
+        rslot[i] = re.x;
+        rneed[i] = re.z >= 0;
+        rlds[i] = rlane[i] ? a.cring[a.ring_off[t] + e].z : 0;
+        eslot[i] = rlane[i] ? q.pub[t * 4 * kMrN + e] : -1;
+    }
+    uint64_t* const words = q.y.words + (size_t)g * q.y.group_words;
+    const unsigned ring_words = 4u * (unsigned)q.y.nslots;
+    const bool pA = lane >= kPartA && lane < kPartA + T, pB = lane >= kPartB && lane < kPartB + T;
+    const unsigned part_src = ring_words + (pB ? 4u * (unsigned)(lane - kPartB) + 2u : pA ? 4u * (unsigned)(lane - kPartA) : 0u);
+    unsigned seq = 0, members = 0;
+    if (tid == 0) s_bad = 0;
+
+    // the last exchange: ring values (RW words: 0 none, 1 FP32, 2 FP64) and the partial sums A, B of every tile. Every
+    // exchange waits for a sum of every tile, so that no word is overwritten before all have read it.
+    auto receive = [&](auto rw, bool B, double (&v)[kRing], double& sA, double& sB) {
+        double part = -0.0;
+        const unsigned odd = seq & 1;
+        const uint64_t* p[kRing];
+#pragma unroll
+        for (int i = 0; i < kRing; ++i) {
+            v[i] = 0.0;
+            p[i] = words + (2u * (unsigned)rslot[i] + odd * (ring_words >> 1));
+        }
+        if (!wait_words<decltype(rw)::value, kRing>(q.y, p, rneed, v, words + (part_src + odd * 4u * (unsigned)T),
+                                                    pA || (B && pB), part, seq) &&
+            lane == 0)
+            s_bad = 1;
+        part_sums(part, sA, sB);  // uniform
+        return part;
+    };
+    const std::integral_constant<int, 0> kNoRing{};
+    const std::integral_constant<int, 1> kRing32{};
+    const std::integral_constant<int, 2> kRing64{};
+    auto publish_part = [&](int k, double v) {
+        put_double(words + (ring_words + ((seq & 1) * (unsigned)T + (unsigned)t) * 4 + 2 * k), v, seq);
+    };
+    // the tile's edge values that other tiles read: of an array (written before a barrier), ...
+    auto send_edges64 = [&](const double* v) {
+#pragma unroll
+        for (int i = 0; i < kRing; ++i) {
+            const int e = anew(tid) + i * kMrThreads, o = e % kMrN;
+            const int j = e < kMrN ? 0 : e < 2 * kMrN ? kMrN - 1 : o, c = e < 2 * kMrN ? o : e < 3 * kMrN ? 0 : kMrN - 1;
+            if (eslot[i] >= 0)
+                put_double(words + (2u * (unsigned)eslot[i] + (seq & 1) * (ring_words >> 1)),
+                           v[t * a.plane + (a.OL + j) * a.nx + a.OL + c], seq);
+        }
+    };
+    // ... or those that keep_edges kept before a barrier
+    auto send_edges32 = [&]() {
+#pragma unroll
+        for (int i = 0; i < kRing; ++i) {
+            const int e = anew(tid) + i * kMrThreads;
+            const float* p = e < 2 * kMrN ? edge + e
+                                          : tile + (e % kMrN + 1) * kMrW + (e < 3 * kMrN ? 0 : 1);
+            if (eslot[i] >= 0) put_float(words + (2u * (unsigned)eslot[i] + (seq & 1) * (ring_words >> 1)), *p, seq);
+        }
+    };
+    // where the slots are, and which are a row's first or last (2 columns and padding)
+    int at[kMrSlots];
+    unsigned ends = 0;  // bit k: first in a row; bit 16 + k: last
+#pragma unroll
+    for (int k = 0; k < kMrSlots; ++k) {
+        const MrSlot P(tid + k * kMrThreads);
+        at[k] = P.j * kMrW + P.c4;
+        ends |= (P.c4 == 0 ? 1u : 0u) << k | (P.c4 + 4 > kMrN ? 0x10000u : 0u) << k;
+    }
+    asm volatile("" : "+v"(ends));
+    auto first = [&](int k) { return (ends >> k & 1u) != 0; };
+    auto last = [&](int k) { return (ends >> (16 + k) & 1u) != 0; };
+    const bool end = MrSlot(tid + (kMrSlots - 1) * kMrThreads).valid;  // the others always are
+    auto valid = [&](int k) { return k < kMrSlots - 1 || end; };
+    // the outermost rows and columns of v, for send_edges32 after a barrier
+    auto keep_edges = [&](const float4 (&v)[kMrSlots]) {
+        // row 0 is in block 0, row 89 in the last two
+        auto row = [&](int k, float4 e) {
+            const MrSlot P(anew(tid) + k * kMrThreads);
+            if (P.j != 0 && P.j != kMrN - 1) return;
+            float* p = edge + (P.j == 0 ? 0 : kMrN) + P.c4;
+            p[0] = e.x;
+            p[1] = e.y;
+            if (P.c4 + 4 <= kMrN) {
+                p[2] = e.z;
+                p[3] = e.w;
+            }
+        };
+        if (wave == 0) row(0, v[0]);
+#pragma unroll
+        for (int k = kMrSlots - 2; k < kMrSlots; ++k)
+            if (wave + k * kMrWaves >= kMrBlocks - 2) row(k, v[k]);
+#pragma unroll
+        for (int k = 0; k < kMrSlots; ++k) {
+            if (first(k)) tile[at[k] + kMrW] = v[k].x;
+            if (last(k)) tile[at[k] + kMrW - (kMrN - 2) + 1] = v[k].y;
+        }
+    };
+    static_assert(kMrNC <= 64 && (kMrN - 1) * kMrNC >= 64 * (kMrBlocks - 2) &&
+                      kMrBlocks - 2 >= (kMrSlots - 2) * kMrWaves, "rows 0 and 89");
+    auto put_tile = [&](const float4 (&v)[kMrSlots], const float (&ring)[kRing]) {
+#pragma unroll
+        for (int k = 0; k < kMrSlots; ++k) {
+            float* p = tile + at[k] + kMrAt;
+            if (last(k))
+                st2(p, make_float2(v[k].x, v[k].y));
+            else
+                st4(p, v[k]);
+        }
+#pragma unroll
+        for (int i = 0; i < kRing; ++i)
+            if (rlane[i]) tile[rlds[i] & ((1 << 30) - 1)] = (rlds[i] >> 30) & 1 ? -ring[i] : ring[i];
+    };
+    // o = A32 v or M32 v of the LDS tile; coef(k): the slot's coefficients, loaded one slot ahead (c0: the first's)
+    auto stencil = [&](auto isA, auto&& coef, MxCoef c, float4 (&o)[kMrSlots]) {
+#pragma unroll
+        for (int k = 0; k < kMrSlots; ++k) {
+            MxCoef next;
+            if (k + 1 < kMrSlots) next = coef(k + 1);
+            const float* x = tile + at[k] + kMrAt;
+            o[k] = stencil4<decltype(isA)::value>(c, c.wr, ld4(x - kMrW), ld4(x), ld4(x + kMrW), x[-1], x[4]);
+            o[k].z = last(k) ? 0.0f : o[k].z;
+            o[k].w = last(k) ? 0.0f : o[k].w;
+            // computed here, not at the first use, and before the loads of the slot after the next: otherwise every
+            // slot's loads come first and what they return is spilled
+            asm volatile("" : "+v"(o[k].x), "+v"(o[k].y), "+v"(o[k].z), "+v"(o[k].w) : : "memory");
+            c = next;
+        }
+    };
+    // the 64-slot block sums of one or two dot products (p's as dot product 0, h's as 1)
+    auto put_sum = [&](double s, int n, auto&& where) {  // where(i): the place of the i-th of n values
+        const int i = mr_lane(lane);
+        if (i >= 0 && i < n) g_rows[where(i)] = s;
+    };
+    auto block_sums1 = [&](const double (&p)[kMrSlots]) {
+        if constexpr (kMrSlots == 3)
+            put_sum(mr_trees(p[0], p[1], p[2], 0.0, 0.0, 0.0), 3, [&](int i) { return wave + i * kMrWaves; });
+        else
+            put_sum(mr_trees(p[0], p[1], p[2], p[3], p[4], 0.0), 5, [&](int i) { return wave + i * kMrWaves; });
+    };
+    auto block_sums2 = [&](const double (&p)[kMrSlots], const double (&h)[kMrSlots]) {
+        constexpr int k = kMrSlots - 3;
+        if constexpr (kMrSlots == 5)
+            put_sum(mr_trees(p[0], p[1], h[0], h[1], 0.0, 0.0), 4,
+                    [&](int i) { return (i & 2 ? 128 : 0) + wave + (i & 1) * kMrWaves; });
+        put_sum(mr_trees(p[k], p[k + 1], p[k + 2], h[k], h[k + 1], h[k + 2]), 6,
+                [&](int i) { return i < 3 ? wave + (k + i) * kMrWaves : 128 + wave + (k + i - 3) * kMrWaves; });
+    };
+    static_assert(kMrSlots == 3 || kMrSlots == 5, "block sums");
+    // after a barrier: dot product k (the block sums in order) as part `part` of the exchange
+    auto send_dot = [&](int k, int part) {
+        if (wave == k) {
+            const double* rb = g_rows + k * 128;
+            const int l = lane & 15;
+            const double s = add16(add16(0.0, rb[l]), rb[16 + l]) + rb[32];
+            if (lane == 0) publish_part(part, s);
+        }
+    };
+    // after a barrier: the FP64 tile sum of the row sums k
+    auto send_rows = [&](int k) {
+        if (wave == k) {
+            const double s = tile_of<MJ_SUM_TREE>(k, lane, nullptr, kMrN, kMrN);
+            if (lane == 0) publish_part(k, s);
+        }
+    };
+
+    for (;;) {
+        ++members;
+        if (tid == 0) {
+            s_next = next_member(q.y, g, t, members);
+            if (s_next < 0) s_bad = 1;
+        }
+        __syncthreads();
+        if (s_bad) break;
+        const int m = s_next;
+        if (m >= a.B) return;
+        double* const x = a.x + m * a.ms;
+        double* const r64 = a.r64 + m * a.ms;
+        const int tbase = t * a.plane + a.OL * a.nx + a.OL;
+        // the member's coefficients: FP32 copies in rows of kMrCPc floats, so that slot f is at 4 f
+        const int64_t oc = coef_base(a, m, t);
+        const float *const gaW = a.aW32 + oc, *const gaS = a.aS32 + oc, *const gaC = a.aC32 + oc;
+        const float *const gpW = a.pW32 + oc, *const gpS = a.pS32 + oc, *const gpC = a.pC32 + oc;
+        constexpr int kKept = F::kOnChip ? kMrSlots : 1;
+        float4 aW[kKept], aC[kKept], pC[kKept];
+        float aWr[kKept];
+        if constexpr (F::kOnChip) {
+#pragma unroll
+            for (int k = 0; k < kMrSlots; ++k) {
+                const MrSlot P(anew(tid) + k * kMrThreads);
+                aW[k] = ld4(gaW + 4 * P.f);
+                aC[k] = ld4(gaC + 4 * P.f);
+                pC[k] = ld4(gpC + 4 * P.f);
+                aWr[k] = gaW[4 * P.f + 4];
+            }
+        }
+        if constexpr (F::kOnChip) {
+            for (int i = tid; i < (kMrN + 1) * kMrNC; i += kMrThreads) {
+                const int j = i / kMrNC, o = j * kMrW + 4 * (i - j * kMrNC);
+                st4(ldsW + o, ld4(gpW + 4 * i));
+                st4(ldsA + o, ld4(gaS + 4 * i));
+                st4(ldsM + o, ld4(gpS + 4 * i));
+            }
+        }
+        // wr, W of the column after the slot, is unused in a row's last slot (its columns 2 and 3 are padding)
+        auto far = [&](const float* W, const float* S, const float* C, int k) {
+            const int slot = anew(tid) + k * kMrThreads;
+            const unsigned f = 16u * (unsigned)(k < kMrSlots - 1 ? slot : min(slot, kMrNS - 1));
+            auto at = [&](const float* p, int d) { return reinterpret_cast<const float*>((const char*)(p + d) + f); };
+            MxCoef c;
+            c.W = ld4(at(W, 0));
+            c.wr = *at(W, 4);
+            c.C = ld4(at(C, 0));
+            c.S0 = ld4(at(S, 0));
+            c.S1 = ld4(at(S, kMrCPc));
+            return c;
+        };
+        auto coefA = [&](int k) {
+            if constexpr (!F::kOnChip) return far(gaW, gaS, gaC, k);
+            MxCoef c;
+            c.W = aW[k % kKept];
+            c.wr = aWr[k % kKept];
+            c.C = aC[k % kKept];
+            c.S0 = ld4(ldsA + at[k]);
+            c.S1 = ld4(ldsA + at[k] + kMrW);
+            return c;
+        };
+        auto coefM = [&](int k) {
+            if constexpr (!F::kOnChip) return far(gpW, gpS, gpC, k);
+            MxCoef c;
+            c.W = ld4(ldsW + at[k]);
+            c.wr = ldsW[at[k] + 4];
+            c.C = pC[k % kKept];
+            c.S0 = ld4(ldsM + at[k]);
+            c.S1 = ld4(ldsM + at[k] + kMrW);
+            return c;
+        };
+        const std::true_type A{};
+        const std::false_type M{};
+        float4 r[kMrSlots], s[kMrSlots], zq[kMrSlots], d[kKept];
+        auto get_d = [&](int k) { return F::kOnChip ? d[k % kKept] : ldsD[k * kMrThreads + tid]; };
+        auto put_d = [&](int k, float4 v) {
+            if (F::kOnChip)
+                d[k % kKept] = v;
+            else
+                ldsD[k * kMrThreads + tid] = v;
+        };
+        float rring[kRing], sring[kRing] = {};
+        double v[kRing], sA, sB;
+
+        // ---- I0, I1
+        unit_I0(a, m, t);
+        ++seq;
+        if (tid == 0) publish_part(0, a.pmax[m * a.T + t]);
+        double rhsMax = 0.0;
+        {
+            const double part = receive(kNoRing, false, v, sA, sB);
+            for (int k = 0; k < T; ++k) rhsMax = fmax(rhsMax, lane_double(part, kPartA + k));
+        }
+        if (t == 0 && tid == 0) a.diag[m].rhsMax = rhsMax;
+        const double rhsNorm = uniform(rhsMax != 0.0 ? 1.0 / rhsMax : 1.0);
+        mx_first_rows(a, m, t, rhsNorm);
+        __syncthreads();
+        if (s_bad) break;
+        ++seq;
+        send_edges64(r64);
+        send_rows(0);
+        send_rows(1);
+
+        int n = 1, n0 = 1, iters = 0, outer = 0;
+        double sigma = 0.0, due = 0.0, eta = 0.0, etaP = 0.0, e = 0.0;  // due: a replacement when err is below
+        bool bad = false, fresh = false;
+        for (;;) {
+            // ---- RST: finish, or (re)place the recursive residual
+            receive(kRing64, outer == 0, v, e, sB);
+            if (outer == 0 && t == 0 && tid == 0) {
+                a.diag[m].firstResidual = sqrt(e);
+                a.diag[m].sumRHS = sB;
+                a.diag[m].launches = 0;
+            }
+            if (e < a.tol_sq || iters >= a.max_iters || outer >= a.max_outer) break;
+            if (outer == 0) sigma = uniform(sqrt(e));
+            n0 = n;
+            fresh = true;
+            ++outer;
+            due = uniform(fmax(a.itol_sq * (e / (sigma * sigma)), a.tol_sq / (sigma * sigma)));
+            {
+#pragma unroll
+                for (int k = 0; k < kMrSlots; ++k) {
+                    const MrSlot P(anew(tid) + k * kMrThreads);
+                    const double* p = r64 + tbase + P.j * a.nx + P.c4;
+                    const double2 R0 = ld2(p), R1 = ld2(p + 2);
+                    r[k] = mask_pad(make_float4((float)(R0.x / sigma), (float)(R0.y / sigma), (float)(R1.x / sigma),
+                                                (float)(R1.y / sigma)), P.c4, kMrN);
+                    put_d(k, make_float4(0.f, 0.f, 0.f, 0.f));
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < kRing; ++i) rring[i] = rneed[i] ? (float)(v[i] / sigma) : 0.0f;
+            put_tile(r, rring);
+            __syncthreads();
+            if ((bad = s_bad)) break;
+            ++seq;
+            stencil(M, coefM, coefM(0), zq);
+            keep_edges(zq);
+            {
+                double p[kMrSlots];
+#pragma unroll
+                for (int k = 0; k < kMrSlots; ++k) p[k] = valid(k) ? dot4(zq[k], r[k]) : 0.0;
+                block_sums1(p);
+            }
+            __syncthreads();
+            send_edges32();
+            send_dot(0, 0);
+            for (;;) {
+                // ---- IB(n): replacement rule on err(n-1); s = z + beta s, q = A32 s, sigma_n
+                double err;
+                receive(kRing32, !fresh, v, eta, err);
+                if (!fresh && (iters >= a.max_iters || n - n0 >= a.inner_max || err < due)) break;
+                fresh = false;
+                float w[kRing];  // the ring's z, then its q
+#pragma unroll
+                for (int i = 0; i < kRing; ++i) w[i] = __uint_as_float((unsigned)__double2loint(v[i]));
+                if (n == 1) {
+#pragma unroll
+                    for (int k = 0; k < kMrSlots; ++k) s[k] = zq[k];
+#pragma unroll
+                    for (int i = 0; i < kRing; ++i) sring[i] = rneed[i] ? w[i] : 0.0f;
+                } else {
+                    const float beta = (float)(eta / etaP);
+#pragma unroll
+                    for (int k = 0; k < kMrSlots; ++k) s[k] = axpy(beta, s[k], zq[k]);
+#pragma unroll
+                    for (int i = 0; i < kRing; ++i) sring[i] = rneed[i] ? w[i] + beta * sring[i] : 0.0f;
+                }
+                put_tile(s, sring);
+                __syncthreads();
+                if ((bad = s_bad)) break;
+                ++seq;
+                stencil(A, coefA, coefA(0), zq);
+                keep_edges(zq);
+                {
+                    double p[kMrSlots];
+#pragma unroll
+                    for (int k = 0; k < kMrSlots; ++k) p[k] = valid(k) ? dot4(s[k], zq[k]) : 0.0;
+                    block_sums1(p);
+                }
+                __syncthreads();
+                send_edges32();
+                send_dot(0, 0);
+                // ---- IC(n): d += alpha s, r32 -= alpha q, z = M32 r32, err(n), eta(n+1)
+                double sig, unused;
+                receive(kRing32, false, v, sig, unused);
+                const float alpha = (float)(eta / sig);
+#pragma unroll
+                for (int k = 0; k < kMrSlots; ++k) {
+                    put_d(k, axpy(alpha, s[k], get_d(k)));
+                    r[k] = axmy(alpha, zq[k], r[k]);
+                }
+#pragma unroll
+                for (int i = 0; i < kRing; ++i) {
+                    w[i] = __uint_as_float((unsigned)__double2loint(v[i]));
+                    rring[i] = rneed[i] ? rring[i] - alpha * w[i] : 0.0f;
+                }
+                put_tile(r, rring);
+                __syncthreads();
+                if ((bad = s_bad)) break;
+                ++seq;
+                stencil(M, coefM, coefM(0), zq);
+                keep_edges(zq);
+                {
+                    double p[kMrSlots], h[kMrSlots];
+#pragma unroll
+                    for (int k = 0; k < kMrSlots; ++k) {
+                        p[k] = valid(k) ? dot4(zq[k], r[k]) : 0.0;
+                        h[k] = valid(k) ? dot4(r[k], r[k]) : 0.0;
+                    }
+                    block_sums2(p, h);
+                }
+                __syncthreads();
+                send_edges32();
+                send_dot(0, 0);
+                send_dot(1, 1);
+                etaP = eta;
+                ++n;
+                ++iters;
+            }
+            if (bad) break;
+            // ---- the increment into x (FP64), then the true residual with the neighbours' x
+            {
+#pragma unroll
+                for (int k = 0; k < kMrSlots; ++k) {
+                    const MrSlot P(anew(tid) + k * kMrThreads);
+                    if (!P.valid) continue;
+                    double* p = x + tbase + P.j * a.nx + P.c4;
+                    const double2 X0 = ld2(p);
+                    const float4 D = get_d(k);
+                    st2(p, make_double2(X0.x + sigma * (double)D.x, X0.y + sigma * (double)D.y));
+                    if (P.c4 + 2 < kMrN) {
+                        const double2 X1 = ld2(p + 2);
+                        st2(p + 2, make_double2(X1.x + sigma * (double)D.z, X1.y + sigma * (double)D.w));
+                    }
+                }
+            }
+            __syncthreads();
+            ++seq;
+            send_edges64(x);
+            if (tid == 0) publish_part(0, 0.0);
+            receive(kRing64, false, v, sA, sB);
+#pragma unroll
+            for (int i = 0; i < kRing; ++i)  // no source: x keeps its halo value
+                if (rneed[i]) x[q.ring[t * 4 * kMrN + tid + i * kMrThreads].w] = (rlds[i] >> 30) & 1 ? -v[i] : v[i];
+            __syncthreads();
+            if ((bad = s_bad)) break;
+            ++seq;
+            mx_true_rows(a, m, t, rhsNorm);
+            __syncthreads();
+            send_edges64(r64);
+            send_rows(0);
+        }
+        if (bad) break;
+        mx_finish(a, m, t, rhsNorm);
+        if (t == 0 && tid == 0) {
+            a.diag[m].lastResidual = sqrt(e);
+            a.diag[m].numIters = iters;
+            a.diag[m].outerIters = outer;
+            a.diag[m].converged = e < a.tol_sq ? 1 : 0;
+        }
+        __syncthreads();
+    }
+    // a wait timed out: every member's record says so
+    for (int m = blockIdx.x * kMrThreads + tid; m < a.B; m += gridDim.x * kMrThreads) a.diag[m].converged = -2;
+}

@@ -2,6 +2,7 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include <stdint.h>
 
 #include <vector>
 
@@ -10,6 +11,25 @@
 
 namespace mj {
 constexpr int kResMaxTiles = 16;  // tiles of a member (a wave polls two partial sums of each at once)
+
+// What the workgroups of a resident solve share, in the workspace. A group is one workgroup per tile of a member.
+struct ResSync {
+    uint64_t* words;     // per group: [2][nslots][2] ring values, [2][T][4] partial sums, by parity of the exchange
+    size_t group_words;
+    uint64_t* next;      // [G] the group's current member
+    int* queue;          // members taken so far
+    int* error;          // a wait timed out
+    unsigned long long limit;  // ticks a wait may take
+    const int* order;    // [B] the order in which members are taken, or NULL (as they come)
+    int G, T, nslots, B;
+};
+// Fills y for a cooperative launch of kfn (threads, dynamic LDS) over cfg's batch and clears its words on the stream;
+// *ok false (and nothing enqueued) when the device or the workspace does not allow it. The launch has y->G * T blocks.
+int resident_prepare(const mj_halo_plan* P, const mj_cg2d_ops* ops, const mj_cg2d_config* cfg, const void* kfn,
+                     int threads, size_t lds, void* workspace, size_t workspace_bytes, hipStream_t st, ResSync* y,
+                     bool* ok);
+// Whether a stream is being captured into a graph (the resident launches are not for that).
+int stream_capturing(hipStream_t st, bool* capturing);
 
 // Whether the solve of this configuration can run resident (layout and plan).
 bool resident_fits(const mj_halo_plan* P, const mj_cg2d_config* c);

@@ -241,14 +241,17 @@ def _time(step: EnsembleStep, steps, warmup):
 
 
 def candidates(precision, B, T=13):
-    """Launch candidates for a batch of B members: persistent shapes only where the units fit one launch."""
+    """Launch candidates for a batch of B members: the library's own choice, then explicit shapes (persistent ones only
+    where the units fit one launch)."""
     out = []
     for ov in (False, True):
         if precision == "mixed":
             for itol in (1e-3, 1e-4):
+                out.append(StepConfig("mixed", "auto", 0, 0, itol, overlap=ov))
                 for bt in (256, 448, 512, 1024):
                     out.append(StepConfig("mixed", "phases", bt, 64, itol, overlap=ov))
         else:
+            out.append(StepConfig("fp64", "auto", 0, 0, overlap=ov))
             for bt in (128, 256, 512, 1024):
                 out.append(StepConfig("fp64", "phases", bt, 64, overlap=ov))
             if B * T <= 512:

@@ -36,7 +36,7 @@ def cg2d_mixed(ex, ops, cg2d_b, cg2d_x, *, cg2dNorm, tolerance, max_iters, out=N
     if x0.shape[0] != B:
         raise ValueError("cg2d_b and cg2d_x batch sizes differ")
     if launch not in ("phases", "phases_fixed", "auto"):
-        raise ValueError("the mixed solve runs as phase launches: launch must be 'phases' or 'phases_fixed'")
+        raise ValueError("the mixed solve's launch must be 'auto', 'phases' (both: the library's choice) or 'phases_fixed'")
     dev = b.device
     ops_s, ops_keep = _ops_struct(ops, B, L, dev, op_index)
     nslots = ops_keep[0].shape[0] if ops_keep[0].dim() == 4 else 1

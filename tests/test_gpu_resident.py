@@ -58,6 +58,29 @@ def test_resident_equals_phases(problem, B, order, tol, iters):
         assert torch.equal(d[k], dr[k]), k
 
 
+@pytest.mark.parametrize("B,kw", [
+    (1, {}), (1, dict(tolerance=1e6)), (3, dict(max_iters=1)), (19, dict(max_iters=37)), (20, dict(max_outer=2)),
+    (49, dict(inner_tolerance=1e-2)), (50, dict(max_iters=0)), (50, dict(inner_max_iters=20)), (61, {})])
+def test_mixed_resident_equals_steps(problem, B, kw):
+    """The mixed solve's resident launches (one workgroup per CU up to 49 members on 256 CUs, two beyond) against its
+    step launches."""
+    from mit_jax_amd import mixed
+    ex, cls, slots = problem
+    index = np.arange(B, dtype=np.int32)[::-1] % len(cls)
+    b, x0, norm = _inputs(ex, cls, B, index)
+    kw = dict(dict(tolerance=1e-11, max_iters=4000), **kw)
+    print(f"mixed resident: B={B} {kw}", flush=True)
+    x, d = mixed.cg2d_mixed(ex, slots, b, x0, cg2dNorm=norm, op_index=index, **kw)
+    torch.cuda.synchronize()
+    d.check()
+    xr, dr = mixed.cg2d_mixed(ex, slots, b, x0, cg2dNorm=norm, op_index=index, block_threads=512, **kw)
+    torch.cuda.synchronize()
+    assert int(d["launches"].max()) == 0 and int(dr["launches"].max()) > 0
+    assert torch.equal(x, xr)
+    for k in FIELDS:
+        assert torch.equal(d[k], dr[k]), k
+
+
 def test_resident_member_stride_and_stream(problem):
     """Members further apart than a field, on a side stream, twice into the same workspace."""
     import ctypes
