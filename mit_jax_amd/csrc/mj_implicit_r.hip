@@ -11,6 +11,8 @@
 // being built (a register ring with compile-time slots), so each lane keeps up to 5 x kPf loads in flight; the
 // columns of a wave are consecutive points of a row (coalesced). The per-level constants sit in LDS and the rows
 // between the first two and the last two run branch-free, so that no wait for a load is forced before its use.
+#include <type_traits>
+
 #include "mj_common.h"
 
 namespace mj {
@@ -408,40 +410,51 @@ extern "C" int mj_gad_implicit_r(const mj_impr_grid* g, const mj_impr_config* c,
 // u = A(kappaRX, wFld)^-1 y per column. Given ubar: lam = A^-T ubar by the same guarded elimination on the
 // transposed diagonals (row m of A^T = (e(m-2), d(m-1), c(m), b(m+1), a(m+2))), ybar = lam, and the cotangents of
 // kappaRX and wFld from the derivatives of the rows in those parameters (diffusion: b(k), d(k-1), c in kappaRX(k);
-// U3: rows K-1 and K in the rCenter of interface K). One thread per column; rows are built two ahead of the
-// transposed elimination, from level data read as needed (the reverse mode is not tuned).
+// U3: rows K-1 and K in the rCenter of interface K). One thread per column, in two walks over the levels.
+//
+// Bound by HBM: five arrays are read on the way down (the matrix and ubar), four on the way up (the parameter
+// cotangents), three written. Reading the level data as needed kept one or two loads in flight per lane (772 us for two
+// members of 50 levels, 1.7 TB/s of these twelve passes); now both walks run on register rings that load kPfA levels
+// ahead, in laps of kPfA rows without branches, and the parameter cotangents of interface m + 1 are formed as soon as
+// lam(m) is known, so that lam is not read back: 252 us, 4.8 TB/s, where a copy reaches 4.65 and reads alone 6. Six levels
+// ahead: four and eight measured within the spread of the runs, and eight no longer fit the registers. For the LLC90 level
+// count the walks are unrolled and y' stays in registers (NR; else it makes a round trip through the output column).
 namespace mj {
 namespace {
+
+#ifndef MJ_IMPR_PFA
+#define MJ_IMPR_PFA 6
+#endif
+constexpr int kPfA = MJ_IMPR_PFA;
+static_assert(kPfA >= 4, "the rings must hold the levels of a row");
 
 struct Row {
     double a, b, c, d, e;
 };
 
-template <bool ADV>
-__device__ Row build_row(const ImprArgs& a, const double* lv, int m, bool in, double rA, double rrA, const double* mCp,
-                         const double* rhp, const double* kp, const double* wp, Iface& up) {
-    const int nr = a.nr;
-    Row r{0.0, 0.0, 1.0, 0.0, 0.0};
-    if (!in) return r;
-    const int64_t P = a.plane;
-    const double dtm = lv[m], rdf = lv[nr + m], rh0 = rhp[m * P];
+// Row m of A from the level data of m - 1 .. m + 2 (mC1, mC0, mCn, mCk: maskC of m-1, m, m+1, min(nr-1, m+2); rh0 of m;
+// kap0, kapn of m, m+1; wn of m+1; up: interface m, replaced by interface m + 1). GEN as in impr_row.
+template <bool GEN, bool ADV>
+__device__ __forceinline__ Row adj_row(const ImprArgs& a, const double* lv, int nr, int m, bool in, double rA, double rrA,
+                                       double mC1, double mC0, double mCn, double mCk, double rh0, double kap0,
+                                       double kapn, double wn, Iface& up) {
+    const double dtm = lv[m], rdf = lv[nr + m];
     const double* rdrC = lv + 2 * nr;
-    const double mC0 = mCp[m * P], mC1 = m >= 1 ? mCp[(m - 1) * P] : 0.0;
-    const double mCn = m + 1 < nr ? mCp[(m + 1) * P] : 0.0;
-    if (m >= 1) r.b = -(((((dtm * mC1) * rh0) * rdf) * kp[m * P]) * rdrC[m]);
-    if (m + 1 < nr) r.d = -(((((dtm * mCn) * rh0) * rdf) * kp[(m + 1) * P]) * rdrC[m + 1]);
+    const bool hasU = !GEN || m >= 1, hasL = !GEN || m + 1 < nr;
+    Row r{0.0, 0.0, 0.0, 0.0, 0.0};
+    if (hasU) r.b = -(((((dtm * mC1) * rh0) * rdf) * kap0) * rdrC[m]);
+    if (hasL) r.d = -(((((dtm * mCn) * rh0) * rdf) * kapn) * rdrC[m + 1]);
     r.c = 1.0 - (r.b + r.d);
     if (ADV) {
         Iface lo{0.0, 0.0, 0.0, 0.0};
-        if (m + 1 < nr) {
-            const double mCk = m + 2 < nr ? mCp[(m + 2) * P] : mCn;
-            lo = iface(a, m + 1, wp[(m + 1) * P], rA, rrA, mC0, m >= 1 ? mC1 : mC0, mCk);
+        if (hasL) {
+            lo = iface(a, m + 1, wn, rA, rrA, mC0, (!GEN || m >= 1) ? mC1 : mC0, mCk);
             r.b = r.b - ((lo.km * dtm) * rh0) * rdf;
             r.c = r.c + (((((lo.rC + lo.rUp) + lo.km) * dtm) * rh0) * rdf);
             r.d = r.d + (((((lo.rC - lo.rUp) + lo.kp) * dtm) * rh0) * rdf);
             r.e = r.e - ((lo.kp * dtm) * rh0) * rdf;
         }
-        if (m >= 1) {
+        if (hasU) {
             r.a = r.a + ((up.km * dtm) * rh0) * rdf;
             r.b = r.b - (((((up.rC + up.rUp) + up.km) * dtm) * rh0) * rdf);
             r.c = r.c - (((((up.rC - up.rUp) + up.kp) * dtm) * rh0) * rdf);
@@ -449,123 +462,242 @@ __device__ Row build_row(const ImprArgs& a, const double* lv, int m, bool in, do
         }
         up = lo;
     }
+    if (!in) r = Row{0.0, 0.0, 1.0, 0.0, 0.0};  // halo columns: identity
     return r;
 }
 
+// Rows of A around the transposed elimination, and its last two rows.
+struct AdjState {
+    Row rM2, rM1, r0, rP1, rP2;
+    Iface up;
+    double mC1;
+    double dp1, ep1, yp1, dp2, ep2, yp2;
+};
+
+// Row m of A^T = (e(m-2), d(m-1), c(m), b(m+1), a(m+2)), eliminated.
+template <bool GEN>
+__device__ __forceinline__ void adj_eliminate(AdjState& c, int m, double y0) {
+    const double ra = c.rM2.e, rb = c.rM1.d, rc = c.r0.c, rd = c.rP1.b;
+    double dq, eq = c.rP2.a, yq;
+    if (GEN && m == 0) {
+        dq = rd;
+        yq = y0;
+        norm3(rc, dq, eq, yq);
+    } else if (GEN && m == 1) {
+        const double c2 = rc - rb * c.dp1;
+        dq = rd - rb * c.ep1;
+        yq = y0 - rb * c.yp1;
+        norm3(c2, dq, eq, yq);
+    } else {
+        const double bb = rb - ra * c.dp2;
+        const double cq = (rc - ra * c.ep2) - bb * c.dp1;
+        dq = rd - bb * c.ep1;
+        yq = (y0 - ra * c.yp2) - bb * c.yp1;
+        norm3(cq, dq, eq, yq);
+    }
+    c.dp2 = c.dp1, c.ep2 = c.ep1, c.yp2 = c.yp1;
+    c.dp1 = dq, c.ep1 = eq, c.yp1 = yq;
+}
+
+// Cotangents of kappaRX and wFld at interface k (levels k - 1 and k): lk, lk1 = lam(k), lam(k-1); u, maskC of the levels
+// k-2 .. k+1 (uM2, uM1, u0, uP1; likewise m..; clamped where they do not exist); rh0, rh1 of k, k-1; w of k.
 template <bool ADV>
+__device__ __forceinline__ void adj_params(const ImprArgs& a, const double* lv, int nr, int k, bool in, double rA,
+                                           double rrA, double lk, double lk1, double uM2, double uM1, double u0,
+                                           double uP1, double mM2, double mM1, double m0, double mP1, double rh0,
+                                           double rh1, double w, double& gk, double& gw) {
+    const double* rdrC = lv + 2 * nr;
+    const double beta = -((((lv[k] * mM1) * rh0) * lv[nr + k]) * rdrC[k]);
+    const double delta = -((((lv[k - 1] * m0) * rh1) * lv[nr + k - 1]) * rdrC[k]);
+    const double du = u0 - uM1;
+    gk = -((lk * beta) * (-du) + (lk1 * delta) * du);
+    gw = 0.0;
+    if (ADV) {
+        const double dw = (((0.5 * rA) * mM1) * rrA) * a.rkSign;
+        const double rC = ((0.5 * ((w * rA) * mM1)) * rrA) * a.rkSign;
+        const double sg = (double)((rC > 0.0) - (rC < 0.0));
+        const double mskM = mM2 * (k <= 1 ? 0.0 : 1.0);
+        const double mskP = mP1 * (k >= nr - 1 ? 0.0 : 1.0);
+        const double drUp = (2.0 * kSixth) * sg;
+        const double dkm = (kSixth * (1.0 + sg)) * mskM;
+        const double dkp = (kSixth * (1.0 - sg)) * mskP;
+        const double uKm2 = k >= 2 ? uM2 : 0.0, uKp1 = k + 1 < nr ? uP1 : 0.0;
+        const double phi = (((-dkm) * uKm2 + ((1.0 + drUp) + dkm) * uM1) + ((1.0 - drUp) + dkp) * u0) - dkp * uKp1;
+        const double s1 = (lv[k - 1] * rh1) * lv[nr + k - 1], s0 = (lv[k] * rh0) * lv[nr + k];
+        const double rCb = -((lk1 * s1) - (lk * s0)) * phi;
+        gw = rCb * dw;
+    }
+    if (!in) gk = 0.0, gw = 0.0;
+}
+
+template <bool ADV, int NR>
 __global__ void __launch_bounds__(kImprThreads)
-    impr_adjoint_kernel(ImprArgs a, const double* __restrict__ u, const double* __restrict__ ubar, double* ybar,
-                        double* kbar, double* wbar) {
+    impr_adjoint_kernel(ImprArgs a, const double* u, const double* ubar, double* ybar, double* kbar, double* wbar) {
     extern __shared__ double lds[];
     const int lane = threadIdx.x;
     const int64_t col = (int64_t)blockIdx.x * kImprThreads + lane;
     const int mem = blockIdx.y;
-    double* lv = lds + (int64_t)2 * a.nr * kImprThreads;
-    for (int k = lane; k < a.nr; k += kImprThreads) {
+    const int nr = NR ? NR : a.nr;
+    double* lv = lds + (int64_t)2 * nr * kImprThreads;
+    for (int k = lane; k < nr; k += kImprThreads) {
         lv[k] = a.dt[k];
-        lv[a.nr + k] = a.rdrF[k];
-        lv[2 * a.nr + k] = a.rdrC[k];
+        lv[nr + k] = a.rdrF[k];
+        lv[2 * nr + k] = a.rdrC[k];
     }
     __syncthreads();
     if (col >= (int64_t)a.T * a.plane) return;  // no barriers below
     const int t = (int)(col / a.plane), q = (int)(col - (int64_t)t * a.plane);
     const int j = q / a.nx, i = q - j * a.nx;
     const bool in = j >= a.OL && j < a.OL + a.sNy && i >= a.OL && i < a.OL + a.sNx;
-    const int nr = a.nr;
     const int64_t P = a.plane;
     const int64_t o3 = mem * a.ms3 + (int64_t)t * nr * P + q;
     const int64_t om = mem * a.mms + (int64_t)t * nr * P + q;
     const int64_t o2 = (int64_t)t * P + q;
-    const double rA = ADV && in ? a.rA[o2] : 0.0;
-    const double rrA = ADV && in ? a.recip_rA[o2] : 0.0;
-    const double *mCp = a.maskC + om, *rhp = a.rh + o3, *kp = a.kap + o3, *wp = a.w + o3;
-    const double *uc = u + o3, *ub = ubar + o3;
-    double* yb = ybar + o3;
-    double* dpL = lds + lane;
-    double* epL = lds + (int64_t)nr * kImprThreads + lane;
-    // transposed elimination, rows of A built two ahead
-    Iface up{0.0, 0.0, 0.0, 0.0};
+    const double rA = ADV ? a.rA[o2] : 0.0;
+    const double rrA = ADV ? a.recip_rA[o2] : 0.0;
+    // a halo column only needs ubar (identity rows): its other loads read those lines again
+    const double* const ub = ubar + o3;
+    const double* const mCp = in ? a.maskC + om : ub;
+    const double *const rhp = in ? a.rh + o3 : ub, *const kp = in ? a.kap + o3 : ub, *const wp = in ? a.w + o3 : ub;
+    const double* const uc = in ? u + o3 : ub;
+    double* const yb = ybar + o3;
+    double* const kb = kbar + o3;
+    double* const wbp = ADV ? wbar + o3 : nullptr;
+    double* const dpL = lds + lane;
+    double* const epL = lds + (int64_t)nr * kImprThreads + lane;
+    double ypR[NR ? NR : 1];
+
+    // ---- down: the rows of A, and two rows behind them those of A^T eliminated. Slot s of the rings holds a level r with
+    // r % kPfA == s; ubar's are read two levels behind.
     const Row zero{0.0, 0.0, 0.0, 0.0, 0.0};
-    Row rM2 = zero, rM1 = zero, r0 = zero, rP1 = zero, rP2 = zero;
-    double dp1 = 0.0, ep1 = 0.0, yp1 = 0.0, dp2 = 0.0, ep2 = 0.0, yp2 = 0.0;
-    for (int r = 0; r < nr + 2; ++r) {
-        rM2 = rM1, rM1 = r0, r0 = rP1, rP1 = rP2;
-        rP2 = r < nr ? build_row<ADV>(a, lv, r, in, rA, rrA, mCp, rhp, kp, wp, up) : zero;
-        const int m = r - 2;
-        if (m < 0) continue;
-        const double ra = rM2.e, rb = rM1.d, rc = r0.c, rd = rP1.b, re = rP2.a;  // row m of A^T
-        double dq, eq = re, yq;
-        const double y0 = ub[m * P];
-        if (m == 0) {
-            dq = rd;
-            yq = y0;
-            norm3(rc, dq, eq, yq);
-        } else if (m == 1) {
-            const double c2 = rc - rb * dp1;
-            dq = rd - rb * ep1;
-            yq = y0 - rb * yp1;
-            norm3(c2, dq, eq, yq);
-        } else {
-            const double bb = rb - ra * dp2;
-            const double cq = (rc - ra * ep2) - bb * dp1;
-            dq = rd - bb * ep1;
-            yq = (y0 - ra * yp2) - bb * yp1;
-            norm3(cq, dq, eq, yq);
-        }
-        dpL[(int64_t)m * kImprThreads] = dq;
-        epL[(int64_t)m * kImprThreads] = eq;
-        yb[m * P] = yq;
-        dp2 = dp1, ep2 = ep1, yp2 = yp1;
-        dp1 = dq, ep1 = eq, yp1 = yq;
-    }
-    if (nr >= 2) {
-        double u1 = yp1;
-        double u0 = yp2 - u1 * dpL[(int64_t)(nr - 2) * kImprThreads];
-        yb[(int64_t)(nr - 2) * P] = u0;
-        double u2 = u1;
-        u1 = u0;
-        for (int m = nr - 3; m >= 0; --m) {
-            const double v = (yb[m * P] - u1 * dpL[(int64_t)m * kImprThreads]) - u2 * epL[(int64_t)m * kImprThreads];
-            yb[m * P] = v;
-            u2 = u1;
-            u1 = v;
-        }
-    }
-    // parameter cotangents (interior columns; level 0 and the surface interface have none)
-    double* kb = kbar + o3;
-    double* wbp = ADV ? wbar + o3 : nullptr;
-    kb[0] = 0.0;
-    if (ADV) wbp[0] = 0.0;
-    const double* rdrC = lv + 2 * nr;
-    for (int k = 1; k < nr; ++k) {
-        double gk = 0.0, gw = 0.0;
-        if (in) {
-            const double lk = yb[k * P], lk1 = yb[(k - 1) * P];
-            const double uk = uc[k * P], uk1 = uc[(k - 1) * P];
-            const double mCk = mCp[k * P], mCk1 = mCp[(k - 1) * P];
-            const double rhk = rhp[k * P], rhk1 = rhp[(k - 1) * P];
-            const double beta = -((((lv[k] * mCk1) * rhk) * lv[nr + k]) * rdrC[k]);
-            const double delta = -((((lv[k - 1] * mCk) * rhk1) * lv[nr + k - 1]) * rdrC[k]);
-            const double du = uk - uk1;
-            gk = -((lk * beta) * (-du) + (lk1 * delta) * du);
-            if (ADV) {
-                const double dw = (((0.5 * rA) * mCk1) * rrA) * a.rkSign;
-                const double rC = ((0.5 * ((wp[k * P] * rA) * mCk1)) * rrA) * a.rkSign;
-                const double sg = (double)((rC > 0.0) - (rC < 0.0));
-                const double mskM = mCp[(k >= 2 ? k - 2 : 0) * P] * (k <= 1 ? 0.0 : 1.0);
-                const double mskP = mCp[(k + 1 < nr ? k + 1 : nr - 1) * P] * (k >= nr - 1 ? 0.0 : 1.0);
-                const double drUp = (2.0 * kSixth) * sg;
-                const double dkm = (kSixth * (1.0 + sg)) * mskM;
-                const double dkp = (kSixth * (1.0 - sg)) * mskP;
-                const double uKm2 = k >= 2 ? uc[(k - 2) * P] : 0.0, uKp1 = k + 1 < nr ? uc[(k + 1) * P] : 0.0;
-                const double phi = (((-dkm) * uKm2 + ((1.0 + drUp) + dkm) * uk1) + ((1.0 - drUp) + dkp) * uk) - dkp * uKp1;
-                const double s1 = (lv[k - 1] * rhk1) * lv[nr + k - 1], s0 = (lv[k] * rhk) * lv[nr + k];
-                const double rCb = -((lk1 * s1) - (lk * s0)) * phi;
-                gw = rCb * dw;
+    AdjState c{zero, zero, zero, zero, zero, {0.0, 0.0, 0.0, 0.0}, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    {
+        double rmC[kPfA], rrh[kPfA], rkap[kPfA], rw[kPfA], ry[kPfA];
+        auto load = [&](int s, int r) {
+            const int64_t ok = (int64_t)(NR ? (r < NR ? r : NR - 1) : min(r, nr - 1)) * P;
+            rmC[s] = mCp[ok];
+            rrh[s] = rhp[ok];
+            rkap[s] = kp[ok];
+            rw[s] = ADV ? wp[ok] : 0.0;
+            ry[s] = ub[ok];
+        };
+        double yB1 = 0.0, yB2 = 0.0;  // ubar of levels r - 1, r - 2
+        auto step = [&](auto gen, int r, int s) {
+            constexpr bool GEN = decltype(gen)::value;
+            const int s1 = (s + 1) % kPfA, s2 = (s + 2) % kPfA;
+            c.rM2 = c.rM1, c.rM1 = c.r0, c.r0 = c.rP1, c.rP1 = c.rP2;
+            c.rP2 = zero;
+            if (!GEN || r < nr) {
+                const double mCk = !GEN || r + 2 < nr ? rmC[s2] : rmC[s1];
+                c.rP2 = adj_row<GEN, ADV>(a, lv, nr, r, in, rA, rrA, c.mC1, rmC[s], rmC[s1], mCk, rrh[s], rkap[s],
+                                          rkap[s1], rw[s1], c.up);
+                c.mC1 = rmC[s];
             }
+            const int m = r - 2;
+            if (!GEN || m >= 0) {
+                adj_eliminate<GEN>(c, m, yB2);
+                dpL[(int64_t)m * kImprThreads] = c.dp1;
+                epL[(int64_t)m * kImprThreads] = c.ep1;
+                if constexpr (NR != 0)
+                    ypR[m >= 0 ? m : 0] = c.yp1;
+                else
+                    yb[m * P] = c.yp1;
+            }
+            yB2 = yB1;
+            yB1 = ry[s];
+            load(s, r + kPfA);
+        };
+#pragma unroll
+        for (int s = 0; s < kPfA; ++s) load(s, s);
+        if constexpr (NR != 0) {
+#pragma unroll
+            for (int r = 0; r < NR + 2; ++r) {
+                if (r < 4 || r > NR - 3)
+                    step(std::true_type{}, r, r % kPfA);
+                else
+                    step(std::false_type{}, r, r % kPfA);
+            }
+        } else {
+            // the first lap, laps of interior rows, the rest
+#pragma unroll
+            for (int s = 0; s < kPfA; ++s)
+                if (s < nr + 2) step(std::true_type{}, s, s);
+            int r0 = kPfA;
+            for (; r0 + kPfA - 1 <= nr - 3; r0 += kPfA) {
+#pragma unroll
+                for (int s = 0; s < kPfA; ++s) step(std::false_type{}, r0 + s, s);
+            }
+#pragma unroll
+            for (int s = 0; s < kPfA + 4; ++s)
+                if (r0 + s < nr + 2) step(std::true_type{}, r0 + s, s % kPfA);
         }
-        kb[k * P] = gk;
-        if (ADV) wbp[k * P] = gw;
+    }
+    // ---- up: lam(m), and with it the cotangents at interface k = m + 1. Slot s of the rings holds level l = m - 1 of step
+    // m, counted down from nr - 1: l = nr - 1 - n with n % kPfA == s.
+    {
+        double rmC[kPfA], rrh[kPfA], rw[kPfA], ru[kPfA], ry[kPfA];
+        auto load = [&](int s, int n) {
+            const int64_t ok = (int64_t)max(nr - 1 - n, 0) * P;
+            rmC[s] = mCp[ok];
+            rrh[s] = rhp[ok];
+            if (ADV) rw[s] = wp[ok];
+            ru[s] = uc[ok];
+            if (NR == 0) ry[s] = yb[ok];
+        };
+#pragma unroll
+        for (int s = 0; s < kPfA; ++s) load(s, s);
+        // levels m + 2, m + 1, m of the window (index 0, 1, 2) and the new level m - 1
+        double W_m[3] = {0.0, 0.0, 0.0}, W_u[3] = {0.0, 0.0, 0.0}, W_rh[3] = {0.0, 0.0, 0.0}, W_w[3] = {0.0, 0.0, 0.0};
+        double W_y = 0.0, u1 = 0.0, u2 = 0.0;
+        auto step = [&](int n, int s) {  // takes level l = nr - 1 - n in; finishes m = l + 1
+            const int m = nr - n;
+            const double nm = rmC[s], nu = ru[s], nrh = rrh[s], nw = ADV ? rw[s] : 0.0;
+            if (m < nr) {  // lam(m)
+                const double y = NR ? ypR[m < 0 ? 0 : m] : W_y;
+                double v;
+                if (m == nr - 1)
+                    v = y;
+                else if (m == nr - 2)
+                    v = y - u1 * dpL[(int64_t)m * kImprThreads];
+                else
+                    v = (y - u1 * dpL[(int64_t)m * kImprThreads]) - u2 * epL[(int64_t)m * kImprThreads];
+                yb[m * P] = v;
+                const int k = m + 1;
+                if (k < nr) {
+                    double gk, gw;
+                    // mask of level k + 1 clamped to nr - 1, of level k - 2 to 0 (nm repeats level 0 there)
+                    const double mP1 = k + 1 < nr ? W_m[0] : W_m[1];
+                    adj_params<ADV>(a, lv, nr, k, in, rA, rrA, u1, v, nu, W_u[2], W_u[1], W_u[0], nm, W_m[2], W_m[1], mP1,
+                                    W_rh[1], W_rh[2], W_w[1], gk, gw);
+                    kb[k * P] = gk;
+                    if (ADV) wbp[k * P] = gw;
+                }
+                u2 = u1;
+                u1 = v;
+            }
+            W_m[0] = W_m[1], W_m[1] = W_m[2], W_m[2] = nm;
+            W_u[0] = W_u[1], W_u[1] = W_u[2], W_u[2] = nu;
+            W_rh[0] = W_rh[1], W_rh[1] = W_rh[2], W_rh[2] = nrh;
+            W_w[0] = W_w[1], W_w[1] = W_w[2], W_w[2] = nw;
+            if (NR == 0) W_y = ry[s];
+            load(s, n + kPfA);
+        };
+        // n = 0 takes level nr - 1 in; n = nr (level 0 again) finishes m = 0
+        if constexpr (NR != 0) {
+#pragma unroll
+            for (int n = 0; n <= NR; ++n) step(n, n % kPfA);
+        } else {
+            int n0 = 0;
+            for (; n0 + kPfA - 1 <= nr; n0 += kPfA) {
+#pragma unroll
+                for (int s = 0; s < kPfA; ++s) step(n0 + s, s);
+            }
+#pragma unroll
+            for (int s = 0; s < kPfA; ++s)
+                if (n0 + s <= nr) step(n0 + s, s);
+        }
+        kb[0] = 0.0;  // level 0 and the surface interface have none
+        if (ADV) wbp[0] = 0.0;
     }
 }
 
@@ -620,16 +752,15 @@ extern "C" int mj_gad_implicit_r_adjoint(const mj_impr_grid* g, const mj_impr_co
     a.out = nullptr;
     hipStream_t st = as_stream(stream);
     const size_t lds = ((size_t)2 * c->nr * kImprThreads + 3 * (size_t)c->nr) * sizeof(double);
-    const void* kern = a.adv ? (const void*)impr_adjoint_kernel<true> : (const void*)impr_adjoint_kernel<false>;
-    if (lds > 65536) MJ_HIP(hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    using Kern = void (*)(ImprArgs, const double*, const double*, double*, double*, double*);
+    const Kern kern = c->nr == 50 ? (a.adv ? impr_adjoint_kernel<true, 50> : impr_adjoint_kernel<false, 50>)
+                                  : (a.adv ? impr_adjoint_kernel<true, 0> : impr_adjoint_kernel<false, 0>);
+    if (lds > 65536)
+        MJ_HIP(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     const int64_t cols = (int64_t)c->ntiles * plane;
     const dim3 grid((unsigned)((cols + kImprThreads - 1) / kImprThreads), (unsigned)c->batch);
-    if (a.adv)
-        hipLaunchKernelGGL(impr_adjoint_kernel<true>, grid, dim3(kImprThreads), lds, st, a, u, ubar, ybar,
-                           kappaRX_bar, wFld_bar);
-    else
-        hipLaunchKernelGGL(impr_adjoint_kernel<false>, grid, dim3(kImprThreads), lds, st, a, u, ubar, ybar,
-                           kappaRX_bar, (double*)nullptr);
+    hipLaunchKernelGGL(kern, grid, dim3(kImprThreads), lds, st, a, u, ubar, ybar, kappaRX_bar,
+                       a.adv ? wFld_bar : (double*)nullptr);
     MJ_HIP(hipGetLastError());
     return MJ_OK;
 }

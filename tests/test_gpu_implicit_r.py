@@ -124,6 +124,37 @@ def test_gad_implicit_r_other_level_counts(dev, K):
     assert np.array_equal(got.cpu().numpy(), ref)
 
 
+@pytest.mark.parametrize("adv", [True, False])
+@pytest.mark.parametrize("K", [2, 3, 4, 5, 6, 7, 8, 10, 11, 16, 17, 64])
+def test_gad_implicit_r_adjoint_other_level_counts(dev, K, adv):
+    """The reverse sweeps at level counts around the laps of their rings (which hold six levels; the first and the last
+    rows run on their own), two members: equal to the oracle's reverse mode to 1e-12 relative, as for 50 levels."""
+    import torch
+    from mit_jax_amd import tracer_implicit as TI
+    g, p, kap, w, tr = _inputs()
+    lev = np.arange(K) % g.maskC.shape[1]
+    sl = lambda a: np.ascontiguousarray(np.asarray(a)[:, lev])  # noqa: E731
+    gk = SimpleNamespace(layout=g.L, maskC=sl(g.maskC), rA=g.rA, recip_rA=g.recip_rA,
+                         recip_drF=np.asarray(g.v["recip_drF"])[lev], recip_drC=np.asarray(g.v["recip_drC"])[lev])
+    pk = SimpleNamespace(dTtracerLev=np.asarray(p.dTtracerLev)[lev], implicitDiffusion=True, rkSign=-1.0)
+    rng = np.random.default_rng(23)
+    fields = [(sl(kap), sl(w), sl(tr), rng.normal(size=sl(tr).shape))]
+    fields.append((0.3 * sl(kap), -0.5 * sl(w), rng.normal(size=sl(tr).shape), rng.normal(size=sl(tr).shape)))
+    two = lambda i: torch.stack([to_dev(f[i], dev) for f in fields])  # noqa: E731
+    rh = sl(g.recip_hFacC)
+    print(f"gad_implicit_r_adjoint: {K} levels, implicitAdvection={adv}", flush=True)
+    got = TI.gad_implicit_r_adjoint(pk, gk, adv, 3, two(0), to_dev(rh, dev).expand(2, *rh.shape).contiguous(), two(1),
+                                    two(2), two(3))
+    for m, (k, ww, u, ub) in enumerate(fields):
+        ref = OI.gad_implicit_r_adjoint(pk, gk, adv, k, rh, ww, u, ub)
+        for name, a, b in zip(("ybar", "kappaRX_bar", "wFld_bar"), got, ref):
+            if a is None:
+                assert not adv and name == "wFld_bar"
+                continue
+            a = a[m].cpu().numpy()
+            assert np.abs(a - b).max() <= 1e-12 * np.abs(b).max(), (name, m)
+
+
 def test_gad_implicit_r_refuses_mismatched_shapes(dev):
     """Forward and reverse mode refuse arrays whose shape differs from the tracer's (the kernels index every array
     with the tracer's strides) before any launch."""
