@@ -377,11 +377,12 @@ int mj_dst3_adv_y(const mj_dst3_flux_config* cfg, double oneSixth, const double*
  * test_gad.py:297-346 does; the R flux, which the reference does not have, differentiated the same way): for the
  * cotangent gTracer_bar of gTracer, writes the cotangents of tracer, uFld and vFld, and with wFld that of wFld
  * (every padded point of [B][T, nr, ny, nx]; levels at or beyond a member's nlev get 0; w at the surface
- * interface, which the R flux does not read, gets 0). The grid, hFac and mask inputs are constants. With wFld the
- * horizontal passes are replayed forward once (localTij into work), the vertical sweep is reversed per column,
- * then the horizontal sweeps per (member, tile, level). work: device, 256-byte aligned, of
- * mj_gad_dst3_adjoint_workspace_bytes(cfg, ntiles, wFld != NULL) bytes (the mask bit planes as in mj_gad_dst3, and the
- * replay scratch). Outputs must not alias inputs or each other. */
+ * interface, which the R flux does not read, gets 0). The grid, hFac and mask inputs are constants. In launches of at
+ * most 1024 (member, tile, level)s (whole columns, at least one) the horizontal passes are replayed forward (the tile
+ * before each sweep, and with wFld localTij, into work), with wFld the vertical sweep is reversed per column, then the
+ * horizontal sweeps per (member, tile, level). work: device, 256-byte aligned, of
+ * mj_gad_dst3_adjoint_workspace_bytes(cfg, ntiles, wFld != NULL) bytes (the mask bit planes as in mj_gad_dst3, and
+ * these). Outputs must not alias inputs or each other. */
 size_t mj_gad_dst3_adjoint_workspace_bytes(const mj_gad_config* cfg, int ntiles, int with_w);
 int mj_gad_dst3_adjoint(const mj_gad_plan* plan, const mj_gad_grid* grid, const mj_gad_config* cfg,
                         const double* uFld, const double* vFld, const double* wFld, const double* tracer,

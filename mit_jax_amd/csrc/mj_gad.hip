@@ -37,16 +37,18 @@ struct GadDev {
     const double *u, *v, *w, *tr, *hFacW, *hFacS, *recip_hFacC;
     double* out;  // gTracer (no R flux) or localTij after the horizontal passes (R flux follows)
     const int32_t* nlev;
-    unsigned long long* mbits;  // maskLocW / maskLocS bit planes per (mask slot, tile, level), gad_maskbits_kernel
+    unsigned* mbits;  // maskLocW / maskLocS bit planes per (mask slot, tile, level), gad_maskbits_kernel
     double2* g2;  // per tile, the 2-D metrics a sweep point reads, in pairs (gad_pack2d_kernel): [3][T][GPLANE]
                   // {dyG, recip_dxC} (X faces), {dxG, recip_dyC} (Y faces), {recip_rA, maskInC}
 };
 
 // Mask slot of member m: members of one level class share their grid masks.
 __device__ __forceinline__ int64_t mask_slot(const GadDev& a, int m) { return a.mask_index ? a.mask_index[m] : m; }
-constexpr int kMaskWords = (GPLANE + 63) / 64;
+// A bit plane: four words a row, bit i of a row in its word i / 32 (one column has the same shift in all rows).
+constexpr int kRowWords = 4, kMaskWords = GNY * kRowWords;
+static_assert(GNX <= 32 * kRowWords && GNX > 64, "two wavefronts' ballots a row");
 // The bit planes of member m's masks at (tile t, level k): maskLocW's kMaskWords words, then maskLocS's.
-__device__ __forceinline__ const unsigned long long* unit_bits(const GadDev& a, int m, int t, int k) {
+__device__ __forceinline__ const unsigned* unit_bits(const GadDev& a, int m, int t, int k) {
     const int64_t s = a.mms ? mask_slot(a, m) : 0;
     return a.mbits + ((s * a.T + t) * a.K + k) * 2 * kMaskWords;
 }
@@ -111,27 +113,31 @@ __device__ __forceinline__ bool corner_pair(const GadDev& a, const MjTilePlan& t
 
 // The fill on a tile (LDS or the block's own global plane): all reads precede all writes.
 __device__ __forceinline__ void corner_fill(double* loc, const GadDev& a, const MjTilePlan& tp, int dir, int tid) {
-    int dst = -1, src = -1;
-    double v = 0.0;
-    const bool on = corner_pair(a, tp, dir, tid, dst, src);
-    if (on) v = loc[src];
-    __syncthreads();
-    if (on) loc[dst] = v;
-    __syncthreads();
+    for (int n0 = 0; n0 < 4 * a.OLx * a.OLx; n0 += blockDim.x) {
+        int dst = -1, src = -1;
+        double v = 0.0;
+        const bool on = corner_pair(a, tp, dir, n0 + tid, dst, src);
+        if (on) v = loc[src];
+        __syncthreads();
+        if (on) loc[dst] = v;
+        __syncthreads();
+    }
 }
 
 // Transpose of the fill on a cotangent plane: the destination's cotangent moves to its source.
 __device__ __forceinline__ void corner_fill_T(double* bar, const GadDev& a, const MjTilePlan& tp, int dir, int tid) {
-    int dst = -1, src = -1;
-    double v = 0.0;
-    const bool on = corner_pair(a, tp, dir, tid, dst, src);
-    if (on) v = bar[dst];
-    __syncthreads();
-    if (on) {
-        bar[src] = bar[src] + v;
-        bar[dst] = 0.0;
+    for (int n0 = 0; n0 < 4 * a.OLx * a.OLx; n0 += blockDim.x) {
+        int dst = -1, src = -1;
+        double v = 0.0;
+        const bool on = corner_pair(a, tp, dir, n0 + tid, dst, src);
+        if (on) v = bar[dst];
+        __syncthreads();
+        if (on) {
+            bar[src] = bar[src] + v;
+            bar[dst] = 0.0;
+        }
+        __syncthreads();
     }
-    __syncthreads();
 }
 
 // Unit (tile, member, level block) of a DST3 launch of gridDim.x >= B*T*ceil(K/L) blocks (a multiple of 8, L =
@@ -152,74 +158,57 @@ __device__ __forceinline__ bool gad_unit(const GadDev& a, int& t, int& m, int& k
     return true;
 }
 
-// The points of the corner squares of the corners the tile has: mask_loc (corner-filled) into the bit planes.
-__device__ __forceinline__ void fix_mask_corners(const GadDev& a, const MjTilePlan& tp, const double* mW,
-                                                 const double* mS, unsigned long long* bw, unsigned long long* bs) {
-    // corner c (sw, se, nw, ne), point p of its OL x OL square, mask u (W) or v (S)
+// maskLocW / maskLocS of every (mask slot, tile, level) as bit planes in global memory, once per call: the DST3
+// blocks of the members that share a slot load its words instead of the two mask planes (2 x 77 KB). The masks are 0/1 by
+// construction (hFac != 0), so a bit and its double 0.0/1.0 carry the same value. Off the four corner halo squares mask_loc
+// is the plain mask, so every wave ballots half rows of maskW / maskS; then the points of the corner squares of the corners
+// the tile has are set from mask_loc.
+//
+// One workgroup per mask plane, all its loads in flight at once: one member of 50 levels (100 MB) took 49 us with both
+// planes in a workgroup of 256 threads and 16 words at a time; 38 us now.
+constexpr int kBitsThreads = 512;
+__global__ void __launch_bounds__(kBitsThreads) gad_maskbits_kernel(GadDev a, int nslots) {
+    __shared__ unsigned b[kMaskWords];
+    const int u = blockIdx.x >> 1, want_u = !(blockIdx.x & 1);
+    const int k = u % a.K, st = u / a.K, t = st % a.T, sl = st / a.T;
+    if (sl >= nslots) return;
+    const MjTilePlan& tp = a.tiles[t];
+    const int64_t bm = sl * a.mms + ((int64_t)t * a.K + k) * GPLANE;
+    const double *const mW = a.maskW + bm, *const mS = a.maskS + bm, *const mk = want_u ? mW : mS;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    constexpr int NW = kBitsThreads / 64, N = (2 * GNY + NW - 1) / NW;  // half rows of a wave
+    double v[N];
+#pragma unroll
+    for (int r = 0; r < N; ++r) {
+        const int h = wave + r * NW, j = h >> 1, i = (h & 1) * 64 + lane;
+        v[r] = h < 2 * GNY && i < GNX ? mk[j * GNX + i] : 0.0;
+    }
+#pragma unroll
+    for (int r = 0; r < N; ++r) {
+        const int h = wave + r * NW;
+        const unsigned long long w = __ballot(v[r] != 0.0);
+        if (lane < 2 && h < 2 * GNY) b[2 * h + lane] = (unsigned)(w >> (32 * lane));
+    }
+    __syncthreads();
+    // corner c (sw, se, nw, ne), point p of its OL x OL square
     const int OL = a.OLx, n = 4 * OL * OL;
-    const int tid = threadIdx.x;
-    if (tid < 2 * n) {
-        const int want_u = tid < n, r = tid % n, c = r / (OL * OL), pp = r % (OL * OL);
+    for (int r = tid; r < n; r += kBitsThreads) {
+        const int c = r / (OL * OL), pp = r % (OL * OL);
         const bool on = c == 0 ? tp.sw : c == 1 ? tp.se : c == 2 ? tp.nw : tp.ne;
         if (on) {
             const int dj = pp / OL, di = pp % OL;
             const int ja = (c < 2) ? dj : a.OLy + a.sNy + dj, ia = (c % 2 == 0) ? di : a.OLx + a.sNx + di;
-            const int q = ja * GNX + ia;
-            const bool v = mask_loc(a, tp, mW, mS, ja, ia, want_u) != 0.0;
-            unsigned long long* word = (want_u ? bw : bs) + (q >> 6);
-            const unsigned long long bit = 1ull << (q & 63);
-            if (v)
+            unsigned* word = b + ja * kRowWords + (ia >> 5);
+            const unsigned bit = 1u << (ia & 31);
+            if (mask_loc(a, tp, mW, mS, ja, ia, want_u) != 0.0)
                 atomicOr(word, bit);
             else
                 atomicAnd(word, ~bit);
         }
     }
     __syncthreads();
-}
-
-// maskLocW / maskLocS of one (member, tile, level) as LDS bit planes (the masks are 0/1 by construction, hFac != 0,
-// so a bit and its double 0.0/1.0 carry the same value). Off the four corner halo squares mask_loc is the plain
-// mask, so every wave ballots the plain maskW / maskS of its words (all its loads in flight at once); then the
-// points of the corner squares of the corners the tile has are set from mask_loc.
-__device__ __forceinline__ void build_mask_bits(const GadDev& a, const MjTilePlan& tp, const double* mW,
-                                                const double* mS, unsigned long long* bw, unsigned long long* bs) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nwaves = blockDim.x >> 6;
-    constexpr int kWordsPerWave = 16;  // words of one wave whose loads are issued together
-    for (int w0 = wave; w0 < kMaskWords; w0 += nwaves * kWordsPerWave) {
-        double vw[kWordsPerWave], vs[kWordsPerWave];
-#pragma unroll
-        for (int r = 0; r < kWordsPerWave; ++r) {
-            const int q = (w0 + r * nwaves) * 64 + lane;
-            const bool in = w0 + r * nwaves < kMaskWords && q < GPLANE;
-            vw[r] = in ? mW[q] : 0.0;
-            vs[r] = in ? mS[q] : 0.0;
-        }
-#pragma unroll
-        for (int r = 0; r < kWordsPerWave; ++r) {
-            const unsigned long long bwv = __ballot(vw[r] != 0.0), bsv = __ballot(vs[r] != 0.0);
-            if (lane == 0 && w0 + r * nwaves < kMaskWords) {
-                bw[w0 + r * nwaves] = bwv;
-                bs[w0 + r * nwaves] = bsv;
-            }
-        }
-    }
-    __syncthreads();
-    fix_mask_corners(a, tp, mW, mS, bw, bs);
-}
-// maskLocW / maskLocS of every (mask slot, tile, level) as bit planes in global memory, once per call: the DST3
-// blocks of the members that share a slot load its 2 x 151 words instead of the two mask planes (2 x 77 KB).
-__global__ void __launch_bounds__(256) gad_maskbits_kernel(GadDev a, int nslots) {
-    __shared__ unsigned long long bw[kMaskWords], bs[kMaskWords];
-    const int u = blockIdx.x;
-    const int k = u % a.K, st = u / a.K, t = st % a.T, sl = st / a.T;
-    if (sl >= nslots) return;
-    const int64_t bm = sl * a.mms + ((int64_t)t * a.K + k) * GPLANE;
-    build_mask_bits(a, a.tiles[t], a.maskW + bm, a.maskS + bm, bw, bs);
-    unsigned long long* o = a.mbits + (int64_t)u * 2 * kMaskWords;
-    for (int i = threadIdx.x; i < kMaskWords; i += blockDim.x) {
-        o[i] = bw[i];
-        o[kMaskWords + i] = bs[i];
-    }
+    unsigned* o = a.mbits + (int64_t)blockIdx.x * kMaskWords;
+    for (int i = tid; i < kMaskWords; i += kBitsThreads) o[i] = b[i];
 }
 
 // The 2-D metrics in the pairs the sweeps load together (one 16-byte load instead of two 8-byte ones), per call.
@@ -234,8 +223,8 @@ __global__ void __launch_bounds__(256) gad_pack2d_kernel(GadDev a) {
 
 // The tracer plane into LDS (into loc and loc2) and the unit's mask bit planes, all loads in flight together (one
 // memory latency for a 1024-thread block).
-__device__ __forceinline__ void load_tile_and_bits(const double* tr, const unsigned long long* gb, double* loc,
-                                                   double* loc2, unsigned long long* bw, unsigned long long* bs) {
+__device__ __forceinline__ void load_tile_and_bits(const double* tr, const unsigned* gb, double* loc,
+                                                   double* loc2, unsigned* bw, unsigned* bs) {
     const int tid = threadIdx.x, nthr = blockDim.x;
     constexpr int KP = (GPLANE + 1023) / 1024;  // per thread at 1024
     for (int it = 0; it * KP * nthr < GPLANE || it * nthr < 2 * kMaskWords; ++it) {
@@ -246,7 +235,7 @@ __device__ __forceinline__ void load_tile_and_bits(const double* tr, const unsig
             v[b] = q < GPLANE ? tr[q] : 0.0;
         }
         const int wd = it * nthr + tid;
-        const unsigned long long word = wd < 2 * kMaskWords ? gb[wd] : 0ull;
+        const unsigned word = wd < 2 * kMaskWords ? gb[wd] : 0u;
 #pragma unroll
         for (int b = 0; b < KP; ++b) {
             const int q = (it * KP + b) * nthr + tid;
@@ -260,22 +249,9 @@ __device__ __forceinline__ void load_tile_and_bits(const double* tr, const unsig
     __syncthreads();
 }
 
-__device__ __forceinline__ double mbit(const unsigned long long* b, int q) {
-    return (double)((b[q >> 6] >> (q & 63)) & 1ull);
-}
-
-// The interface fluxes a sweep's update reads: faces q and q + d (d = 1 in X, GNX in Y) of every box point.
-template <class F>
-__device__ __forceinline__ void flux_boxes(const MjSweep& S, int dir, double* af, F&& flux) {
-    for (int bx = 0; bx < S.nbox; ++bx) {
-        const MjBox B = S.box[bx];
-        const int i1 = B.i1 + (dir == 0 ? 1 : 0), j1 = B.j1 + (dir == 1 ? 1 : 0);
-        const int bw = i1 - B.i0, n = bw * (j1 - B.j0);
-        for (int idx = threadIdx.x; idx < n; idx += blockDim.x) {
-            const int q = (B.j0 + idx / bw) * GNX + B.i0 + idx % bw;
-            af[q] = flux(q);
-        }
-    }
+// The mask of point (j, i) of a plane.
+__device__ __forceinline__ double mbit(const unsigned* b, int j, int i) {
+    return (double)((b[j * kRowWords + (i >> 5)] >> (i & 31)) & 1u);
 }
 
 // Box point idx (row-major, width bw) of box B: array index.
@@ -293,9 +269,11 @@ __device__ __forceinline__ int box_point(const MjBox& B, int bw, float inv_bw, i
 constexpr int kHzThreads = 1024;
 constexpr int kHzPts = (GPLANE + kHzThreads - 1) / kHzThreads;  // box points per thread (disjoint boxes in the plane)
 
-// One (member, tile, level) plane of the horizontal passes, LDS planes given.
+// One (member, tile, level) plane of the horizontal passes, LDS planes given. SNAP: the state before the second, third, ...
+// sweep goes to the planes at snap (the reverse mode's), and the result is written only if a.out is given.
+template <bool SNAP>
 __device__ __forceinline__ void hz_plane(const GadDev& a, int t, int m, int k, double* loc, double* trc,
-                                         unsigned long long* mlw, unsigned long long* mls) {
+                                         unsigned* mlw, unsigned* mls, double* snap) {
     constexpr int NT = kHzThreads;
     const int tid = threadIdx.x;
     const MjTilePlan& tp = a.tiles[t];
@@ -311,38 +289,41 @@ __device__ __forceinline__ void hz_plane(const GadDev& a, int t, int m, int k, d
 
     load_tile_and_bits(tr, unit_bits(a, m, t, k), loc, trc, mlw, mls);
 
+    int ns = 0;
     for (int pass = 0; pass < 3; ++pass) {
         for (int dir = 0; dir < 2; ++dir) {
             const MjSweep& S = tp.sweep[pass][dir];
             if (!S.run) continue;
+            if (SNAP && ns++ > 0) {
+                for (int q = tid; q < GPLANE; q += NT) snap[q] = loc[q];
+                snap += GPLANE;
+            }
             const double* __restrict__ vel = (dir == 0 ? a.u : a.v) + b3;
             const double* __restrict__ hf = (dir == 0 ? a.hFacW : a.hFacS) + b3;
             const double2* __restrict__ gr = a.g2 + dir * (int64_t)a.T * GPLANE + b2;  // {dyG|dxG, recip_dxC|dyC}
-            const unsigned long long* mb = dir == 0 ? mlw : mls;
+            const unsigned* mb = dir == 0 ? mlw : mls;
             const int d = dir == 0 ? 1 : GNX, cmax = dir == 0 ? GNX - 2 : GNY - 2;
             auto trans = [&](double vv, double g, double h) { return vv * (g * deepFacC * drF * h) * rhoFacC; };
             // interface value of face q (gad.py:482-485 transport; 0 outside the Fortran flux loops
             // i = 1-OLx+2 .. sNx+OLx-1, gad_dst3_adv_x.F:80, and j = 1-OLy+2 .. sNy+OLy-1, gad_dst3_adv_y.F:78)
-            auto in_range = [&](int q) {
-                const int j = q / GNX, c = dir == 0 ? q - j * GNX : j;
-                return c >= 2 && c <= cmax;
-            };
             // the interface values of faces q and q + d of a point: the masked differences Rj, Rjp of face q are
             // Rjm, Rj of face q + d, so they are formed once (the same operations as one face at a time)
             auto faces = [&](int q, double V0, double T0, double R0, double V1, double T1, double R1, double& f0,
                              double& f1) {
-                const bool in0 = in_range(q), in1 = in_range(q + d);
+                const int j = q / GNX, i = q - j * GNX, c = dir == 0 ? i : j;
+                const bool in0 = c >= 2 && c <= cmax, in1 = c + 1 >= 2 && c + 1 <= cmax;
+                auto bit = [&](int n) { return dir == 0 ? mbit(mb, j, i + n) : mbit(mb, j + n, i); };
                 f0 = 0.0;
                 f1 = 0.0;
                 if (!in0 && !in1) return;
                 const double t_m1 = loc[q - d], t_0 = loc[q], t_p1 = loc[q + d];
-                const double D0 = (t_0 - t_m1) * mbit(mb, q), Dp1 = (t_p1 - t_0) * mbit(mb, q + d);
+                const double D0 = (t_0 - t_m1) * bit(0), Dp1 = (t_p1 - t_0) * bit(1);
                 if (in0) {
-                    const double Dm1 = (t_m1 - loc[q - 2 * d]) * mbit(mb, q - d);
+                    const double Dm1 = (t_m1 - loc[q - 2 * d]) * bit(-1);
                     f0 = dst3_flux_r(T0, fabs(V0 * dt * R0 * rdeepC), oneSixth, t_m1, t_0, Dm1, D0, Dp1);
                 }
                 if (in1) {
-                    const double Dp2 = (loc[q + 2 * d] - t_p1) * mbit(mb, q + 2 * d);
+                    const double Dp2 = (loc[q + 2 * d] - t_p1) * bit(2);
                     f1 = dst3_flux_r(T1, fabs(V1 * dt * R1 * rdeepC), oneSixth, t_0, t_p1, D0, Dp1, Dp2);
                 }
             };
@@ -388,6 +369,7 @@ __device__ __forceinline__ void hz_plane(const GadDev& a, int t, int m, int k, d
             __syncthreads();
         }
     }
+    if (SNAP && !a.out) return;
     double* out = a.out + b3;
     for (int q = tid; q < GPLANE; q += NT) {
         if (a.w)
@@ -399,8 +381,8 @@ __device__ __forceinline__ void hz_plane(const GadDev& a, int t, int m, int k, d
 
 // The plane as a call of its own (the multi-level blocks: inlined into the level loop it spills registers).
 __device__ __noinline__ void hz_plane_call(const GadDev& a, int t, int m, int k, double* loc, double* trc,
-                                           unsigned long long* mlw, unsigned long long* mls) {
-    hz_plane(a, t, m, k, loc, trc, mlw, mls);
+                                           unsigned* mlw, unsigned* mls) {
+    hz_plane<false>(a, t, m, k, loc, trc, mlw, mls, nullptr);
 }
 
 // One workgroup per (member, tile, level block): LEVELS false, one level per block (a.lpb == 1); true, a.lpb
@@ -409,12 +391,12 @@ template <bool LEVELS>
 __global__ void __launch_bounds__(kHzThreads, 4) gad_hz_kernel(GadDev a) {
     __shared__ double loc[GPLANE];
     __shared__ double trc[GPLANE];
-    __shared__ unsigned long long mlw[kMaskWords], mls[kMaskWords];
+    __shared__ unsigned mlw[kMaskWords], mls[kMaskWords];
     int t, m, k0;
     if (!gad_unit(a, t, m, k0)) return;
     if (!LEVELS) {
         if (a.nlev && k0 >= a.nlev[m]) return;
-        hz_plane(a, t, m, k0, loc, trc, mlw, mls);
+        hz_plane<false>(a, t, m, k0, loc, trc, mlw, mls, nullptr);
         return;
     }
     const int kend = min(k0 + a.lpb, a.nlev ? min(a.nlev[m], a.K) : a.K);
@@ -425,7 +407,8 @@ __global__ void __launch_bounds__(kHzThreads, 4) gad_hz_kernel(GadDev a) {
 }
 
 // ------------------------------------------------------------------------------------------------ reverse mode
-constexpr int kAdjChunk = 1024;  // blocks per reverse launch (each uses 7 planes of the workspace)
+constexpr int kAdjChunk = 1024;  // (member, tile, level)s per reverse launch, in whole columns (at least one)
+constexpr int kAdjSnaps = 5;     // snapshots of one: six sweeps, the first from the tracer itself
 // Partial derivatives of one DST3 interface value f = A (t_m1 + d0 Rj + d1 Rjm) + Bm (t_0 - d0 Rj - d1 Rjp)
 // (A = (tr + |tr|)/2, Bm = (tr - |tr|)/2, d0 = (2-c)(1-c)/6, d1 = (1-c^2)/6): w[0..3] = df/dt_m2, df/dt_m1,
 // df/dt_0, df/dt_p1 (independent of the tracer), dtr = df/dtr, dc = df/dcfl. The derivative of |x| at 0 is taken
@@ -455,213 +438,422 @@ __device__ __forceinline__ FluxPartials dst3_partials(double tr_, double cfl, do
     return P;
 }
 
-// Reverse mode of gad_hz_kernel (horizontal DST3 without R flux) for one (member, tile, level): given the
-// cotangent gbar of gTracer, writes the cotangents of the tracer, uFld and vFld planes (every padded point; the
-// grid, hFac and mask inputs are treated as constants). The forward is replayed with a snapshot of the tile
-// before each sweep (work: 7 planes per block, the first holds the running cotangent of localTij); the sweeps
-// are then reversed: the box update (af, tracer and transport terms), the corner fill after the flux, the flux
-// (weights of the four tracer values, transport and CFL terms), the corner fill before it.
-//
-// With lbar (the R flux's reverse mode) the sweeps start from lbar, the cotangent of localTij after the horizontal
-// passes, instead of from gbar, and the tracer cotangent already holds the vertical part (added to, not set).
-__global__ void __launch_bounds__(1024) gad_hz_adjoint_kernel(GadDev a, const double* gbar, double* trb, double* ub,
-                                                              double* vb, double* work, int blk0, const double* lbar) {
-    __shared__ double loc[GPLANE];
-    __shared__ double fb[GPLANE];
-    __shared__ unsigned long long mlw[kMaskWords], mls[kMaskWords];
-    const int tid = threadIdx.x, nthr = blockDim.x;
-    const int blk = blk0 + blockIdx.x;
-    const int k = blk % a.K;
-    const int mt = blk / a.K;
-    const int t = mt % a.T, m = mt / a.T;
-    const int64_t b3 = m * a.ms3 + ((int64_t)t * a.K + k) * GPLANE;
-    double* TB = trb + b3;
-    double* UB = ub + b3;
-    double* VB = vb + b3;
-    if (a.nlev && k >= a.nlev[m]) {  // no dependence: zero cotangents
-        for (int q = tid; q < GPLANE; q += nthr) {
-            TB[q] = 0.0;
-            UB[q] = 0.0;
-            VB[q] = 0.0;
+// The value of the next lane; `last` (uniform) in lane 63.
+__device__ __forceinline__ double next_lane(double v, double last) {
+    const int lo = __builtin_amdgcn_update_dpp(__double2loint(last), __double2loint(v), 0x130, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(__double2hiint(last), __double2hiint(v), 0x130, 0xf, 0xf, false);
+    return __hiloint2double(hi, lo);
+}
+__device__ __forceinline__ double lane_value(double v, int lane) {
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
+                            __builtin_amdgcn_readlane(__double2loint(v), lane));
+}
+// Bit p of b as 0.0 / 1.0.
+__device__ __forceinline__ double bit01(unsigned b, int p) {
+    return __hiloint2double((((int)(b << (31 - p))) >> 31) & 0x3ff00000, 0);
+}
+// Bits i - 1, i, i + 1 of a row of a bit plane (0 before its first).
+__device__ __forceinline__ unsigned three_bits(const unsigned* row, int i) {
+    const int w = max(i - 1, 0) >> 5;
+    const unsigned long long v = ((unsigned long long)row[min(w + 1, kRowWords - 1)] << 32) | row[w];
+    return (unsigned)((i > 0 ? v >> ((i - 1) & 31) : v << 1) & 7u);
+}
+
+
+// The plan of the block's tile is kept in LDS (a byte or half word of global memory is a vector load, and would wait for
+// all loads issued before it). A sweep's entry, read uniformly; index s = 2 pass + dir.
+constexpr int kSweepWords = sizeof(MjSweep) / 4, kPlanWords = sizeof(MjTilePlan) / 4;
+static_assert(sizeof(MjSweep) == 20 && sizeof(MjTilePlan) == 124, "plan words");
+struct HzBox {
+    int i0, i1, j0, j1;
+    __device__ __forceinline__ bool has(int j, int i) const { return (i >= i0) & (i < i1) & (j >= j0) & (j < j1); }
+};
+struct HzSweep {
+    int fill_before, fill_after;
+    HzBox box[2];  // empty where the sweep has fewer
+    __device__ __forceinline__ HzSweep(const MjTilePlan& lp, int s) {
+        const int* w = (const int*)&lp + s * kSweepWords;
+        auto u = [&](int i) { return __builtin_amdgcn_readfirstlane(w[i]); };
+        const int f = u(0), nbox = f >> 24;
+        fill_before = (f >> 8) & 0xff;
+        fill_after = (f >> 16) & 0xff;
+        for (int b = 0; b < 2; ++b) {
+            const int i = u(1 + 2 * b), j = u(2 + 2 * b);
+            box[b] = b < nbox ? HzBox{i & 0xffff, i >> 16, j & 0xffff, j >> 16} : HzBox{0, 0, 0, 0};
         }
+    }
+    // the rows j0 .. j0 + n - 1, the columns i0 .. i0 + n - 1: is one in a box's range?
+    __device__ __forceinline__ bool rows(int j, int n) const {
+        return ((j < box[0].j1) & (j + n > box[0].j0)) | ((j < box[1].j1) & (j + n > box[1].j0));
+    }
+    __device__ __forceinline__ bool cols(int i, int n) const {
+        return ((i < box[0].i1) & (i + n > box[0].i0)) | ((i < box[1].i1) & (i + n > box[1].i0));
+    }
+    __device__ __forceinline__ bool has(int j, int i) const { return box[0].has(j, i) | box[1].has(j, i); }
+};
+// The next sweep from index s on that runs, 6: none.
+__device__ __forceinline__ int next_sweep(const MjTilePlan& lp, int s) {
+    while (s < 6 && !(__builtin_amdgcn_readfirstlane(((const int*)&lp)[s * kSweepWords]) & 0xff)) ++s;
+    return s;
+}
+
+// The value of the lane before; `first` (uniform) in lane 0.
+__device__ __forceinline__ double prev_lane(double v, double first) {
+    const int lo = __builtin_amdgcn_update_dpp(__double2loint(first), __double2loint(v), 0x138, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(__double2hiint(first), __double2hiint(v), 0x138, 0xf, 0xf, false);
+    return __hiloint2double(hi, lo);
+}
+
+// Element i of a plane: base in scalar registers, 32-bit offset.
+template <class T>
+__device__ __forceinline__ T ld(const T* p, int i) {
+    return *(const T*)((const char*)p + (unsigned)(i * (int)sizeof(T)));
+}
+
+// Forms v here: the compiler would move the arithmetic behind all loads that follow, and spill what it reads.
+__device__ __forceinline__ void pin(double& v) { asm volatile("" : "+v"(v)); }
+
+// Unit of a reverse launch: n (member, tile, level)s from u0 on, level fastest, cut into 8 contiguous ranges, one per XCD
+// (gad_unit's reason). i: its number in the launch.
+__device__ __forceinline__ bool adj_unit(const GadDev& a, int u0, int n, int& i, int& t, int& m, int& k) {
+    const int chunk = (n + 7) / 8, pos = blockIdx.x / 8;
+    i = (blockIdx.x % 8) * chunk + pos;
+    if (pos >= chunk || i >= n) return false;
+    k = (u0 + i) % a.K;
+    const int mt = (u0 + i) / a.K;
+    t = mt % a.T;
+    m = mt / a.T;
+    return true;
+}
+
+// The forward sweeps for the reverse mode: snapshots, and localTij at a.out if given.
+__global__ void __launch_bounds__(kHzThreads, 4) gad_hz_snap_kernel(GadDev a, int u0, int n, double* snap) {
+    __shared__ double loc[GPLANE];
+    __shared__ double trc[GPLANE];
+    __shared__ unsigned mlw[kMaskWords], mls[kMaskWords];
+    int i, t, m, k;
+    if (!adj_unit(a, u0, n, i, t, m, k)) return;
+    if (a.nlev && k >= a.nlev[m]) return;
+    hz_plane<true>(a, t, m, k, loc, trc, mlw, mls, snap + (size_t)i * kAdjSnaps * GPLANE);
+}
+
+// Reverse mode of gad_hz_kernel (horizontal DST3 without R flux) for one (member, tile, level): given the cotangent gbar
+// of gTracer, writes the cotangents of the tracer, uFld and vFld planes (every padded point; the grid, hFac and mask inputs
+// are treated as constants). The sweeps are reversed, each from the snapshot of the tile before it: the box update (af,
+// tracer and transport terms), the corner fill after the flux, the flux (weights of the four tracer values, transport and
+// CFL terms), the corner fill before it.
+//
+// With lbar (the R flux's reverse mode) the sweeps start from lbar, the cotangent of localTij after the horizontal passes,
+// instead of from gbar, and the tracer cotangent already holds the vertical part (added to, not set).
+//
+// Thread (seg, col) = (tid / 98, tid % 98) owns the rows 14 seg .. 14 seg + 13 of column col. Every face's partials are evaluated once, by its owner: in X the four points that they go to take them from
+// the lanes beside (DPP shifts; the three faces beside a wave's 64 points are evaluated by lanes 3 r + 0 .. 2 for row r),
+// in Y a thread walks up its column and evaluates the faces of three rows more. The update's cotangents are formed from
+// localTij's cotangent before a barrier, which is then updated in place behind it. LDS: the tile and that cotangent,
+// 154 KB, one workgroup of 11 waves a CU.
+//
+// What a row reads from memory is loaded a row ahead, and no row has a branch: the loads of all rows issued together spill,
+// and a load issued behind a row's stores waits for them too (both count in order). Bound by HBM (15 planes of 77 KB a unit,
+// 59 us of a CU's share for two sweeps) and the rounds of 650 units on 256 CUs; it reaches 85 us a unit.
+//
+// Evaluating all five partials that a point needs, with a second flux plane and no more than a point's loads in flight,
+// took 958 us for one member of 50 levels together with the replay of the forward sweeps (two of three, each with a
+// snapshot); 291 us now, and 152 us for the replay, whose launch with the R flux also makes the localTij that took another
+// 136 us. Ten rows a thread (1024 threads, 128 VGPRs) and twenty (512, 256) measured 540 to 560 us in the form without the
+// loads ahead, as did fourteen; two rows ahead spill (400 us).
+constexpr int kAdjRows = 14, kAdjSegs = GNY / kAdjRows, kAdjThreads = 704;
+static_assert(kAdjSegs * kAdjRows == GNY && kAdjSegs * GNX <= kAdjThreads && 3 * kAdjRows <= 64, "a thread per column and segment, a lane per edge face");
+
+struct AdjLds {
+    double loc[GPLANE], lb[GPLANE];
+    unsigned mlw[kMaskWords], mls[kMaskWords];
+    MjTilePlan plan;
+};
+
+__global__ void __launch_bounds__(kAdjThreads, 3)
+    gad_hz_adjoint_kernel(GadDev a, const double* gbar, double* trb, double* ub, double* vb, const double* snap, int u0,
+                          int n, const double* lbar) {
+    constexpr int R = kAdjRows;
+    __shared__ AdjLds S;
+    int unit, t, m, k;
+    if (!adj_unit(a, u0, n, unit, t, m, k)) return;
+    int tid = threadIdx.x;
+    const int64_t b3 = m * a.ms3 + ((int64_t)t * a.K + k) * GPLANE;
+    const bool own = tid < kAdjSegs * GNX;
+    const int seg = own ? tid / GNX : 0;
+    int col = own ? tid - seg * GNX : 0, j0 = seg * R;
+    int q0 = j0 * GNX + col;
+    double *const TB = trb + b3, *const UB = ub + b3, *const VB = vb + b3;
+    if (a.nlev && k >= a.nlev[m]) {  // no dependence: zero cotangents
+        for (int r = 0; own && r < R; ++r) TB[q0 + r * GNX] = UB[q0 + r * GNX] = VB[q0 + r * GNX] = 0.0;
         return;
     }
-    const MjTilePlan& tp = a.tiles[t];
     const int64_t b2 = (int64_t)t * GPLANE;
-    const double* tr = a.tr + b3;
-    const double* u = a.u + b3;
-    const double* v = a.v + b3;
-    const double* hW = a.hFacW + b3;
-    const double* hS = a.hFacS + b3;
-    const double* rhC = a.recip_hFacC + b3;
-    const double *dyG = a.dyG + b2, *dxG = a.dxG + b2, *rdxC = a.recip_dxC + b2, *rdyC = a.recip_dyC + b2;
-    const double *rrA = a.recip_rA + b2, *mInC = a.maskInC + b2;
-    const double dt = a.dTlev[k];
-    const double deepFacC = a.deepFacC[k], rdeepC = a.recip_deepFacC[k], rdeep2C = a.recip_deepFac2C[k];
-    const double rhoFacC = a.rhoFacC[k], rrhoFacC = a.recip_rhoFacC[k], drF = a.drF[k], rdrF = a.recip_drF[k];
-    const double oneSixth = a.oneSixth;
-    double* Lb = work + (size_t)blockIdx.x * 7 * GPLANE;
-    double* snap = Lb + GPLANE;
+    const double *const tr = a.tr + b3, *const rhC = a.recip_hFacC + b3;
+    const double2* const am = a.g2 + 2 * (int64_t)a.T * GPLANE + b2;  // {recip_rA, maskInC}
+    // the level's factors in scalar registers
+    auto level = [&](const double* p) {
+        const double v = p[k];
+        return __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(v)),
+                                __builtin_amdgcn_readfirstlane(__double2loint(v)));
+    };
+    const double dt = level(a.dTlev), deepFacC = level(a.deepFacC), rdeepC = level(a.recip_deepFacC);
+    const double rdeep2C = level(a.recip_deepFac2C), rhoFacC = level(a.rhoFacC), rrhoFacC = level(a.recip_rhoFacC);
+    const double drF = level(a.drF), rdrF = level(a.recip_drF), oneSixth = a.oneSixth;
+    snap += (size_t)unit * kAdjSnaps * GPLANE;
+    auto update_coef = [&](double RH, double2 AM) { return dt * rrhoFacC * RH * rdrF * AM.x * rdeep2C * AM.y; };
 
-    auto uTrans = [&](int q) { return u[q] * (dyG[q] * deepFacC * drF * hW[q]) * rhoFacC; };
-    auto vTrans = [&](int q) { return v[q] * (dxG[q] * deepFacC * drF * hS[q]) * rhoFacC; };
-    auto coef = [&](int q) { return dt * rrhoFacC * rhC[q] * rdrF * rrA[q] * rdeep2C; };
-    auto in_box = [&](const MjSweep& S, int q) {
-        const int j = q / GNX, i = q - j * GNX;
-        for (int bx = 0; bx < S.nbox; ++bx)
-            if (i >= S.box[bx].i0 && i < S.box[bx].i1 && j >= S.box[bx].j0 && j < S.box[bx].j1) return true;
-        return false;
+    // element q + r GNX of a plane: 32-bit offsets and an immediate (which ends at 4095 bytes)
+    auto at8 = [&](const double* p, int q, int r) {
+        const int c = r < 7 ? 3 : 10;
+        return ((const double*)((const char*)p + (unsigned)(q + c * GNX) * 8))[(r - c) * GNX];
     };
-    // flux partials at q in direction dir from the tile state in loc; false outside the flux domain
-    auto partials = [&](int dir, int q, FluxPartials& P) {
-        const int j = q / GNX, i = q - j * GNX;
-        if (dir == 0) {
-            if (i < 2 || i > GNX - 2) return false;
-            const double cfl = fabs(u[q] * dt * rdxC[q] * rdeepC);
-            P = dst3_partials(uTrans(q), cfl, oneSixth, loc[q - 2], loc[q - 1], loc[q], loc[q + 1], mbit(mlw, q - 1),
-                              mbit(mlw, q), mbit(mlw, q + 1));
-        } else {
-            if (j < 2 || j > GNY - 2) return false;
-            const double cfl = fabs(v[q] * dt * rdyC[q] * rdeepC);
-            P = dst3_partials(vTrans(q), cfl, oneSixth, loc[q - 2 * GNX], loc[q - GNX], loc[q], loc[q + GNX],
-                              mbit(mls, q - GNX), mbit(mls, q), mbit(mls, q + GNX));
-        }
-        return true;
+    auto at16 = [&](const double2* p, int q, int r) {
+        const int c = r / 5 * 5 + 2;
+        return ((const double2*)((const char*)p + (unsigned)(q + c * GNX) * 16))[(r - c) * GNX];
     };
-    auto flux = [&](int dir, int q) {
-        const int j = q / GNX, i = q - j * GNX;
-        if (dir == 0) {
-            if (i < 2 || i > GNX - 2) return 0.0;
-            const double cfl = fabs(u[q] * dt * rdxC[q] * rdeepC);
-            return dst3_flux(uTrans(q), cfl, oneSixth, loc[q - 2], loc[q - 1], loc[q], loc[q + 1], mbit(mlw, q - 1),
-                             mbit(mlw, q), mbit(mlw, q + 1));
-        }
-        if (j < 2 || j > GNY - 2) return 0.0;
-        const double cfl = fabs(v[q] * dt * rdyC[q] * rdeepC);
-        return dst3_flux(vTrans(q), cfl, oneSixth, loc[q - 2 * GNX], loc[q - GNX], loc[q], loc[q + GNX],
-                         mbit(mls, q - GNX), mbit(mls, q), mbit(mls, q + GNX));
-    };
-
-    // ---- forward replay, snapshot before each sweep
-    int order[6], ns = 0;
-    for (int q = tid; q < GPLANE; q += nthr) loc[q] = tr[q];
     {
-        const unsigned long long* gb = unit_bits(a, m, t, k);
-        for (int wd = tid; wd < 2 * kMaskWords; wd += nthr) {
-            if (wd < kMaskWords)
-                mlw[wd] = gb[wd];
-            else
-                mls[wd - kMaskWords] = gb[wd];
+        double x[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r) x[r] = at8(lbar ? lbar + b3 : gbar + b3, q0, r);
+        if (!lbar) {
+#pragma unroll
+            for (int r = 0; r < R; ++r) x[r] = x[r] / dt;
         }
+        if (own) {
+#pragma unroll
+            for (int r = 0; r < R; ++r) S.lb[q0 + r * GNX] = x[r];
+            if (!lbar) {
+#pragma unroll
+                for (int r = 0; r < R; ++r) TB[q0 + r * GNX] = -x[r];
+            }
+        }
+        const unsigned* gb = unit_bits(a, m, t, k);
+        static_assert(kMaskWords <= kAdjThreads, "a word of each plane per thread");
+        if (tid < kMaskWords) {
+            S.mlw[tid] = gb[tid];
+            S.mls[tid] = gb[kMaskWords + tid];
+        }
+        if (tid < kPlanWords) ((int*)&S.plan)[tid] = ((const int*)&a.tiles[t])[tid];
     }
     __syncthreads();
-    for (int pass = 0; pass < 3; ++pass) {
-        for (int dir = 0; dir < 2; ++dir) {
-            const MjSweep& S = tp.sweep[pass][dir];
-            if (!S.run) continue;
-            double* sn = snap + (size_t)ns * GPLANE;
-            for (int q = tid; q < GPLANE; q += nthr) sn[q] = loc[q];
-            order[ns++] = pass * 2 + dir;
-            if (S.fill_before) corner_fill(loc, a, tp, S.fill_before, tid);
-            if (S.nbox) {
-                flux_boxes(S, dir, fb, [&](int q) { return flux(dir, q); });
-                __syncthreads();
-            }
-            if (S.fill_after) corner_fill(loc, a, tp, S.fill_after, tid);
-            for (int bx = 0; bx < S.nbox; ++bx) {
-                const MjBox Bx = S.box[bx];
-                const int bw = Bx.i1 - Bx.i0, n = bw * (Bx.j1 - Bx.j0);
-                for (int idx = tid; idx < n; idx += nthr) {
-                    const int q = (Bx.j0 + idx / bw) * GNX + Bx.i0 + idx % bw;
-                    double daf, dtr;
-                    if (dir == 0) {
-                        daf = fb[q + 1] - fb[q];
-                        dtr = uTrans(q + 1) - uTrans(q);
-                    } else {
-                        daf = fb[q + GNX] - fb[q];
-                        dtr = vTrans(q + GNX) - vTrans(q);
+    // masks of the Y faces of the thread's column: rows j0 - 2 .. j0 + R + 2, from bit 0 on
+    unsigned my = 0;
+#pragma unroll
+    for (int r = -2; r < R + 3; ++r)
+        my |= (S.mls[max(min(j0 + r, GNY - 1), 0) * kRowWords + (col >> 5)] >> (col & 31) & 1u) << (r + 2);
+    int left = 0;  // sweeps to reverse
+    for (int s = 0; s < 6; ++s) left += next_sweep(S.plan, s) == s;
+    bool first[2] = {true, true};  // no cotangent of this velocity written yet
+    for (int s = 5; s >= 0; --s) {
+        if (next_sweep(S.plan, s) != s) continue;
+        --left;
+        // positions made anew for each sweep: the compiler would keep every address derived from them in registers
+        asm volatile("" : "+v"(tid), "+v"(q0), "+v"(col), "+v"(j0), "+v"(my));
+        const int dir = s & 1, lane = tid & 63;
+        const HzSweep P(S.plan, s);
+        const double* const sn = left ? snap + (size_t)(left - 1) * GPLANE : tr;
+        const double* const vel = (dir == 0 ? a.u : a.v) + b3;
+        const double* const hf = (dir == 0 ? a.hFacW : a.hFacS) + b3;
+        const double2* const gr = a.g2 + dir * (int64_t)a.T * GPLANE + b2;  // {dyG|dxG, recip_dxC|dyC}
+        double* const vbar = dir == 0 ? UB : VB;
+        const bool init = dir == 0 ? first[0] : first[1];
+        if (dir == 0) first[0] = false; else first[1] = false;
+        // box update: loc[q] -= c_q (af[q+d] - af[q] - tr[q] (T[q+d] - T[q])), c_q = coef(q) maskInC(q); cg: the cotangent
+        // c_q lb[q] of the increment, 0 off the boxes
+        auto update_bar = [&](bool in, double c, double lb) {
+            double x = c * lb;
+            pin(x);  // else the loads move behind a branch, one after the other
+            return in ? x : 0.0;
+        };
+        // a face whose interface value has the cotangent g: c[0..3] to the tracer values q - 2d .. q + d, vv to the velocity
+        // (its transport T = V L rhoFacC); bits from bit p on: the masks of the faces before, at and behind it
+        auto face = [&](bool in, double g, double V, double L, double T, double rd, double tm2, double tm1, double t0,
+                        double tp1, unsigned bits, int p, double (&c)[4], double& vv) {
+            const double arg = V * dt * rd * rdeepC;
+            const FluxPartials F = dst3_partials(T, fabs(arg), oneSixth, tm2, tm1, t0, tp1, bit01(bits, p),
+                                                 bit01(bits, p + 1), bit01(bits, p + 2));
+            const bool act = in && g != 0.0;
+            const double sgn = arg > 0.0 ? 1.0 : (arg < 0.0 ? -1.0 : 0.0);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) c[i] = act ? F.w[i] * g : 0.0;
+            vv = act ? (F.dtr * g) * (L * rhoFacC) + (F.dc * g) * (sgn * dt * rd * rdeepC) : 0.0;
+        };
+        // the velocity's cotangent at row r: the transport's tb, then the flux part; o: what is there from a sweep before
+        auto put_vel = [&](int r, double tb, double L, double vv, double o) {
+            const double x = tb != 0.0 ? tb * (L * rhoFacC) : 0.0, b = init ? 0.0 : o;
+            vbar[q0 + r * GNX] = (b + x) + vv;
+        };
+        const double* const old = init ? vel : vbar;  // not looked at when there is nothing yet
+        // ---- before the barrier: the tile, the update's cotangents of the thread's rows (in Y of two more on each side)
+        // and in X of the points beside the wave
+        // strips: most wavefronts (X) or lanes (Y, whose columns have nothing to do with each other) have no point of them
+        const bool act = dir == 0 ? __any(P.rows(j0, R)) : P.cols(col, 1);
+        auto beside = [&](int r) { return max(min(j0 + r, GNY - 1), 0) * GNX + col; };  // rows beside the thread's own
+        auto at = [&](const double* p, int r) { return r >= 0 && r < R ? at8(p, q0, r) : ld(p, beside(r)); };
+        auto at2 = [&](const double2* p, int r) { return r >= 0 && r < R ? at16(p, q0, r) : ld(p, beside(r)); };
+        auto lds = [&](int r) { return r >= 0 && r < R ? q0 + r * GNX : beside(r); };
+        // X: lane 3 r + f has row r of the point before the wave's first (f = 0), of the two behind its last (1, 2)
+        const int er = lane / 3, ef = lane - er * 3, te = ef == 0 ? (tid & ~63) - 1 : (tid | 63) + ef;
+        const bool edge = er < R && te >= 0 && te < kAdjSegs * GNX;
+        const int eseg = edge ? te / GNX : 0, ei = edge ? te - eseg * GNX : 0, ej = edge ? eseg * R + er : 0;
+        const int eq = ej * GNX + ei, em = max(eq - 1, 0);
+        double cg[R + 4], ecg = 0.0, ecm = 0.0;
+        unsigned inb = 0;  // bit r + 2: row r is in a box
+        {
+            double sv[R];
+#pragma unroll
+            for (int r = 0; r < R; ++r) sv[r] = at8(sn, q0, r);
+            if (act) {
+                double RH[R];
+                double2 A[R];
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    RH[r] = at8(rhC, q0, r);
+                    A[r] = at16(am, q0, r);
+                }
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    const bool inp = P.has(j0 + r, col);
+                    inb |= (unsigned)inp << (r + 2);
+                    cg[r + 2] = update_bar(inp, update_coef(RH[r], A[r]), S.lb[q0 + r * GNX]);
+                    pin(cg[r + 2]);
+                }
+                if (dir == 0) {
+                    ecg = update_bar(edge & P.has(ej, ei), update_coef(ld(rhC, eq), ld(am, eq)), S.lb[eq]);
+                    ecm = update_bar(edge & (ei > 0) & P.has(ej, ei - 1), update_coef(ld(rhC, em), ld(am, em)), S.lb[em]);
+                } else {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const int r = i < 2 ? i - 2 : R + i - 2;
+                        const bool inp = (j0 + r >= 0) & P.has(j0 + r, col);
+                        inb |= (unsigned)inp << (r + 2);
+                        cg[r + 2] = update_bar(inp, update_coef(at(rhC, r), at2(am, r)), S.lb[lds(r)]);
                     }
-                    loc[q] = loc[q] - coef(q) * (daf - tr[q] * dtr) * mInC[q];
                 }
             }
-            __syncthreads();
+            if (own) {
+#pragma unroll
+                for (int r = 0; r < R; ++r) S.loc[q0 + r * GNX] = sv[r];
+            }
         }
-    }
-
-    // ---- cotangent of the output (localTij - tracer) / dt, or of localTij itself (lbar)
-    for (int q = tid; q < GPLANE; q += nthr) {
-        if (lbar) {
-            Lb[q] = lbar[b3 + q];
+        __syncthreads();  // the tile is loaded; every read of the cotangent precedes its updates
+        if (P.fill_before) corner_fill(S.loc, a, S.plan, P.fill_before, tid);
+        if (P.fill_after) corner_fill_T(S.lb, a, S.plan, P.fill_after, tid);
+        // ---- the faces; what a row reads is loaded kAhead rows before it
+        constexpr int kAhead = 1;
+        struct RowIn {
+            double V, H, TR, old, tb;
+            double2 G;
+        } in[kAhead + 1];
+        if (dir == 0 && act) {
+            double ec[4], eT, ect;
+            {
+                const double* const l = S.loc + max(min(eq, GPLANE - 2), 2);
+                const double2 G = ld(gr, eq);
+                const double V = ld(vel, eq), L = G.x * deepFacC * drF * ld(hf, eq);
+                double vv;
+                eT = V * L * rhoFacC;
+                ect = ecg * ld(tr, eq);
+                pin(ect);
+                ect = edge & P.has(ej, ei) ? ect : 0.0;
+                face(edge && ei >= 2 && ei <= GNX - 2, ecg - ecm, V, L, eT, G.y, l[-2], l[-1], l[0], l[1],
+                     three_bits(S.mlw + ej * kRowWords, ei), 0, ec, vv);
+            }
+            auto load = [&](int r) {
+                if (r < R) in[r % (kAhead + 1)] = RowIn{at8(vel, q0, r), at8(hf, q0, r), at8(tr, q0, r),
+                                                           at8(old, q0, r), at8(TB, q0, r), at16(gr, q0, r)};
+            };
+#pragma unroll
+            for (int r = 0; r < kAhead; ++r) load(r);
+            const bool inx = col >= 2 && col <= GNX - 2;  // columns 0, 1 and 97 have no flux: they read beside them
+            const double* const l0 = S.loc + j0 * GNX + max(min(col, GNX - 2), 2);
+            if (own) {
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    __builtin_amdgcn_sched_barrier(0);
+                    load(r + kAhead);
+                    const int q = q0 + r * GNX;
+                    const RowIn I = in[r % (kAhead + 1)];
+                    const double L = I.G.x * deepFacC * drF * I.H, T = I.V * L * rhoFacC, g = cg[r + 2];
+                    const bool inp = inb >> (r + 2) & 1;
+                    const double ct = inp ? g * I.TR : 0.0;
+                    const double cm = prev_lane(g, lane_value(ecg, 3 * r)), cmt = prev_lane(ct, lane_value(ect, 3 * r));
+                    const double* const l = l0 + r * GNX;
+                    double c[4], vv;
+                    face(inx, g - cm, I.V, L, T, I.G.y, l[-2], l[-1], l[0], l[1],
+                         three_bits(S.mlw + (j0 + r) * kRowWords, col), 0, c, vv);
+                    // to this point from the faces q + 2, q + 1, q, q - 1
+                    const double c0 =
+                        next_lane(next_lane(c[0], lane_value(ec[0], 3 * r + 1)), lane_value(ec[0], 3 * r + 2));
+                    const double c1 = next_lane(c[1], lane_value(ec[1], 3 * r + 1));
+                    const double c3 = prev_lane(c[3], lane_value(ec[3], 3 * r));
+                    const double T1 = next_lane(T, lane_value(eT, 3 * r + 1));
+                    S.lb[q] = S.lb[q] + (((c0 + c1) + c[2]) + c3);
+                    TB[q] = inp ? I.tb + g * (T1 - T) : I.tb;
+                    put_vel(r, (0.0 - ct) + cmt, L, vv, I.old);
+                }
+            }
+        } else if (dir != 0 && act) {
+            // up the column: face r gives to the rows r - 2 .. r + 1; a0: row r + 1, complete with it, a1, a2: r, r - 1;
+            // ct: of row r
+            auto load = [&](int r) {
+                if (r >= -1)
+                    in[(r + 1) % (kAhead + 1)] = RowIn{at(vel, r), at(hf, r), r >= 0 && r <= R ? at(tr, r - 1) : 0.0,
+                                                       r >= 0 && r < R ? at8(old, q0, r) : 0.0,
+                                                       r >= 0 && r < R ? at8(TB, q0, r) : 0.0, at2(gr, r)};
+            };
+#pragma unroll
+            for (int r = R + 1; r > R + 1 - kAhead; --r) load(r);
+            if (own) {
+                double a0 = 0.0, a1 = 0.0, a2 = 0.0, T1 = 0.0, ct = 0.0;
+                double t0 = S.loc[lds(R + 1)], tp1 = S.loc[lds(R + 2)], tm1 = S.loc[lds(R)];
+#pragma unroll
+                for (int r = R + 1; r >= -1; --r) {
+                    __builtin_amdgcn_sched_barrier(0);
+                    load(r - kAhead);
+                    const RowIn I = in[(r + 1) % (kAhead + 1)];
+                    const int j = j0 + r;
+                    const double L = I.G.x * deepFacC * drF * I.H, T = I.V * L * rhoFacC;
+                    const double tm2 = S.loc[lds(r - 2)];
+                    double c[4], vv;
+                    face(j >= 2 && j <= GNY - 2, cg[r + 2] - cg[r + 1], I.V, L, T, I.G.y, tm2, tm1, t0, tp1, my, r + 1, c, vv);
+                    if (r >= -1 && r + 1 < R) {
+                        const int ql = q0 + (r + 1) * GNX;
+                        S.lb[ql] = S.lb[ql] + (a0 + c[3]);
+                    }
+                    if (r >= 0 && r <= R) {
+                        const double cmt = inb >> (r + 1) & 1 ? cg[r + 1] * I.TR : 0.0;
+                        if (r < R) {
+                            TB[q0 + r * GNX] = inb >> (r + 2) & 1 ? I.tb + cg[r + 2] * (T1 - T) : I.tb;
+                            put_vel(r, (0.0 - ct) + cmt, L, vv, I.old);
+                        }
+                        ct = cmt;
+                    }
+                    a0 = a1 + c[2];
+                    a1 = a2 + c[1];
+                    a2 = c[0];
+                    T1 = T;
+                    tp1 = t0, t0 = tm1, tm1 = tm2;
+                }
+            }
         } else {
-            const double g = gbar[b3 + q];
-            Lb[q] = g / dt;
-            TB[q] = -(g / dt);
+            if (init && own) {
+#pragma unroll
+                for (int r = 0; r < R; ++r) vbar[q0 + r * GNX] = 0.0;
+            }
         }
-        UB[q] = 0.0;
-        VB[q] = 0.0;
+        __syncthreads();
+        if (P.fill_before) corner_fill_T(S.lb, a, S.plan, P.fill_before, tid);
     }
-    __syncthreads();
-
-    // ---- sweeps in reverse
-    for (int s = ns - 1; s >= 0; --s) {
-        const int pass = order[s] >> 1, dir = order[s] & 1;
-        const MjSweep& S = tp.sweep[pass][dir];
-        const int d = dir == 0 ? 1 : GNX;
-        double* VBd = dir == 0 ? UB : VB;
-        const double* vel = dir == 0 ? u : v;
-        const double* rdC = dir == 0 ? rdxC : rdyC;
-        const double* len = dir == 0 ? dyG : dxG;
-        const double* hF = dir == 0 ? hW : hS;
-        const double* sn = snap + (size_t)s * GPLANE;
-        for (int q = tid; q < GPLANE; q += nthr) loc[q] = sn[q];
-        __syncthreads();
-        if (S.fill_before) corner_fill(loc, a, tp, S.fill_before, tid);
-        auto trans = [&](int q) { return dir == 0 ? uTrans(q) : vTrans(q); };
-        // box update: loc[q] -= c_q (af[q+d] - af[q] - tr[q] (T[q+d] - T[q])), c_q = coef(q) maskInC(q)
-        for (int p = tid; p < GPLANE; p += nthr) {
-            double f = 0.0, tb = 0.0;
-            if (S.nbox) {
-                const bool inp = in_box(S, p), inm = p - d >= 0 && in_box(S, p - d);
-                if (inp) {
-                    const double cg = coef(p) * mInC[p] * Lb[p];
-                    f = f + cg;
-                    tb = tb - cg * tr[p];
-                    TB[p] = TB[p] + cg * (trans(p + d) - trans(p));
-                }
-                if (inm) {
-                    const double cg = coef(p - d) * mInC[p - d] * Lb[p - d];
-                    f = f - cg;
-                    tb = tb + cg * tr[p - d];
-                }
-            }
-            fb[p] = f;
-            // transport cotangent -> velocity: T = vel (len deepFacC drF hFac) rhoFacC
-            if (tb != 0.0) VBd[p] = VBd[p] + tb * ((len[p] * deepFacC * drF * hF[p]) * rhoFacC);
-        }
-        __syncthreads();
-        if (S.fill_after) corner_fill_T(Lb, a, tp, S.fill_after, tid);
-        // flux: Lb[p] += sum_k w_k(q) fb[q] over the fluxes q = p + 2d, p + d, p, p - d that read p
-        for (int p = tid; p < GPLANE; p += nthr) {
-            double acc = 0.0;
-            FluxPartials P;
-            for (int kk = 0; kk < 4; ++kk) {
-                const int q = p + (2 - kk) * d;  // loc index p is t_m2 (kk=0) .. t_p1 (kk=3) of flux q
-                if (q < 0 || q >= GPLANE || fb[q] == 0.0) continue;
-                if (partials(dir, q, P)) acc = acc + P.w[kk] * fb[q];
-            }
-            Lb[p] = Lb[p] + acc;
-            if (fb[p] != 0.0 && partials(dir, p, P)) {
-                const double g = fb[p];
-                const double dT = (len[p] * deepFacC * drF * hF[p]) * rhoFacC;
-                const double arg = vel[p] * dt * rdC[p] * rdeepC;
-                const double sgn = arg > 0.0 ? 1.0 : (arg < 0.0 ? -1.0 : 0.0);
-                VBd[p] = VBd[p] + (P.dtr * g) * dT + (P.dc * g) * (sgn * dt * rdC[p] * rdeepC);
-            }
-        }
-        __syncthreads();
-        if (S.fill_before) corner_fill_T(Lb, a, tp, S.fill_before, tid);
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        if (!own) continue;
+        const int q = q0 + r * GNX;
+        TB[q] = TB[q] + S.lb[q];
+        if (first[0]) UB[q] = 0.0;
+        if (first[1]) VB[q] = 0.0;
     }
-    for (int q = tid; q < GPLANE; q += nthr) TB[q] = TB[q] + Lb[q];
 }
 
 // Vertical DST3 (R) sweep after the horizontal passes, per column (member, tile, j, i), k = 0..nlev-1 downward.
@@ -739,12 +931,18 @@ __global__ void __launch_bounds__(256) gad_vert_kernel(GadDev a, const double* _
 // cotangent e(k-1) - e(k) and rTrans(k) e(k) tracer(k) - e(k-1) tracer(k-1); the interface value's partials
 // (dst3_partials: the four tracer weights, d/dtransport, d/dcfl) carry them on to loc_h and to w through
 // rTrans = w rA mk and cfl = |w dt recip_drC| (d|x|/dx = sign x, 0 at 0).
-__global__ void __launch_bounds__(256) gad_vert_adjoint_kernel(GadDev a, const double* __restrict__ loc_h,
+//
+// One walk down the column: step k takes level k in, evaluates interface k - 1 (which reads the levels k - 3 .. k) and
+// writes what is complete, so each of the six arrays is read once and each of the three written once; the level data are
+// loaded kVertAhead steps ahead. Bound by HBM: reading them as needed, with locbar updated in memory, took 240 us for one
+// member of 50 levels; 82 us now (450 MB, 5.5 TB/s).
+constexpr int kVertAhead = 4;
+__global__ void __launch_bounds__(256) gad_vert_adjoint_kernel(GadDev a, int col0, const double* __restrict__ loc_h,
                                                                const double* __restrict__ gbar,
                                                                double* __restrict__ locbar, double* __restrict__ trb,
                                                                double* __restrict__ wb) {
     const int q = blockIdx.x * blockDim.x + threadIdx.x;
-    const int mt = blockIdx.y;
+    const int mt = col0 + blockIdx.y;
     if (q >= GPLANE) return;
     const int t = mt % a.T, m = mt / a.T;
     const int K = a.K;
@@ -762,40 +960,64 @@ __global__ void __launch_bounds__(256) gad_vert_adjoint_kernel(GadDev a, const d
     double* __restrict__ tb = trb + c3;
     double* __restrict__ wbar = wb + c3;
     auto L = [](int k) { return (int64_t)k * GPLANE; };
-    auto Tk = [&](int k) { return (k >= 0 && k < kmax) ? lh[L(k)] : 0.0; };
-    auto Mk = [&](int k) { return (k >= 0 && k < kmax) ? mc[L(k)] : 0.0; };
-    auto mk = [&](int k) { return (k >= 1 && k <= kmax - 1) ? Mk(k - 1) * Mk(k) : 0.0; };
-    auto rT = [&](int k) { return (k >= 1 && k <= kmax - 1) ? w[L(k)] * rA * mk(k) : 0.0; };
-    auto e = [&](int k) {
-        if (k < 0 || k >= kmax) return 0.0;
-        const double cf = a.dTlev[k] * a.recip_rhoFacC[k] * rhC[L(k)] * a.recip_drF[k] * rrA * a.recip_deepFac2C[k];
-        return cf * Mk(k) * (gb[L(k)] / a.dTlev[k]);
+    double rw[kVertAhead], rtr[kVertAhead], rrh[kVertAhead], rlh[kVertAhead], rgb[kVertAhead], rmc[kVertAhead];
+    auto load = [&](int s, int k) {
+        const int64_t o = L(max(min(k, kmax - 1), 0));
+        rw[s] = w[o];
+        rtr[s] = tr[o];
+        rrh[s] = rhC[o];
+        rlh[s] = lh[o];
+        rgb[s] = gb[o];
+        rmc[s] = mc[o];
     };
-    for (int k = 0; k < K; ++k) {
-        double l = 0.0, tv = 0.0;
-        if (k < kmax) {
-            const double g = gb[L(k)];
-            l = g / a.dTlev[k];
-            tv = -(g / a.dTlev[k]) + e(k) * (rT(k) - rT(k + 1));
+#pragma unroll
+    for (int s = 0; s < kVertAhead; ++s) load(s, s);
+    // levels k - 1, k - 2, k - 3 (1, 2, 3)
+    double T1 = 0.0, T2 = 0.0, T3 = 0.0, M1 = 0.0, mk1 = 0.0, mk2 = 0.0, e1 = 0.0, e2 = 0.0, w1 = 0.0,
+           tr1 = 0.0, tr2 = 0.0, rT1 = 0.0, tv1 = 0.0, l1 = 0.0, l2 = 0.0, l3 = 0.0;
+    auto step = [&](int k, int s) {
+        const bool wet = k < kmax;
+        const double T0 = wet ? rlh[s] : 0.0, M0 = wet ? rmc[s] : 0.0, w0 = rw[s], tr0 = rtr[s], g = rgb[s], rh = rrh[s];
+        load(s, k + kVertAhead);
+        const bool inner = k >= 1 && wet;
+        const double mk0 = inner ? M1 * M0 : 0.0, rT0 = inner ? w0 * rA * mk0 : 0.0;
+        double e0 = 0.0, l0 = 0.0, tv0 = 0.0;
+        if (wet) {
+            const double cf = a.dTlev[k] * a.recip_rhoFacC[k] * rh * a.recip_drF[k] * rrA * a.recip_deepFac2C[k];
+            l0 = g / a.dTlev[k];
+            e0 = cf * M0 * l0;
+            tv0 = -l0;
         }
-        lb[L(k)] = l;
-        tb[L(k)] = tv;
-        wbar[L(k)] = 0.0;
+        if (k >= 1 && k - 1 < kmax) tb[L(k - 1)] = tv1 + e1 * (rT1 - rT0);
+        const int ki = k - 1;
+        if (ki >= 1 && ki <= kmax - 1) {
+            const double wTb = e2 - e1;
+            const double arg = w1 * a.dTlev[ki] * a.recip_drC[ki];
+            const FluxPartials P = dst3_partials(rT1, fabs(arg), a.oneSixth, T0, T1, T2, T3, mk0, mk1, mk2);
+            if (wet) l0 = l0 + P.w[0] * wTb;
+            l1 = l1 + P.w[1] * wTb;
+            l2 = l2 + P.w[2] * wTb;
+            l3 = l3 + P.w[3] * wTb;
+            const double rTb = e1 * tr1 - e2 * tr2 + P.dtr * wTb;
+            const double sgn = arg > 0.0 ? 1.0 : (arg < 0.0 ? -1.0 : 0.0);
+            wbar[L(ki)] = rTb * (rA * mk1) + (P.dc * wTb) * (sgn * a.dTlev[ki] * a.recip_drC[ki]);
+        } else if (ki == 0) {
+            wbar[0] = 0.0;
+        }
+        if (k >= 3 && k - 3 < kmax) lb[L(k - 3)] = l3;
+        T3 = T2, T2 = T1, T1 = T0;
+        M1 = M0, mk2 = mk1, mk1 = mk0;
+        e2 = e1, e1 = e0;
+        w1 = w0, tr2 = tr1, tr1 = tr0, rT1 = rT0, tv1 = tv0;
+        l3 = l2, l2 = l1, l1 = l0;
+    };
+    // steps 0 .. kmax + 2, the last three to complete the column
+    for (int k0 = 0; k0 < kmax + 3; k0 += kVertAhead) {
+#pragma unroll
+        for (int s = 0; s < kVertAhead; ++s)
+            if (k0 + s < kmax + 3) step(k0 + s, s);
     }
-    for (int ki = 1; ki <= kmax - 1; ++ki) {
-        const double wk = w[L(ki)];
-        const double wTb = e(ki - 1) - e(ki);
-        const double arg = wk * a.dTlev[ki] * a.recip_drC[ki];
-        const FluxPartials P = dst3_partials(rT(ki), fabs(arg), a.oneSixth, Tk(ki + 1), Tk(ki), Tk(ki - 1),
-                                             Tk(ki - 2), mk(ki + 1), mk(ki), mk(ki - 1));
-        if (ki + 1 < kmax) lb[L(ki + 1)] = lb[L(ki + 1)] + P.w[0] * wTb;
-        lb[L(ki)] = lb[L(ki)] + P.w[1] * wTb;
-        lb[L(ki - 1)] = lb[L(ki - 1)] + P.w[2] * wTb;
-        if (ki - 2 >= 0) lb[L(ki - 2)] = lb[L(ki - 2)] + P.w[3] * wTb;
-        const double rTb = e(ki) * tr[L(ki)] - e(ki - 1) * tr[L(ki - 1)] + P.dtr * wTb;
-        const double sgn = arg > 0.0 ? 1.0 : (arg < 0.0 ? -1.0 : 0.0);
-        wbar[L(ki)] = rTb * (rA * mk(ki)) + (P.dc * wTb) * (sgn * a.dTlev[ki] * a.recip_drC[ki]);
-    }
+    for (int k = kmax; k < K; ++k) lb[L(k)] = tb[L(k)] = wbar[L(k)] = 0.0;
 }
 
 }  // namespace mj
@@ -1006,7 +1228,7 @@ int mask_slots_of(const mj_gad_config* c) {
 }
 // The bit planes of every (mask slot, tile, level), then the packed 2-D metrics.
 size_t mask_bits_bytes(const mj_gad_config* c, int ntiles) {
-    return (size_t)mask_slots_of(c) * ntiles * c->nr * 2 * kMaskWords * sizeof(unsigned long long);
+    return (size_t)mask_slots_of(c) * ntiles * c->nr * 2 * kMaskWords * sizeof(unsigned);
 }
 size_t pre_bytes(const mj_gad_config* c, int ntiles) {
     return al256(mask_bits_bytes(c, ntiles)) + al256((size_t)3 * ntiles * GPLANE * sizeof(double2));
@@ -1016,19 +1238,25 @@ size_t batch3_bytes(const mj_gad_config* c, int ntiles) {
     return (size_t)c->batch * (size_t)std::max<int64_t>(c->member_stride3d, (int64_t)ntiles * c->nr * GPLANE) *
            sizeof(double);
 }
-// The reverse mode's part of its workspace (before the bit planes).
+// (member, tile)s of one reverse launch.
+int adjoint_columns(const mj_gad_config* c, int ntiles) {
+    return (int)std::min<int64_t>((int64_t)c->batch * ntiles, std::max(1, kAdjChunk / c->nr));
+}
+// The reverse mode's part of its workspace (before the bit planes): the snapshots, and with the R flux localTij and its
+// cotangent.
+size_t adjoint_snap_bytes(const mj_gad_config* c, int ntiles) {
+    return al256((size_t)adjoint_columns(c, ntiles) * c->nr * kAdjSnaps * GPLANE * sizeof(double));
+}
 size_t adjoint_scratch_bytes(const mj_gad_config* c, int ntiles, int with_w) {
-    size_t n = (size_t)kAdjChunk * 7 * GPLANE * sizeof(double);  // the replay scratch of the horizontal reverse
-    if (with_w) n += 2 * batch3_bytes(c, ntiles);
-    return al256(n);
+    return adjoint_snap_bytes(c, ntiles) + (with_w ? 2 * al256(batch3_bytes(c, ntiles)) : 0);
 }
 // The per-call tables at `pre` (pre_bytes): the bit planes of maskLocW / maskLocS for every (mask slot, tile,
 // level) and the packed 2-D metrics; sets a.mbits and a.g2.
 int launch_pre(GadDev& a, const mj_gad_config* c, void* pre, hipStream_t st) {
     const int nslots = mask_slots_of(c);
-    a.mbits = (unsigned long long*)pre;
+    a.mbits = (unsigned*)pre;
     a.g2 = (double2*)((char*)pre + al256(mask_bits_bytes(c, a.T)));
-    hipLaunchKernelGGL(gad_maskbits_kernel, dim3((unsigned)(nslots * a.T * a.K)), dim3(256), 0, st, a, nslots);
+    hipLaunchKernelGGL(gad_maskbits_kernel, dim3((unsigned)(2 * nslots * a.T * a.K)), dim3(kBitsThreads), 0, st, a, nslots);
     MJ_HIP(hipGetLastError());
     hipLaunchKernelGGL(gad_pack2d_kernel, dim3((unsigned)((a.T * GPLANE + 255) / 256)), dim3(256), 0, st, a);
     MJ_HIP(hipGetLastError());
@@ -1174,30 +1402,29 @@ extern "C" int mj_gad_dst3_adjoint(const mj_gad_plan* P, const mj_gad_grid* g, c
     MJ_REQUIRE(work_bytes >= need, "mj_gad_dst3_adjoint: work %zu < %zu bytes", work_bytes, need);
     MJ_REQUIRE(((uintptr_t)work & 255) == 0, "mj_gad_dst3_adjoint: work must be 256-byte aligned");
     hipStream_t st = as_stream(stream);
-    const int nblk = c->batch * P->ntiles * c->nr;
     GadDev a = gad_dev(P, g, c, uFld, vFld, nullptr, tracer, hFacW, hFacS, recip_hFacC);
     if ((rc = launch_pre(a, c, (char*)work + adjoint_scratch_bytes(c, P->ntiles, wFld != nullptr), st))) return rc;
+    GadDev f = a;  // the forward replay, with the R flux localTij after the horizontal passes
+    f.w = wFld;
+    f.out = nullptr;
     double* lbar = nullptr;
     if (wFld) {
-        // forward replay of the horizontal passes (localTij), then the vertical reverse per column
-        double* loc_h = work + (size_t)kAdjChunk * 7 * GPLANE;
-        lbar = loc_h + batch3_bytes(c, P->ntiles) / sizeof(double);
-        GadDev f = gad_dev(P, g, c, uFld, vFld, wFld, tracer, hFacW, hFacS, recip_hFacC);
-        f.mbits = a.mbits;
-        f.g2 = a.g2;
-        f.out = loc_h;
-        f.lpb = 1;
-        const unsigned nb8 = (unsigned)((nblk + 7) / 8 * 8);
-        hipLaunchKernelGGL(gad_hz_kernel<false>, dim3(nb8), dim3(kHzThreads), 0, st, f);
-        MJ_HIP(hipGetLastError());
-        hipLaunchKernelGGL(gad_vert_adjoint_kernel, dim3((GPLANE + 255) / 256, (unsigned)(c->batch * P->ntiles)),
-                           dim3(256), 0, st, f, (const double*)loc_h, gTracer_bar, lbar, tracer_bar, wFld_bar);
-        MJ_HIP(hipGetLastError());
+        f.out = (double*)((char*)work + adjoint_snap_bytes(c, P->ntiles));
+        lbar = (double*)((char*)f.out + al256(batch3_bytes(c, P->ntiles)));
     }
-    for (int b0 = 0; b0 < nblk; b0 += kAdjChunk) {
-        const int n = std::min(kAdjChunk, nblk - b0);
-        hipLaunchKernelGGL(gad_hz_adjoint_kernel, dim3((unsigned)n), dim3(1024), 0, st, a, gTracer_bar, tracer_bar,
-                           uFld_bar, vFld_bar, work, b0, (const double*)lbar);
+    const int ncol = c->batch * P->ntiles, step = adjoint_columns(c, P->ntiles);
+    for (int c0 = 0; c0 < ncol; c0 += step) {
+        const int nc = std::min(step, ncol - c0), n = nc * c->nr;
+        const unsigned nblk = (unsigned)((n + 7) / 8 * 8);
+        hipLaunchKernelGGL(gad_hz_snap_kernel, dim3(nblk), dim3(kHzThreads), 0, st, f, c0 * c->nr, n, work);
+        MJ_HIP(hipGetLastError());
+        if (wFld) {
+            hipLaunchKernelGGL(gad_vert_adjoint_kernel, dim3((GPLANE + 255) / 256, (unsigned)nc), dim3(256), 0, st, f, c0,
+                               (const double*)f.out, gTracer_bar, lbar, tracer_bar, wFld_bar);
+            MJ_HIP(hipGetLastError());
+        }
+        hipLaunchKernelGGL(gad_hz_adjoint_kernel, dim3(nblk), dim3(kAdjThreads), 0, st, a, gTracer_bar, tracer_bar,
+                           uFld_bar, vFld_bar, (const double*)work, c0 * c->nr, n, (const double*)lbar);
         MJ_HIP(hipGetLastError());
     }
     return MJ_OK;

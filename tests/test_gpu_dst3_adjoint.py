@@ -199,3 +199,37 @@ def test_r_flux_gradients_vs_finite_differences(dev):
                 print(f"R {name} {pt} h={hh:.1e}: ad {gg[pt]:.10e} fd {fd:.10e} rel {r:.2e}", flush=True)
                 best = min(best, r)
             assert best < 1e-6, (name, pt, best)
+
+
+@pytest.mark.parametrize("K,nlev,vertical", [(50, [50, 31, 4], True), (50, [50, 31, 4], False), (7, [7, 7, 1], True),
+                                             (1, None, False)])
+def test_reverse_launches_of_whole_columns(dev, K, nlev, vertical):
+    """The reverse mode runs in launches of at most 1024 (member, tile, level)s, in whole columns: three members of 50
+    levels take two, of 7 levels one. Every member's cotangents are the bits that it gets alone, in which the X and Y
+    strips, their corner fills and the wavefronts' edges are those of the 13 tiles; levels beyond a member's count are 0."""
+    import torch
+    from mit_jax_amd import gad, synthetic as S
+    g, u, v, w, tr = dst3_case(0)
+    g2, vg = S.gad_inputs(g)
+    cut = lambda a: np.ascontiguousarray(a[:, :K]) if np.ndim(a) == 4 else a  # noqa: E731
+    g2d = {k: to_dev(cut(np.asarray(a)), dev) for k, a in g2.items()}
+    vk = {k: np.asarray(a)[:K] for k, a in vg.items()}
+    params = gad.GADParams.llc90(Nr=K, implicitAdvection=not vertical)
+    rng = np.random.default_rng(17)
+    B = 3
+    three = lambda a, s: torch.stack([to_dev(cut(a) * f, dev) for f in s])  # noqa: E731
+    U, V, W = three(u, (1.0, -0.7, 0.4)), three(v, (1.0, 0.6, -0.9)), three(w, (1.0, -0.5, 0.8))
+    TR = torch.stack([to_dev(cut(tr) + 0.1 * m * rng.normal(size=cut(tr).shape), dev) for m in range(B)])
+    H = [three(a, (1.0, 1.0, 1.0)) for a in (g.hFacW, g.hFacS, g.recip_hFacC)]
+    bar = to_dev(rng.normal(size=tuple(TR.shape)), dev)
+    print(f"reverse launches: {K} levels, {nlev}, vertical {vertical}", flush=True)
+    got = gad.advect_tiles_adjoint(params, None, g2d, vk, U, V, TR, *H, bar, nlev=nlev, wFld=W if vertical else None)
+    assert len(got) == (4 if vertical else 3)
+    for m in range(B):
+        one = [a[m:m + 1].contiguous() for a in (U, V, TR, *H, bar)]
+        ref = gad.advect_tiles_adjoint(params, None, g2d, vk, *one, nlev=None if nlev is None else nlev[m:m + 1],
+                                       wFld=W[m:m + 1].contiguous() if vertical else None)
+        for a, b in zip(got, ref):
+            assert torch.equal(a[m], b[0]) and bool(a[m].isfinite().all())
+            if nlev is not None:
+                assert bool((a[m][:, nlev[m]:] == 0).all())
