@@ -221,188 +221,364 @@ __global__ void __launch_bounds__(256) gad_pack2d_kernel(GadDev a) {
     a.g2[2 * n + q] = make_double2(a.recip_rA[q], a.maskInC[q]);
 }
 
-// The tracer plane into LDS (into loc and loc2) and the unit's mask bit planes, all loads in flight together (one
-// memory latency for a 1024-thread block).
-__device__ __forceinline__ void load_tile_and_bits(const double* tr, const unsigned* gb, double* loc,
-                                                   double* loc2, unsigned* bw, unsigned* bs) {
-    const int tid = threadIdx.x, nthr = blockDim.x;
-    constexpr int KP = (GPLANE + 1023) / 1024;  // per thread at 1024
-    for (int it = 0; it * KP * nthr < GPLANE || it * nthr < 2 * kMaskWords; ++it) {
-        double v[KP];
-#pragma unroll
-        for (int b = 0; b < KP; ++b) {
-            const int q = (it * KP + b) * nthr + tid;
-            v[b] = q < GPLANE ? tr[q] : 0.0;
-        }
-        const int wd = it * nthr + tid;
-        const unsigned word = wd < 2 * kMaskWords ? gb[wd] : 0u;
-#pragma unroll
-        for (int b = 0; b < KP; ++b) {
-            const int q = (it * KP + b) * nthr + tid;
-            if (q < GPLANE) loc[q] = loc2[q] = v[b];
-        }
-        if (wd < kMaskWords)
-            bw[wd] = word;
-        else if (wd < 2 * kMaskWords)
-            bs[wd - kMaskWords] = word;
-    }
-    __syncthreads();
-}
-
-// The mask of point (j, i) of a plane.
-__device__ __forceinline__ double mbit(const unsigned* b, int j, int i) {
-    return (double)((b[j * kRowWords + (i >> 5)] >> (i & 31)) & 1u);
-}
-
 // Box point idx (row-major, width bw) of box B: array index.
-__device__ __forceinline__ int box_point(const MjBox& B, int bw, float inv_bw, int idx) {
+template <class Box>
+__device__ __forceinline__ int box_point(const Box& B, int bw, float inv_bw, int idx) {
     const int r = (int)(((float)idx + 0.5f) * inv_bw);  // idx / bw, exact for idx < 2^14 and bw <= 128
     return (B.j0 + r) * GNX + B.i0 + (idx - r * bw);
 }
 
-// One workgroup of 1024 threads per (member, tile, level). Every box point of a sweep evaluates the interface
-// values of both its faces (q and q + d) itself, with no flux plane: from the same loads and in the same order of
-// operations, so the two points beside a face get the same bits, and the update is the same IEEE expression as
-// with one shared evaluation. The point keeps its increment in a register until every thread has read the tracer
-// plane, and only then updates it. LDS: the working plane, the input tracer (read by every update and by the
-// output) and the mask bits, 156 KB.
-constexpr int kHzThreads = 1024;
-constexpr int kHzPts = (GPLANE + kHzThreads - 1) / kHzThreads;  // box points per thread (disjoint boxes in the plane)
+// The value of the next lane; `last` (uniform) in lane 63.
+__device__ __forceinline__ double next_lane(double v, double last) {
+    const int lo = __builtin_amdgcn_update_dpp(__double2loint(last), __double2loint(v), 0x130, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(__double2hiint(last), __double2hiint(v), 0x130, 0xf, 0xf, false);
+    return __hiloint2double(hi, lo);
+}
+__device__ __forceinline__ double lane_value(double v, int lane) {
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
+                            __builtin_amdgcn_readlane(__double2loint(v), lane));
+}
+// Bit p of b as 0.0 / 1.0.
+__device__ __forceinline__ double bit01(unsigned b, int p) {
+    return __hiloint2double((((int)(b << (31 - p))) >> 31) & 0x3ff00000, 0);
+}
+// Bits i - 1, i, i + 1 of a row of a bit plane (0 before its first).
+__device__ __forceinline__ unsigned three_bits(const unsigned* row, int i) {
+    const int w = max(i - 1, 0) >> 5;
+    const unsigned long long v = ((unsigned long long)row[min(w + 1, kRowWords - 1)] << 32) | row[w];
+    return (unsigned)((i > 0 ? v >> ((i - 1) & 31) : v << 1) & 7u);
+}
 
-// One (member, tile, level) plane of the horizontal passes, LDS planes given. SNAP: the state before the second, third, ...
-// sweep goes to the planes at snap (the reverse mode's), and the result is written only if a.out is given.
+
+// The plan of the block's tile is kept in LDS (a byte or half word of global memory is a vector load, and would wait for
+// all loads issued before it). A sweep's entry, read uniformly; index s = 2 pass + dir.
+constexpr int kSweepWords = sizeof(MjSweep) / 4, kPlanWords = sizeof(MjTilePlan) / 4;
+static_assert(sizeof(MjSweep) == 20 && sizeof(MjTilePlan) == 124, "plan words");
+struct HzBox {
+    int i0, i1, j0, j1;
+    __device__ __forceinline__ int points() const { return (i1 - i0) * (j1 - j0); }
+    __device__ __forceinline__ bool has(int j, int i) const { return (i >= i0) & (i < i1) & (j >= j0) & (j < j1); }
+};
+struct HzSweep {
+    int fill_before, fill_after;
+    HzBox box[2];  // empty where the sweep has fewer
+    __device__ __forceinline__ HzSweep(const MjTilePlan& lp, int s) {
+        const int* w = (const int*)&lp + s * kSweepWords;
+        auto u = [&](int i) { return __builtin_amdgcn_readfirstlane(w[i]); };
+        const int f = u(0), nbox = f >> 24;
+        fill_before = (f >> 8) & 0xff;
+        fill_after = (f >> 16) & 0xff;
+        for (int b = 0; b < 2; ++b) {
+            const int i = u(1 + 2 * b), j = u(2 + 2 * b);
+            box[b] = b < nbox ? HzBox{i & 0xffff, i >> 16, j & 0xffff, j >> 16} : HzBox{0, 0, 0, 0};
+        }
+    }
+    __device__ __forceinline__ int points() const { return box[0].points() + box[1].points(); }
+    // the rows j0 .. j0 + n - 1, the columns i0 .. i0 + n - 1: is one in a box's range?
+    __device__ __forceinline__ bool rows(int j, int n) const {
+        return ((j < box[0].j1) & (j + n > box[0].j0)) | ((j < box[1].j1) & (j + n > box[1].j0));
+    }
+    __device__ __forceinline__ bool cols(int i, int n) const {
+        return ((i < box[0].i1) & (i + n > box[0].i0)) | ((i < box[1].i1) & (i + n > box[1].i0));
+    }
+    __device__ __forceinline__ bool has(int j, int i) const { return box[0].has(j, i) | box[1].has(j, i); }
+};
+// The next sweep from index s on that runs, 6: none.
+__device__ __forceinline__ int next_sweep(const MjTilePlan& lp, int s) {
+    while (s < 6 && !(__builtin_amdgcn_readfirstlane(((const int*)&lp)[s * kSweepWords]) & 0xff)) ++s;
+    return s;
+}
+
+// The value of the lane before; `first` (uniform) in lane 0.
+__device__ __forceinline__ double prev_lane(double v, double first) {
+    const int lo = __builtin_amdgcn_update_dpp(__double2loint(first), __double2loint(v), 0x138, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(__double2hiint(first), __double2hiint(v), 0x138, 0xf, 0xf, false);
+    return __hiloint2double(hi, lo);
+}
+
+// Element i of a plane: base in scalar registers, 32-bit offset.
+template <class T>
+__device__ __forceinline__ T ld(const T* p, int i) {
+    return *(const T*)((const char*)p + (unsigned)(i * (int)sizeof(T)));
+}
+
+// Forms v here: the compiler would move the arithmetic behind all loads that follow, and spill what it reads.
+__device__ __forceinline__ void pin(double& v) { asm volatile("" : "+v"(v)); }
+
+// Element q + r GNX, r = 0 .. 13, of a plane: 32-bit offsets and an immediate (which ends at 4095 bytes).
+__device__ __forceinline__ double plane8(const double* p, int q, int r) {
+    const int c = r < 7 ? 3 : 10;
+    return ((const double*)((const char*)p + (unsigned)(q + c * GNX) * 8))[(r - c) * GNX];
+}
+__device__ __forceinline__ double2 plane16(const double2* p, int q, int r) {
+    const int c = r / 5 * 5 + 2;
+    return ((const double2*)((const char*)p + (unsigned)(q + c * GNX) * 16))[(r - c) * GNX];
+}
+// A level's factor, in scalar registers.
+__device__ __forceinline__ double level_value(const double* p, int k) {
+    const double v = p[k];
+    return __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(v)),
+                            __builtin_amdgcn_readfirstlane(__double2loint(v)));
+}
+
+// One workgroup of 704 threads per (member, tile, level). Thread (seg, col) = (tid / 98, tid % 98) owns the rows 14 seg ..
+// 14 seg + 13 of column col through all sweeps: the coefficient of its points' updates is formed once and stays in
+// registers. A face's transport and interface value are evaluated once, by the owner of the point behind it: in X a point
+// takes those of its other face from the lane of the next column (a DPP shift; the faces beside a wave's last lane are
+// evaluated by its lanes 0 .. 13, a row each), in Y a thread walks down its rows and evaluates one face more, the first of
+// the segment below. The values are those of one evaluation per face in a flux plane, in the same order of operations. A
+// point keeps its increment in a register until every thread has read the tracer plane, and only then updates it. What a
+// row reads from memory is loaded kHzAhead rows before it. LDS: the working plane, the input tracer (read by every update
+// and by the output) and the mask bits, 156 KB.
+//
+// Sweeps with at most 1024 points (the overlap strips of passes 1 and 2) run one point a thread over the boxes, both faces
+// evaluated by the point: on the columns 94 of 98 lanes would be idle there.
+//
+// Bound by HBM: a unit moves seven planes (540 KB, 28 us of a CU's share) and takes 37 us, of which some 4 are phases
+// without loads; one member of 50 levels is 650 units on 256 CUs. Evaluating both faces at each of ten points a thread, all
+// loads of a point behind one another, took 136 us for it (122 now) and 1700 us for 24 members of mixed level counts (1615
+// now). One row ahead instead of two measured 3 % more for both, four 8 % more for the members.
+constexpr int kHzRows = 14, kHzSegs = GNY / kHzRows, kHzThreads = 704, kHzSmall = 1024;
+constexpr int kHzAhead = 2;
+static_assert(kHzSegs * kHzRows == GNY && kHzSegs * GNX <= kHzThreads, "a thread per column and segment");
+
+struct HzLds {
+    double loc[GPLANE], trc[GPLANE];
+    unsigned mlw[kMaskWords], mls[kMaskWords];
+    MjTilePlan plan;
+};
+
+// One (member, tile, level) plane of the horizontal passes. SNAP: the state before the second, third, ... sweep goes to the
+// planes at snap (the reverse mode's), and the result is written only if a.out is given.
 template <bool SNAP>
-__device__ __forceinline__ void hz_plane(const GadDev& a, int t, int m, int k, double* loc, double* trc,
-                                         unsigned* mlw, unsigned* mls, double* snap) {
-    constexpr int NT = kHzThreads;
-    const int tid = threadIdx.x;
-    const MjTilePlan& tp = a.tiles[t];
+__device__ __forceinline__ void hz_plane(const GadDev& a, int t, int m, int k, HzLds& S, double* snap) {
+    constexpr int R = kHzRows, N = kHzAhead + 1;
+    double *const loc = S.loc, *const trc = S.trc;
+    int tid = threadIdx.x;
     const int64_t b3 = m * a.ms3 + ((int64_t)t * a.K + k) * GPLANE;
     const int64_t b2 = (int64_t)t * GPLANE;
-    const double* __restrict__ tr = a.tr + b3;
-    const double* __restrict__ rhC = a.recip_hFacC + b3;
-    const double2* __restrict__ am = a.g2 + 2 * (int64_t)a.T * GPLANE + b2;  // {recip_rA, maskInC}
-    const double dt = a.dTlev[k];
-    const double deepFacC = a.deepFacC[k], rdeepC = a.recip_deepFacC[k], rdeep2C = a.recip_deepFac2C[k];
-    const double rhoFacC = a.rhoFacC[k], rrhoFacC = a.recip_rhoFacC[k], drF = a.drF[k], rdrF = a.recip_drF[k];
+    const double* const rhC = a.recip_hFacC + b3;
+    const double2* const am = a.g2 + 2 * (int64_t)a.T * GPLANE + b2;  // {recip_rA, maskInC}
+    const double dt = level_value(a.dTlev, k), deepFacC = level_value(a.deepFacC, k), rdeepC = level_value(a.recip_deepFacC, k);
+    const double rdeep2C = level_value(a.recip_deepFac2C, k), rhoFacC = level_value(a.rhoFacC, k);
+    const double rrhoFacC = level_value(a.recip_rhoFacC, k), drF = level_value(a.drF, k), rdrF = level_value(a.recip_drF, k);
     const double oneSixth = a.oneSixth;
-
-    load_tile_and_bits(tr, unit_bits(a, m, t, k), loc, trc, mlw, mls);
-
-    int ns = 0;
-    for (int pass = 0; pass < 3; ++pass) {
-        for (int dir = 0; dir < 2; ++dir) {
-            const MjSweep& S = tp.sweep[pass][dir];
-            if (!S.run) continue;
-            if (SNAP && ns++ > 0) {
-                for (int q = tid; q < GPLANE; q += NT) snap[q] = loc[q];
-                snap += GPLANE;
-            }
-            const double* __restrict__ vel = (dir == 0 ? a.u : a.v) + b3;
-            const double* __restrict__ hf = (dir == 0 ? a.hFacW : a.hFacS) + b3;
-            const double2* __restrict__ gr = a.g2 + dir * (int64_t)a.T * GPLANE + b2;  // {dyG|dxG, recip_dxC|dyC}
-            const unsigned* mb = dir == 0 ? mlw : mls;
-            const int d = dir == 0 ? 1 : GNX, cmax = dir == 0 ? GNX - 2 : GNY - 2;
-            auto trans = [&](double vv, double g, double h) { return vv * (g * deepFacC * drF * h) * rhoFacC; };
-            // interface value of face q (gad.py:482-485 transport; 0 outside the Fortran flux loops
-            // i = 1-OLx+2 .. sNx+OLx-1, gad_dst3_adv_x.F:80, and j = 1-OLy+2 .. sNy+OLy-1, gad_dst3_adv_y.F:78)
-            // the interface values of faces q and q + d of a point: the masked differences Rj, Rjp of face q are
-            // Rjm, Rj of face q + d, so they are formed once (the same operations as one face at a time)
-            auto faces = [&](int q, double V0, double T0, double R0, double V1, double T1, double R1, double& f0,
-                             double& f1) {
-                const int j = q / GNX, i = q - j * GNX, c = dir == 0 ? i : j;
-                const bool in0 = c >= 2 && c <= cmax, in1 = c + 1 >= 2 && c + 1 <= cmax;
-                auto bit = [&](int n) { return dir == 0 ? mbit(mb, j, i + n) : mbit(mb, j + n, i); };
-                f0 = 0.0;
-                f1 = 0.0;
-                if (!in0 && !in1) return;
-                const double t_m1 = loc[q - d], t_0 = loc[q], t_p1 = loc[q + d];
-                const double D0 = (t_0 - t_m1) * bit(0), Dp1 = (t_p1 - t_0) * bit(1);
-                if (in0) {
-                    const double Dm1 = (t_m1 - loc[q - 2 * d]) * bit(-1);
-                    f0 = dst3_flux_r(T0, fabs(V0 * dt * R0 * rdeepC), oneSixth, t_m1, t_0, Dm1, D0, Dp1);
-                }
-                if (in1) {
-                    const double Dp2 = (loc[q + 2 * d] - t_p1) * bit(2);
-                    f1 = dst3_flux_r(T1, fabs(V1 * dt * R1 * rdeepC), oneSixth, t_0, t_p1, D0, Dp1, Dp2);
-                }
-            };
-            if (S.fill_before) corner_fill(loc, a, tp, S.fill_before, tid);
-            // the boxes' points as one index range (the boxes are disjoint, so at most GPLANE points)
-            const MjBox B0 = S.box[0], B1 = S.box[1];
-            const int bw0 = B0.i1 - B0.i0, n0 = S.nbox > 0 ? bw0 * (B0.j1 - B0.j0) : 0;
-            const int bw1 = B1.i1 - B1.i0, n1 = S.nbox > 1 ? bw1 * (B1.j1 - B1.j0) : 0;
-            const float inv0 = 1.0f / (float)max(bw0, 1), inv1 = 1.0f / (float)max(bw1, 1);
-            auto point = [&](int idx) {
-                return idx < n0 ? box_point(B0, bw0, inv0, idx) : box_point(B1, bw1, inv1, idx - n0);
-            };
-            double inc[kHzPts];
+    const bool own = tid < kHzSegs * GNX;
+    const int seg = own ? tid / GNX : 0;
+    int col = own ? tid - seg * GNX : 0, j0 = seg * R, q0 = j0 * GNX + col;
+    auto at8 = [&](const double* p, int r) { return plane8(p, q0, r); };
+    auto at16 = [&](const double2* p, int r) { return plane16(p, q0, r); };
+    // X: lane r has row r of the point behind the wave's last lane
+    int qe;
+    {
+        const int lane = tid & 63, te = (tid | 63) + 1, sege = te / GNX;
+        const bool edge = lane < R && te < kHzSegs * GNX;
+        qe = edge ? (sege * R + lane) * GNX + te - sege * GNX : q0;
+    }
+    auto trans = [&](double V, double G, double H) { return V * (G * deepFacC * drF * H) * rhoFacC; };
+    // interface value (gad.py:482-485 transport; 0 outside the Fortran flux loops i = 1-OLx+2 .. sNx+OLx-1,
+    // gad_dst3_adv_x.F:80, and j = 1-OLy+2 .. sNy+OLy-1, gad_dst3_adv_y.F:78); bits from bit p on: the masks of the faces
+    // before, at and behind it
+    auto flux = [&](bool in, double T, double V, double rd, double t_m2, double t_m1, double t_0, double t_p1,
+                    unsigned bits, int p) {
+        const double Dm1 = (t_m1 - t_m2) * bit01(bits, p), D0 = (t_0 - t_m1) * bit01(bits, p + 1),
+                     Dp1 = (t_p1 - t_0) * bit01(bits, p + 2);
+        const double f = dst3_flux_r(T, fabs(V * dt * rd * rdeepC), oneSixth, t_m1, t_0, Dm1, D0, Dp1);
+        return in ? f : 0.0;
+    };
+    double coef[R];
+    {
+        const double* const tr = a.tr + b3;
+        double tv[R], rh[R], ra[R];
+        const int pw = tid < kPlanWords ? ((const int*)&a.tiles[t])[tid] : 0;
+        static_assert(kMaskWords <= kHzThreads, "a word of each plane per thread");
+        const unsigned* gb = unit_bits(a, m, t, k);
+        const unsigned w0 = tid < kMaskWords ? gb[tid] : 0, w1 = tid < kMaskWords ? gb[kMaskWords + tid] : 0;
 #pragma unroll
-            for (int r = 0; r < kHzPts; ++r) {
-                const int idx = tid + r * NT;
-                inc[r] = 0.0;
-                if (idx < n0 + n1) {
-                    const int qq = point(idx), qd = qq + d;
-                    const double2 GR0 = gr[qq], GR1 = gr[qd], AM = am[qq];
-                    const double V0 = vel[qq], G0 = GR0.x, H0 = hf[qq], R0 = GR0.y;
-                    const double V1 = vel[qd], G1 = GR1.x, H1 = hf[qd], R1 = GR1.y;
-                    const double TR = trc[qq], RH = rhC[qq], RA = AM.x, MI = AM.y;
-                    const double T0 = trans(V0, G0, H0), T1 = trans(V1, G1, H1);
-                    double f0, f1;
-                    faces(qq, V0, T0, R0, V1, T1, R1, f0, f1);
-                    // local - coef*(d(af) - tracer*d(trans))*maskInC (gad.py:511-514), coefficient gad.py:494
+        for (int r = 0; r < R; ++r) {
+            tv[r] = at8(tr, r);
+            rh[r] = at8(rhC, r);
+            ra[r] = at16(am, r).x;
+        }
+        if (tid < kPlanWords) ((int*)&S.plan)[tid] = pw;
+        if (tid < kMaskWords) S.mlw[tid] = w0, S.mls[tid] = w1;
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            coef[r] = dt * rrhoFacC * rh[r] * rdrF * ra[r] * rdeep2C;  // gad.py:494
+            pin(coef[r]);
+        }
+        if (own) {
+#pragma unroll
+            for (int r = 0; r < R; ++r) loc[q0 + r * GNX] = trc[q0 + r * GNX] = tv[r];
+        }
+    }
+    __syncthreads();
+    // masks of the thread's Y faces: rows j0 - 1 .. j0 + R + 1
+    unsigned my = 0;
+#pragma unroll
+    for (int r = 0; r < R + 3; ++r)
+        my |= (S.mls[max(min(j0 - 1 + r, GNY - 1), 0) * kRowWords + (col >> 5)] >> (col & 31) & 1u) << r;
+    int ns = 0;
+    for (int s = next_sweep(S.plan, 0); s < 6;) {
+        // positions and masks made anew for each sweep: the compiler would keep all that is derived from them in registers
+        asm volatile("" : "+v"(tid), "+v"(q0), "+v"(col), "+v"(j0), "+v"(qe), "+v"(my));
+        const int dir = s & 1;
+        const HzSweep P(S.plan, s);
+        const int npt = P.points();
+        const double* const vel = (dir == 0 ? a.u : a.v) + b3;
+        const double* const hf = (dir == 0 ? a.hFacW : a.hFacS) + b3;
+        const double2* const gr = a.g2 + dir * (int64_t)a.T * GPLANE + b2;  // {dyG|dxG, recip_dxC|dyC}
+        struct RowIn {
+            double V, H, MI;
+            double2 G;
+        } in[N];
+        if (P.fill_before) corner_fill(loc, a, S.plan, P.fill_before, tid);
+        // local - coef*(d(af) - tracer*d(trans))*maskInC (gad.py:511-514)
+        if (npt <= kHzSmall) {
+            const int d = dir == 0 ? 1 : GNX;
+            constexpr int C = (kHzSmall + kHzThreads - 1) / kHzThreads;
+            double inc[C];
+            int qq[C];
+#pragma unroll
+            for (int n = 0; n < C; ++n) {
+                const int idx = tid + n * kHzThreads;
+                if (idx >= npt) continue;
+                const int n0 = P.box[0].points(), bw0 = P.box[0].i1 - P.box[0].i0, bw1 = P.box[1].i1 - P.box[1].i0;
+                const int q = idx < n0 ? box_point(P.box[0], bw0, 1.0f / (float)max(bw0, 1), idx)
+                                       : box_point(P.box[1], bw1, 1.0f / (float)max(bw1, 1), idx - n0);
+                qq[n] = q;
+                const double2 G0 = ld(gr, q), G1 = ld(gr, q + d), A = ld(am, q);
+                const double V0 = ld(vel, q), H0 = ld(hf, q), V1 = ld(vel, q + d), H1 = ld(hf, q + d), RH = ld(rhC, q);
+                const unsigned* mb = dir == 0 ? S.mlw : S.mls;
+                const int j = q / GNX, i = q - j * GNX, c = dir == 0 ? i : j, cmax = (dir == 0 ? GNX : GNY) - 2;
+                const double T0 = trans(V0, G0.x, H0), T1 = trans(V1, G1.x, H1);
+                auto at = [&](int o) { return loc[max(min(q + o * d, GPLANE - 1), 0)]; };
+                auto bit = [&](int o) {
+                    const int jb = min(max(j + (dir == 0 ? 0 : o), 0), GNY - 1), ib = min(max(i + (dir == 0 ? o : 0), 0), GNX - 1);
+                    return (mb[jb * kRowWords + (ib >> 5)] >> (ib & 31)) & 1u;
+                };
+                const unsigned bits = bit(-1) | bit(0) << 1 | bit(1) << 2 | bit(2) << 3;
+                const double f0 = flux(c >= 2 && c <= cmax, T0, V0, G0.y, at(-2), at(-1), at(0), at(1), bits, 0);
+                const double f1 = flux(c + 1 >= 2 && c + 1 <= cmax, T1, V1, G1.y, at(-1), at(0), at(1), at(2), bits, 1);
+                const double daf = f1 - f0, dtr = T1 - T0, cf = dt * rrhoFacC * RH * rdrF * A.x * rdeep2C;
+                inc[n] = cf * (daf - trc[q] * dtr) * A.y;
+            }
+            __syncthreads();  // every read of the plane precedes the updates
+            if (P.fill_after) corner_fill(loc, a, S.plan, P.fill_after, tid);
+#pragma unroll
+            for (int n = 0; n < C; ++n)
+                if (tid + n * kHzThreads < npt) loc[qq[n]] = loc[qq[n]] - inc[n];
+        } else {
+            double inc[R];
+            if (dir == 0) {
+                auto load = [&](int r) {
+                    if (r < R) in[r % N] = RowIn{at8(vel, r), at8(hf, r), at16(am, r).y, at16(gr, r)};
+                };
+                const double Ve = ld(vel, qe), He = ld(hf, qe);
+                const double2 Ge = ld(gr, qe);
+#pragma unroll
+                for (int r = 0; r < kHzAhead; ++r) load(r);
+                const int je = qe / GNX, ie = qe - je * GNX;  // columns 0, 1 and 97 have no flux: their lanes read beside them
+                const double* const le = loc + max(min(qe, GPLANE - 2), 2);
+                const double Te = trans(Ve, Ge.x, He);
+                const double fe = flux(ie >= 2 && ie <= GNX - 2, Te, Ve, Ge.y, le[-2], le[-1], le[0], le[1],
+                                       three_bits(S.mlw + je * kRowWords, ie), 0);
+                const bool inx = col >= 2 && col <= GNX - 2;
+                const double* const l0 = loc + j0 * GNX + max(min(col, GNX - 2), 2);
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    __builtin_amdgcn_sched_barrier(0);
+                    load(r + kHzAhead);
+                    const RowIn I = in[r % N];
+                    const double* const l = l0 + r * GNX;
+                    const double T0 = trans(I.V, I.G.x, I.H);
+                    const double f0 = flux(inx, T0, I.V, I.G.y, l[-2], l[-1], l[0], l[1],
+                                           three_bits(S.mlw + (j0 + r) * kRowWords, col), 0);
+                    const double f1 = next_lane(f0, lane_value(fe, r)), T1 = next_lane(T0, lane_value(Te, r));
                     const double daf = f1 - f0, dtr = T1 - T0;
-                    const double coef = dt * rrhoFacC * RH * rdrF * RA * rdeep2C;
-                    inc[r] = coef * (daf - TR * dtr) * MI;
+                    inc[r] = coef[r] * (daf - trc[q0 + r * GNX] * dtr) * I.MI;
+                    pin(inc[r]);
+                }
+            } else {
+                // rows beside the thread's own
+                auto beside = [&](int r) { return max(min(j0 + r, GNY - 1), 0) * GNX + col; };
+                auto lds = [&](int r) { return r >= 0 && r < R ? loc[q0 + r * GNX] : loc[beside(r)]; };
+                auto load = [&](int r) {
+                    if (r < R)
+                        in[r % N] = RowIn{at8(vel, r), at8(hf, r), at16(am, r).y, at16(gr, r)};
+                    else if (r == R)
+                        in[r % N] = RowIn{ld(vel, beside(r)), ld(hf, beside(r)), 0.0, ld(gr, beside(r))};
+                };
+#pragma unroll
+                for (int r = 0; r < kHzAhead; ++r) load(r);
+                double tm2 = lds(-2), tm1 = lds(-1), t0 = lds(0), T0 = 0.0, f0 = 0.0, MI = 0.0;
+#pragma unroll
+                for (int r = 0; r <= R; ++r) {
+                    __builtin_amdgcn_sched_barrier(0);
+                    load(r + kHzAhead);
+                    const RowIn I = in[r % N];
+                    const double tp1 = lds(r + 1);
+                    const double T1 = trans(I.V, I.G.x, I.H);
+                    const double f1 = flux(j0 + r >= 2 && j0 + r <= GNY - 2, T1, I.V, I.G.y, tm2, tm1, t0, tp1, my, r);
+                    if (r > 0) {
+                        const double daf = f1 - f0, dtr = T1 - T0;
+                        inc[r - 1] = coef[r - 1] * (daf - trc[q0 + (r - 1) * GNX] * dtr) * MI;
+                        pin(inc[r - 1]);
+                    }
+                    tm2 = tm1, tm1 = t0, t0 = tp1, T0 = T1, f0 = f1, MI = I.MI;
                 }
             }
             __syncthreads();  // every read of the plane precedes the updates
-            if (S.fill_after) corner_fill(loc, a, tp, S.fill_after, tid);
+            if (P.fill_after) corner_fill(loc, a, S.plan, P.fill_after, tid);
+            if (own) {
 #pragma unroll
-            for (int r = 0; r < kHzPts; ++r) {
-                const int idx = tid + r * NT;
-                if (idx < n0 + n1) {
-                    const int qq = point(idx);
-                    loc[qq] = loc[qq] - inc[r];
+                for (int r = 0; r < R; ++r) {
+                    const double l = loc[q0 + r * GNX];
+                    loc[q0 + r * GNX] = P.has(j0 + r, col) ? l - inc[r] : l;
                 }
             }
-            __syncthreads();
+        }
+        __syncthreads();
+        s = next_sweep(S.plan, s + 1);
+        if (SNAP && s < 6 && own) {
+            double* const sp = snap + (size_t)ns * GPLANE;
+#pragma unroll
+            for (int r = 0; r < R; ++r) sp[q0 + r * GNX] = loc[q0 + r * GNX];
+            ++ns;
         }
     }
-    if (SNAP && !a.out) return;
-    double* out = a.out + b3;
-    for (int q = tid; q < GPLANE; q += NT) {
-        if (a.w)
-            out[q] = loc[q];
-        else
-            out[q] = (loc[q] - trc[q]) / dt;  // gad.py:539
+    if (!own || (SNAP && !a.out)) return;
+    double* const out = a.out + b3;
+    if (a.w) {
+#pragma unroll
+        for (int r = 0; r < R; ++r) out[q0 + r * GNX] = loc[q0 + r * GNX];
+    } else {
+#pragma unroll
+        for (int r = 0; r < R; ++r) out[q0 + r * GNX] = (loc[q0 + r * GNX] - trc[q0 + r * GNX]) / dt;  // gad.py:539
     }
 }
 
 // The plane as a call of its own (the multi-level blocks: inlined into the level loop it spills registers).
-__device__ __noinline__ void hz_plane_call(const GadDev& a, int t, int m, int k, double* loc, double* trc,
-                                           unsigned* mlw, unsigned* mls) {
-    hz_plane<false>(a, t, m, k, loc, trc, mlw, mls, nullptr);
+__device__ __noinline__ void hz_plane_call(const GadDev& a, int t, int m, int k, HzLds& S) {
+    hz_plane<false>(a, t, m, k, S, nullptr);
 }
 
 // One workgroup per (member, tile, level block): LEVELS false, one level per block (a.lpb == 1); true, a.lpb
 // consecutive levels, one after the other in the same LDS planes.
 template <bool LEVELS>
-__global__ void __launch_bounds__(kHzThreads, 4) gad_hz_kernel(GadDev a) {
-    __shared__ double loc[GPLANE];
-    __shared__ double trc[GPLANE];
-    __shared__ unsigned mlw[kMaskWords], mls[kMaskWords];
+__global__ void __launch_bounds__(kHzThreads, 3) gad_hz_kernel(GadDev a) {
+    __shared__ HzLds S;
     int t, m, k0;
     if (!gad_unit(a, t, m, k0)) return;
     if (!LEVELS) {
         if (a.nlev && k0 >= a.nlev[m]) return;
-        hz_plane<false>(a, t, m, k0, loc, trc, mlw, mls, nullptr);
+        hz_plane<false>(a, t, m, k0, S, nullptr);
         return;
     }
     const int kend = min(k0 + a.lpb, a.nlev ? min(a.nlev[m], a.K) : a.K);
     for (int k = k0; k < kend; ++k) {
         if (k > k0) __syncthreads();  // the previous level's output has read the LDS planes
-        hz_plane_call(a, t, m, k, loc, trc, mlw, mls);
+        hz_plane_call(a, t, m, k, S);
     }
 }
 
@@ -438,81 +614,6 @@ __device__ __forceinline__ FluxPartials dst3_partials(double tr_, double cfl, do
     return P;
 }
 
-// The value of the next lane; `last` (uniform) in lane 63.
-__device__ __forceinline__ double next_lane(double v, double last) {
-    const int lo = __builtin_amdgcn_update_dpp(__double2loint(last), __double2loint(v), 0x130, 0xf, 0xf, false);
-    const int hi = __builtin_amdgcn_update_dpp(__double2hiint(last), __double2hiint(v), 0x130, 0xf, 0xf, false);
-    return __hiloint2double(hi, lo);
-}
-__device__ __forceinline__ double lane_value(double v, int lane) {
-    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
-                            __builtin_amdgcn_readlane(__double2loint(v), lane));
-}
-// Bit p of b as 0.0 / 1.0.
-__device__ __forceinline__ double bit01(unsigned b, int p) {
-    return __hiloint2double((((int)(b << (31 - p))) >> 31) & 0x3ff00000, 0);
-}
-// Bits i - 1, i, i + 1 of a row of a bit plane (0 before its first).
-__device__ __forceinline__ unsigned three_bits(const unsigned* row, int i) {
-    const int w = max(i - 1, 0) >> 5;
-    const unsigned long long v = ((unsigned long long)row[min(w + 1, kRowWords - 1)] << 32) | row[w];
-    return (unsigned)((i > 0 ? v >> ((i - 1) & 31) : v << 1) & 7u);
-}
-
-
-// The plan of the block's tile is kept in LDS (a byte or half word of global memory is a vector load, and would wait for
-// all loads issued before it). A sweep's entry, read uniformly; index s = 2 pass + dir.
-constexpr int kSweepWords = sizeof(MjSweep) / 4, kPlanWords = sizeof(MjTilePlan) / 4;
-static_assert(sizeof(MjSweep) == 20 && sizeof(MjTilePlan) == 124, "plan words");
-struct HzBox {
-    int i0, i1, j0, j1;
-    __device__ __forceinline__ bool has(int j, int i) const { return (i >= i0) & (i < i1) & (j >= j0) & (j < j1); }
-};
-struct HzSweep {
-    int fill_before, fill_after;
-    HzBox box[2];  // empty where the sweep has fewer
-    __device__ __forceinline__ HzSweep(const MjTilePlan& lp, int s) {
-        const int* w = (const int*)&lp + s * kSweepWords;
-        auto u = [&](int i) { return __builtin_amdgcn_readfirstlane(w[i]); };
-        const int f = u(0), nbox = f >> 24;
-        fill_before = (f >> 8) & 0xff;
-        fill_after = (f >> 16) & 0xff;
-        for (int b = 0; b < 2; ++b) {
-            const int i = u(1 + 2 * b), j = u(2 + 2 * b);
-            box[b] = b < nbox ? HzBox{i & 0xffff, i >> 16, j & 0xffff, j >> 16} : HzBox{0, 0, 0, 0};
-        }
-    }
-    // the rows j0 .. j0 + n - 1, the columns i0 .. i0 + n - 1: is one in a box's range?
-    __device__ __forceinline__ bool rows(int j, int n) const {
-        return ((j < box[0].j1) & (j + n > box[0].j0)) | ((j < box[1].j1) & (j + n > box[1].j0));
-    }
-    __device__ __forceinline__ bool cols(int i, int n) const {
-        return ((i < box[0].i1) & (i + n > box[0].i0)) | ((i < box[1].i1) & (i + n > box[1].i0));
-    }
-    __device__ __forceinline__ bool has(int j, int i) const { return box[0].has(j, i) | box[1].has(j, i); }
-};
-// The next sweep from index s on that runs, 6: none.
-__device__ __forceinline__ int next_sweep(const MjTilePlan& lp, int s) {
-    while (s < 6 && !(__builtin_amdgcn_readfirstlane(((const int*)&lp)[s * kSweepWords]) & 0xff)) ++s;
-    return s;
-}
-
-// The value of the lane before; `first` (uniform) in lane 0.
-__device__ __forceinline__ double prev_lane(double v, double first) {
-    const int lo = __builtin_amdgcn_update_dpp(__double2loint(first), __double2loint(v), 0x138, 0xf, 0xf, false);
-    const int hi = __builtin_amdgcn_update_dpp(__double2hiint(first), __double2hiint(v), 0x138, 0xf, 0xf, false);
-    return __hiloint2double(hi, lo);
-}
-
-// Element i of a plane: base in scalar registers, 32-bit offset.
-template <class T>
-__device__ __forceinline__ T ld(const T* p, int i) {
-    return *(const T*)((const char*)p + (unsigned)(i * (int)sizeof(T)));
-}
-
-// Forms v here: the compiler would move the arithmetic behind all loads that follow, and spill what it reads.
-__device__ __forceinline__ void pin(double& v) { asm volatile("" : "+v"(v)); }
-
 // Unit of a reverse launch: n (member, tile, level)s from u0 on, level fastest, cut into 8 contiguous ranges, one per XCD
 // (gad_unit's reason). i: its number in the launch.
 __device__ __forceinline__ bool adj_unit(const GadDev& a, int u0, int n, int& i, int& t, int& m, int& k) {
@@ -527,14 +628,12 @@ __device__ __forceinline__ bool adj_unit(const GadDev& a, int u0, int n, int& i,
 }
 
 // The forward sweeps for the reverse mode: snapshots, and localTij at a.out if given.
-__global__ void __launch_bounds__(kHzThreads, 4) gad_hz_snap_kernel(GadDev a, int u0, int n, double* snap) {
-    __shared__ double loc[GPLANE];
-    __shared__ double trc[GPLANE];
-    __shared__ unsigned mlw[kMaskWords], mls[kMaskWords];
+__global__ void __launch_bounds__(kHzThreads, 3) gad_hz_snap_kernel(GadDev a, int u0, int n, double* snap) {
+    __shared__ HzLds S;
     int i, t, m, k;
     if (!adj_unit(a, u0, n, i, t, m, k)) return;
     if (a.nlev && k >= a.nlev[m]) return;
-    hz_plane<true>(a, t, m, k, loc, trc, mlw, mls, snap + (size_t)i * kAdjSnaps * GPLANE);
+    hz_plane<true>(a, t, m, k, S, snap + (size_t)i * kAdjSnaps * GPLANE);
 }
 
 // Reverse mode of gad_hz_kernel (horizontal DST3 without R flux) for one (member, tile, level): given the cotangent gbar
@@ -591,27 +690,14 @@ __global__ void __launch_bounds__(kAdjThreads, 3)
     const int64_t b2 = (int64_t)t * GPLANE;
     const double *const tr = a.tr + b3, *const rhC = a.recip_hFacC + b3;
     const double2* const am = a.g2 + 2 * (int64_t)a.T * GPLANE + b2;  // {recip_rA, maskInC}
-    // the level's factors in scalar registers
-    auto level = [&](const double* p) {
-        const double v = p[k];
-        return __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(v)),
-                                __builtin_amdgcn_readfirstlane(__double2loint(v)));
-    };
-    const double dt = level(a.dTlev), deepFacC = level(a.deepFacC), rdeepC = level(a.recip_deepFacC);
-    const double rdeep2C = level(a.recip_deepFac2C), rhoFacC = level(a.rhoFacC), rrhoFacC = level(a.recip_rhoFacC);
-    const double drF = level(a.drF), rdrF = level(a.recip_drF), oneSixth = a.oneSixth;
+    const double dt = level_value(a.dTlev, k), deepFacC = level_value(a.deepFacC, k), rdeepC = level_value(a.recip_deepFacC, k);
+    const double rdeep2C = level_value(a.recip_deepFac2C, k), rhoFacC = level_value(a.rhoFacC, k), rrhoFacC = level_value(a.recip_rhoFacC, k);
+    const double drF = level_value(a.drF, k), rdrF = level_value(a.recip_drF, k), oneSixth = a.oneSixth;
     snap += (size_t)unit * kAdjSnaps * GPLANE;
     auto update_coef = [&](double RH, double2 AM) { return dt * rrhoFacC * RH * rdrF * AM.x * rdeep2C * AM.y; };
 
-    // element q + r GNX of a plane: 32-bit offsets and an immediate (which ends at 4095 bytes)
-    auto at8 = [&](const double* p, int q, int r) {
-        const int c = r < 7 ? 3 : 10;
-        return ((const double*)((const char*)p + (unsigned)(q + c * GNX) * 8))[(r - c) * GNX];
-    };
-    auto at16 = [&](const double2* p, int q, int r) {
-        const int c = r / 5 * 5 + 2;
-        return ((const double2*)((const char*)p + (unsigned)(q + c * GNX) * 16))[(r - c) * GNX];
-    };
+    auto at8 = [&](const double* p, int q, int r) { return plane8(p, q, r); };
+    auto at16 = [&](const double2* p, int q, int r) { return plane16(p, q, r); };
     {
         double x[R];
 #pragma unroll
@@ -1123,8 +1209,8 @@ static int build_plan_host(mj_gad_plan* P, int ntiles, const int32_t* face, cons
     return MJ_OK;
 }
 
-// What gad_hz_kernel relies on: the update boxes of a sweep are disjoint and lie in the plane together with the
-// face q + d of each of their points (so a sweep has at most GPLANE points, kHzPts per thread).
+// What the kernels rely on: the update boxes of a sweep are disjoint and lie in the plane together with the face q + d of
+// each of their points.
 static int check_boxes(const mj_gad_plan& P) {
     for (int t = 0; t < P.ntiles; ++t)
         for (int pass = 0; pass < 3; ++pass)
