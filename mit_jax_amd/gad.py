@@ -167,6 +167,12 @@ def _dev(a, device, name):
     return torch.as_tensor(np.ascontiguousarray(a, dtype=np.float64), device=device)
 
 
+def _within(t, lo, hi):
+    """Are all values of a device tensor in lo..hi? (one wait for the device, not one per bound)"""
+    a, b = torch.stack(torch.aminmax(t)).tolist()
+    return lo <= a and b <= hi
+
+
 def _prepare(params, tables, grid2d, vgrid, uFld, vFld, tracer, hFacW, hFacS, recip_hFacC, wFld, nlev):
     """Checked device arguments of the DST3 entry points."""
     L = params.layout
@@ -205,7 +211,7 @@ def _prepare(params, tables, grid2d, vgrid, uFld, vFld, tracer, hFacW, hFacS, re
         if mi is not None:
             midx = torch.as_tensor(np.asarray(mi, np.int32).reshape(-1), device=dev) \
                 if not isinstance(mi, torch.Tensor) else mi.to(device=dev, dtype=torch.int32).contiguous()
-            if midx.numel() != B or int(midx.min()) < 0 or int(midx.max()) >= mshape[0]:
+            if midx.numel() != B or not _within(midx, 0, mshape[0] - 1):
                 raise ValueError(f"mask_index: {B} slot numbers in 0..{mshape[0] - 1} expected")
         elif mshape[0] != B:
             raise ValueError(f"maskW: {mshape[0]} mask slots for {B} members need grid2d['mask_index']")
@@ -220,11 +226,11 @@ def _prepare(params, tables, grid2d, vgrid, uFld, vFld, tracer, hFacW, hFacS, re
         "drF": vgrid["drF"], "recip_drF": vgrid["recip_drF"], "rhoFacC": vgrid["rhoFacC"],
         "recip_drC": vgrid.get("recip_drC"),
     }
-    vt = {}
+    vert = {k: v for k, v in vert.items() if v is not None}
+    host = [k for k, v in vert.items() if not isinstance(v, torch.Tensor)]
+    vt = dict(zip(host, _lib.to_device_f64([vert[k] for k in host], dev)))
     for k, v in vert.items():
-        if v is None:
-            continue
-        t = _dev(np.asarray(v, np.float64) if not isinstance(v, torch.Tensor) else v, dev, k).reshape(-1)
+        t = vt[k] if k in vt else _dev(v, dev, k).reshape(-1)
         if t.numel() < K:
             raise ValueError(f"{k}: {t.numel()} levels < {K}")
         vt[k] = t
@@ -243,7 +249,7 @@ def _prepare(params, tables, grid2d, vgrid, uFld, vFld, tracer, hFacW, hFacS, re
     if nlev is not None:
         nl = torch.as_tensor(np.asarray(nlev, np.int32).reshape(-1), device=dev) if not isinstance(nlev, torch.Tensor) \
             else nlev.to(device=dev, dtype=torch.int32).contiguous()
-        if nl.numel() != B or int(nl.max()) > K or int(nl.min()) < 0:
+        if nl.numel() != B or not _within(nl, 0, K):
             raise ValueError("nlev: one value in 0..K per member")
     cfg = _lib.GadConfig(B, K, T * K * ny * nx, mms, _lib.ptr(nl), _lib.ptr(midx))
     cfg.mask_slots = mshape[0] if len(mshape) == 5 else 1

@@ -68,10 +68,10 @@ def _structs(p, g, L, B, T, K, ny, nx, implicitAdvection, dev):
         if tuple(mC.shape) != (B, T, K, ny, nx):
             raise ValueError("maskC: expected [T, Nr, ny, nx] or [B, T, Nr, ny, nx]")
         mms = T * K * ny * nx
-    keep = dict(maskC=mC, rA=_f64(g.rA, dev, "rA"), recip_rA=_f64(g.recip_rA, dev, "recip_rA"),
-                dt=_f64(np.asarray(p.dTtracerLev, np.float64).reshape(-1)[:K], dev, "dTtracerLev"),
-                rdrF=_f64(np.asarray(g.recip_drF, np.float64).reshape(-1)[:K], dev, "recip_drF"),
-                rdrC=_f64(np.asarray(g.recip_drC, np.float64).reshape(-1)[:K], dev, "recip_drC"))
+    dt, rdrF, rdrC = _lib.to_device_f64([np.asarray(a, np.float64).reshape(-1)[:K]
+                                         for a in (p.dTtracerLev, g.recip_drF, g.recip_drC)], dev)
+    keep = dict(maskC=mC, rA=_f64(g.rA, dev, "rA"), recip_rA=_f64(g.recip_rA, dev, "recip_rA"), dt=dt, rdrF=rdrF,
+                rdrC=rdrC)
     for n in ("dt", "rdrF", "rdrC"):
         if keep[n].numel() != K:
             raise ValueError(f"{n}: fewer than {K} levels")
