@@ -952,6 +952,12 @@ __global__ void __launch_bounds__(kAdjThreads, 3)
 // with t = localTij after the horizontal passes. Update (the horizontal form, net outflow wT(k) - wT(k+1)):
 //   local(k) <- local(k) - coef(k) ((wT(k) - wT(k+1)) - tracer(k) (rTrans(k) - rTrans(k+1))) maskC(k),
 // gTracer = (local - tracer)/dt(k) on the whole tile array.
+//
+// Bound by HBM: one walk down the column, step k takes level k in, evaluates interface k - 1 and completes level k - 2; the
+// level data are loaded kVertAhead steps ahead. With one step's loads in flight one member of 50 levels (300 MB) took 98 us;
+// 75 us now, 4 TB/s. 24 members, which fill the card by themselves, take 1.01 ms either way (5.1 TB/s with the masks that
+// members share). One, two and four steps ahead measure the same, six 2 us more.
+constexpr int kVertAhead = 2;
 __global__ void __launch_bounds__(256) gad_vert_kernel(GadDev a, const double* __restrict__ loc_h) {
     const int q = blockIdx.x * blockDim.x + threadIdx.x;
     const int mt = blockIdx.y;
@@ -961,50 +967,57 @@ __global__ void __launch_bounds__(256) gad_vert_kernel(GadDev a, const double* _
     const int kmax = a.nlev ? a.nlev[m] : K;
     const int64_t b2 = (int64_t)t * GPLANE + q;
     const double rA = a.rA[b2], rrA = a.recip_rA[b2];
-    const double* __restrict__ w = a.w + m * a.ms3 + (int64_t)t * K * GPLANE + q;
-    const double* __restrict__ tr = a.tr + m * a.ms3 + (int64_t)t * K * GPLANE + q;
-    const double* __restrict__ rhC = a.recip_hFacC + m * a.ms3 + (int64_t)t * K * GPLANE + q;
-    const double* __restrict__ lh = loc_h + m * a.ms3 + (int64_t)t * K * GPLANE + q;
+    const int64_t c3 = m * a.ms3 + (int64_t)t * K * GPLANE + q;
+    const double* __restrict__ w = a.w + c3;
+    const double* __restrict__ tr = a.tr + c3;
+    const double* __restrict__ rhC = a.recip_hFacC + c3;
+    const double* __restrict__ lh = loc_h + c3;
     const double* __restrict__ mc = a.maskC + mask_slot(a, m) * a.mms + (int64_t)t * K * GPLANE + q;
-    double* __restrict__ out = a.out + m * a.ms3 + (int64_t)t * K * GPLANE + q;
-    // the column as a window over k: T(k-1) .. T(k+2), maskC(k-1) .. maskC(k+2) (0 outside 0 .. kmax-1); each level
-    // loads one new localTij, maskC and w value (the expressions are those of the formulas above)
-    auto Tk = [&](int k) { return (k >= 0 && k < kmax) ? lh[(int64_t)k * GPLANE] : 0.0; };
-    auto Mk = [&](int k) { return (k >= 0 && k < kmax) ? mc[(int64_t)k * GPLANE] : 0.0; };
-    double Tm1 = 0.0, T0 = Tk(0), Tp1 = Tk(1), Tp2 = Tk(2);
-    double Mm1 = 0.0, M0 = Mk(0), Mp1 = Mk(1), Mp2 = Mk(2);
-    // interface k + 1 from the window centred on level k: mk(k+1) = M0 Mp1, mk(k+2) = Mp1 Mp2, mk(k) = Mm1 M0
-    auto iface = [&](int k, double& wTk, double& rTk) {
-        wTk = 0.0;
-        rTk = 0.0;
-        const int ki = k + 1;
-        if (ki < 1 || ki > kmax - 1) return;
-        const double wk = w[(int64_t)ki * GPLANE];
-        const double mk1 = M0 * Mp1;
-        rTk = wk * rA * mk1;
-        const double cfl = fabs(wk * a.dTlev[ki] * a.recip_drC[ki]);
-        // upstream for positive (upward) transport: cell k+1, then k+2; downstream: k, then k-1
-        wTk = dst3_flux(rTk, cfl, a.oneSixth, Tp2, Tp1, T0, Tm1, Mp1 * Mp2, mk1, Mm1 * M0);
+    double* __restrict__ out = a.out + c3;
+    auto L = [](int k) { return (int64_t)k * GPLANE; };
+    double rw[kVertAhead], rtr[kVertAhead], rrh[kVertAhead], rlh[kVertAhead], rmc[kVertAhead];
+    auto load = [&](int s, int k) {
+        const int64_t o = L(max(min(k, kmax - 1), 0));
+        rw[s] = w[o];
+        rtr[s] = tr[o];
+        rrh[s] = rhC[o];
+        rlh[s] = lh[o];
+        rmc[s] = mc[o];
     };
-    double wTop = 0.0, rTop = 0.0;  // interface 0: the surface
-    for (int k = 0; k < kmax; ++k) {
-        double wBot, rBot;
-        iface(k, wBot, rBot);
-        const double trk = tr[(int64_t)k * GPLANE];
-        const double cf = a.dTlev[k] * a.recip_rhoFacC[k] * rhC[(int64_t)k * GPLANE] * a.recip_drF[k] * rrA *
-                          a.recip_deepFac2C[k];
-        const double loc = T0 - cf * ((wTop - wBot) - trk * (rTop - rBot)) * M0;
-        out[(int64_t)k * GPLANE] = (loc - trk) / a.dTlev[k];
-        wTop = wBot;
-        rTop = rBot;
-        Tm1 = T0;
-        T0 = Tp1;
-        Tp1 = Tp2;
-        Tp2 = Tk(k + 3);
-        Mm1 = M0;
-        M0 = Mp1;
-        Mp1 = Mp2;
-        Mp2 = Mk(k + 3);
+#pragma unroll
+    for (int s = 0; s < kVertAhead; ++s) load(s, s);
+    // levels k - 1, k - 2, k - 3 (1, 2, 3), 0 outside 0 .. kmax - 1; wT2, rT2: interface k - 2
+    double T1 = 0.0, T2 = 0.0, T3 = 0.0, M1 = 0.0, M2 = 0.0, mk1 = 0.0, mk2 = 0.0, w1 = 0.0, tr1 = 0.0, tr2 = 0.0, rh1 = 0.0,
+           rh2 = 0.0, wT2 = 0.0, rT2 = 0.0;
+    auto step = [&](int k, int s) {
+        const bool wet = k < kmax;
+        const double T0 = wet ? rlh[s] : 0.0, M0 = wet ? rmc[s] : 0.0, w0 = rw[s], tr0 = rtr[s], rh0 = rrh[s];
+        load(s, k + kVertAhead);
+        const double mk0 = k >= 1 ? M1 * M0 : 0.0;
+        // interface k - 1: upstream for positive (upward) transport: cell k-1, then k; downstream: k-2, then k-3
+        double wT1 = 0.0, rT1 = 0.0;
+        const int ki = k - 1;
+        if (ki >= 1 && ki <= kmax - 1) {
+            rT1 = w1 * rA * mk1;
+            const double cfl = fabs(w1 * a.dTlev[ki] * a.recip_drC[ki]);
+            wT1 = dst3_flux(rT1, cfl, a.oneSixth, T0, T1, T2, T3, mk0, mk1, mk2);
+        }
+        const int l = k - 2;
+        if (l >= 0) {
+            const double cf = a.dTlev[l] * a.recip_rhoFacC[l] * rh2 * a.recip_drF[l] * rrA * a.recip_deepFac2C[l];
+            const double loc = T2 - cf * ((wT2 - wT1) - tr2 * (rT2 - rT1)) * M2;
+            out[L(l)] = (loc - tr2) / a.dTlev[l];
+        }
+        T3 = T2, T2 = T1, T1 = T0;
+        M2 = M1, M1 = M0;
+        mk2 = mk1, mk1 = mk0;
+        w1 = w0, tr2 = tr1, tr1 = tr0, rh2 = rh1, rh1 = rh0, wT2 = wT1, rT2 = rT1;
+    };
+    // steps 0 .. kmax + 1, the last two to complete the column
+    for (int k0 = 0; k0 < kmax + 2; k0 += kVertAhead) {
+#pragma unroll
+        for (int s = 0; s < kVertAhead; ++s)
+            if (k0 + s < kmax + 2 && kmax > 0) step(k0 + s, s);
     }
 }
 
@@ -1022,7 +1035,6 @@ __global__ void __launch_bounds__(256) gad_vert_kernel(GadDev a, const double* _
 // writes what is complete, so each of the six arrays is read once and each of the three written once; the level data are
 // loaded kVertAhead steps ahead. Bound by HBM: reading them as needed, with locbar updated in memory, took 240 us for one
 // member of 50 levels; 82 us now (450 MB, 5.5 TB/s).
-constexpr int kVertAhead = 4;
 __global__ void __launch_bounds__(256) gad_vert_adjoint_kernel(GadDev a, int col0, const double* __restrict__ loc_h,
                                                                const double* __restrict__ gbar,
                                                                double* __restrict__ locbar, double* __restrict__ trb,
