@@ -113,7 +113,7 @@ def _norm_tensor(cg2dNorm, B, device):
     if isinstance(cg2dNorm, torch.Tensor):
         n = cg2dNorm.to(device=device, dtype=torch.float64).reshape(-1)
     else:
-        n = torch.as_tensor(np.asarray(cg2dNorm, dtype=np.float64).reshape(-1), device=device)
+        n = _lib.to_device_f64([cg2dNorm], device)[0]
     if n.numel() == 1 and B > 1:
         n = n.expand(B)
     if n.numel() != B:
