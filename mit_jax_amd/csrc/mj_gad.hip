@@ -37,8 +37,8 @@ struct GadDev {
     const double *u, *v, *w, *tr, *hFacW, *hFacS, *recip_hFacC;
     double* out;  // gTracer (no R flux) or localTij after the horizontal passes (R flux follows)
     const int32_t* nlev;
-    unsigned* mbits;  // maskLocW / maskLocS bit planes per (mask slot, tile, level), gad_maskbits_kernel
-    double2* g2;  // per tile, the 2-D metrics a sweep point reads, in pairs (gad_pack2d_kernel): [3][T][GPLANE]
+    unsigned* mbits;  // maskLocW / maskLocS bit planes per (mask slot, tile, level), gad_pre_kernel
+    double2* g2;  // per tile, the 2-D metrics a sweep point reads, in pairs (gad_pre_kernel): [3][T][GPLANE]
                   // {dyG, recip_dxC} (X faces), {dxG, recip_dyC} (Y faces), {recip_rA, maskInC}
 };
 
@@ -158,44 +158,73 @@ __device__ __forceinline__ bool gad_unit(const GadDev& a, int& t, int& m, int& k
     return true;
 }
 
-// maskLocW / maskLocS of every (mask slot, tile, level) as bit planes in global memory, once per call: the DST3
-// blocks of the members that share a slot load its words instead of the two mask planes (2 x 77 KB). The masks are 0/1 by
-// construction (hFac != 0), so a bit and its double 0.0/1.0 carry the same value. Off the four corner halo squares mask_loc
-// is the plain mask, so every wave ballots half rows of maskW / maskS; then the points of the corner squares of the corners
-// the tile has are set from mask_loc.
+// The tables of a call. First maskLocW / maskLocS of every (mask slot, tile, level) as bit planes in global memory: the
+// DST3 blocks of the members that share a slot load its words instead of the two mask planes (2 x 77 KB). The masks are 0/1
+// by construction (hFac != 0), so a bit and its double 0.0/1.0 carry the same value. Off the four corner halo squares
+// mask_loc is the plain mask, so every wave ballots rows of maskW / maskS, a pair of points a lane; then the points of the
+// corner squares of the corners the tile has are set from mask_loc. Then, in the blocks behind them, the 2-D metrics in the
+// pairs the sweeps load together (one 16-byte load instead of two 8-byte ones).
 //
-// One workgroup per mask plane, all its loads in flight at once: one member of 50 levels (100 MB) took 49 us with both
-// planes in a workgroup of 256 threads and 16 words at a time; 38 us now.
-constexpr int kBitsThreads = 512;
-__global__ void __launch_bounds__(kBitsThreads) gad_maskbits_kernel(GadDev a, int nslots) {
+// Bound by HBM: one workgroup per mask plane, all its loads in flight at once. One member of 50 levels (100 MB) took 49 us
+// with both planes in a workgroup of 256 threads and 16 words at a time, 38 us with single points, and the metrics 5 us in
+// a launch of their own; 25 us together now (4 TB/s).
+constexpr int kPreThreads = 512;
+__device__ __forceinline__ unsigned spread16(unsigned x) {  // bit i to bit 2 i
+    x = (x | x << 8) & 0x00ff00ffu;
+    x = (x | x << 4) & 0x0f0f0f0fu;
+    x = (x | x << 2) & 0x33333333u;
+    return (x | x << 1) & 0x55555555u;
+}
+__global__ void __launch_bounds__(kPreThreads) gad_pre_kernel(GadDev a, int nplanes) {
+    const int tid = threadIdx.x;
+    if ((int)blockIdx.x >= nplanes) {
+        const int64_t n = (int64_t)a.T * GPLANE, q = (int64_t)(blockIdx.x - nplanes) * kPreThreads + tid;
+        if (q >= n) return;
+        a.g2[q] = make_double2(a.dyG[q], a.recip_dxC[q]);
+        a.g2[n + q] = make_double2(a.dxG[q], a.recip_dyC[q]);
+        a.g2[2 * n + q] = make_double2(a.recip_rA[q], a.maskInC[q]);
+        return;
+    }
     __shared__ unsigned b[kMaskWords];
     const int u = blockIdx.x >> 1, want_u = !(blockIdx.x & 1);
     const int k = u % a.K, st = u / a.K, t = st % a.T, sl = st / a.T;
-    if (sl >= nslots) return;
     const MjTilePlan& tp = a.tiles[t];
     const int64_t bm = sl * a.mms + ((int64_t)t * a.K + k) * GPLANE;
     const double *const mW = a.maskW + bm, *const mS = a.maskS + bm, *const mk = want_u ? mW : mS;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    constexpr int NW = kBitsThreads / 64, N = (2 * GNY + NW - 1) / NW;  // half rows of a wave
-    double v[N];
+    const int lane = tid & 63, wave = tid >> 6;
+    constexpr int NW = kPreThreads / 64, N = (GNY + NW - 1) / NW;  // rows of a wave
+    static_assert(GNX % 2 == 0 && GNX / 2 <= 64, "a pair of points a lane");
+    const bool on = lane < GNX / 2;
+    double2 v[N];
+    if (((uintptr_t)mk & 15) == 0) {
 #pragma unroll
-    for (int r = 0; r < N; ++r) {
-        const int h = wave + r * NW, j = h >> 1, i = (h & 1) * 64 + lane;
-        v[r] = h < 2 * GNY && i < GNX ? mk[j * GNX + i] : 0.0;
+        for (int r = 0; r < N; ++r) {
+            const int j = wave + r * NW;
+            v[r] = on && j < GNY ? *(const double2*)(mk + j * GNX + 2 * lane) : make_double2(0.0, 0.0);
+        }
+    } else {
+#pragma unroll
+        for (int r = 0; r < N; ++r) {
+            const int j = wave + r * NW;
+            const double* const p = mk + j * GNX + 2 * lane;
+            v[r] = on && j < GNY ? make_double2(p[0], p[1]) : make_double2(0.0, 0.0);
+        }
     }
 #pragma unroll
     for (int r = 0; r < N; ++r) {
-        const int h = wave + r * NW;
-        const unsigned long long w = __ballot(v[r] != 0.0);
-        if (lane < 2 && h < 2 * GNY) b[2 * h + lane] = (unsigned)(w >> (32 * lane));
+        const int j = wave + r * NW;
+        const unsigned long long e = __ballot(v[r].x != 0.0), o = __ballot(v[r].y != 0.0);
+        if (lane < kRowWords && j < GNY)
+            b[j * kRowWords + lane] = spread16((unsigned)(e >> (16 * lane)) & 0xffffu) |
+                                      spread16((unsigned)(o >> (16 * lane)) & 0xffffu) << 1;
     }
     __syncthreads();
     // corner c (sw, se, nw, ne), point p of its OL x OL square
     const int OL = a.OLx, n = 4 * OL * OL;
-    for (int r = tid; r < n; r += kBitsThreads) {
+    for (int r = tid; r < n; r += kPreThreads) {
         const int c = r / (OL * OL), pp = r % (OL * OL);
-        const bool on = c == 0 ? tp.sw : c == 1 ? tp.se : c == 2 ? tp.nw : tp.ne;
-        if (on) {
+        const bool has = c == 0 ? tp.sw : c == 1 ? tp.se : c == 2 ? tp.nw : tp.ne;
+        if (has) {
             const int dj = pp / OL, di = pp % OL;
             const int ja = (c < 2) ? dj : a.OLy + a.sNy + dj, ia = (c % 2 == 0) ? di : a.OLx + a.sNx + di;
             unsigned* word = b + ja * kRowWords + (ia >> 5);
@@ -208,17 +237,7 @@ __global__ void __launch_bounds__(kBitsThreads) gad_maskbits_kernel(GadDev a, in
     }
     __syncthreads();
     unsigned* o = a.mbits + (int64_t)blockIdx.x * kMaskWords;
-    for (int i = tid; i < kMaskWords; i += kBitsThreads) o[i] = b[i];
-}
-
-// The 2-D metrics in the pairs the sweeps load together (one 16-byte load instead of two 8-byte ones), per call.
-__global__ void __launch_bounds__(256) gad_pack2d_kernel(GadDev a) {
-    const int64_t n = (int64_t)a.T * GPLANE;
-    const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (q >= n) return;
-    a.g2[q] = make_double2(a.dyG[q], a.recip_dxC[q]);
-    a.g2[n + q] = make_double2(a.dxG[q], a.recip_dyC[q]);
-    a.g2[2 * n + q] = make_double2(a.recip_rA[q], a.maskInC[q]);
+    for (int i = tid; i < kMaskWords; i += kPreThreads) o[i] = b[i];
 }
 
 // Box point idx (row-major, width bw) of box B: array index.
@@ -1354,16 +1373,16 @@ int launch_pre(GadDev& a, const mj_gad_config* c, void* pre, hipStream_t st) {
     const int nslots = mask_slots_of(c);
     a.mbits = (unsigned*)pre;
     a.g2 = (double2*)((char*)pre + al256(mask_bits_bytes(c, a.T)));
-    hipLaunchKernelGGL(gad_maskbits_kernel, dim3((unsigned)(2 * nslots * a.T * a.K)), dim3(kBitsThreads), 0, st, a, nslots);
-    MJ_HIP(hipGetLastError());
-    hipLaunchKernelGGL(gad_pack2d_kernel, dim3((unsigned)((a.T * GPLANE + 255) / 256)), dim3(256), 0, st, a);
+    const int nplanes = 2 * nslots * a.T * a.K;
+    const int npack = (a.T * GPLANE + kPreThreads - 1) / kPreThreads;
+    hipLaunchKernelGGL(gad_pre_kernel, dim3((unsigned)(nplanes + npack)), dim3(kPreThreads), 0, st, a, nplanes);
     MJ_HIP(hipGetLastError());
     return MJ_OK;
 }
 int check_mask_slots(const mj_gad_config* c, int ntiles) {
     MJ_REQUIRE(c->mask_member_stride == 0 || c->mask_index == nullptr || c->mask_slots >= 1,
                "mj_gad: mask_slots (the number of mask slots) is required with mask_index");
-    MJ_REQUIRE((int64_t)mask_slots_of(c) * ntiles * c->nr < (1ll << 31), "mj_gad: too many mask slots");
+    MJ_REQUIRE((int64_t)mask_slots_of(c) * ntiles * c->nr < (1ll << 30), "mj_gad: too many mask slots");
     return MJ_OK;
 }
 

@@ -233,3 +233,23 @@ def test_reverse_launches_of_whole_columns(dev, K, nlev, vertical):
             assert torch.equal(a[m], b[0]) and bool(a[m].isfinite().all())
             if nlev is not None:
                 assert bool((a[m][:, nlev[m]:] == 0).all())
+
+
+def test_unaligned_masks(dev):
+    """Masks that begin 8 bytes off a 16-byte boundary (the bit planes' pair loads fall back to single ones): the same
+    bits as aligned ones, forward and reverse."""
+    import torch
+    from mit_jax_amd import gad
+    g, g2d, vg, params, u, v, tr = _setup(dev)
+    args = [to_dev(a, dev) for a in (u, v, tr, g.hFacW, g.hFacS, g.recip_hFacC)]
+    bar = to_dev(np.random.default_rng(5).normal(size=tr.shape), dev)
+    off = dict(g2d)
+    for k in ("maskW", "maskS"):
+        buf = torch.empty(g2d[k].numel() + 1, dtype=torch.float64, device=dev)
+        off[k] = buf[1:].view(g2d[k].shape).copy_(g2d[k])
+        assert off[k].data_ptr() % 16 == 8
+    print("unaligned masks", flush=True)
+    a, b = (gad.advect_tiles(params, None, m, vg, *args) for m in (g2d, off))
+    assert torch.equal(a, b)
+    for x, y in zip(*(gad.advect_tiles_adjoint(params, None, m, vg, *args, bar) for m in (g2d, off))):
+        assert torch.equal(x, y)
