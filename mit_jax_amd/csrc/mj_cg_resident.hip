@@ -88,26 +88,6 @@ __device__ __forceinline__ int row_of_lane(int lane) {
     return pair < 0 ? -1 : 2 * pair + (lane >> 4 & 1);
 }
 
-// s = s + v[0], s + v[1], ... over the 16 lanes of the lane's row of 16; fma(v, 1, s) is the addition (one rounding),
-// and its operand can be broadcast within the instruction.
-__device__ __forceinline__ double add16(double s, double v) {
-    double one = 1.0;
-#define MJ_ADD1(i) "v_fmac_f64_dpp %0, %1, %2 row_newbcast:" #i " row_mask:0xf bank_mask:0xf\n"
-    asm volatile("s_nop 1\n" MJ_ADD1(0) MJ_ADD1(1) MJ_ADD1(2) MJ_ADD1(3) MJ_ADD1(4) MJ_ADD1(5) MJ_ADD1(6) MJ_ADD1(7)
-                     MJ_ADD1(8) MJ_ADD1(9) MJ_ADD1(10) MJ_ADD1(11) MJ_ADD1(12) MJ_ADD1(13) MJ_ADD1(14) MJ_ADD1(15)
-                 : "+v"(s)
-                 : "v"(v), "v"(one));
-#undef MJ_ADD1
-    return s;
-}
-// Tile-order sums of the partials in lanes kPartA.. and kPartB.. (rows 2 and 3 of 16 lanes; -0.0 in those of no tile:
-// s + -0.0 is s).
-__device__ __forceinline__ void part_sums(double v, double& A, double& B) {
-    const double s = add16(0.0, v);
-    A = lane_double(s, kPartA);
-    B = lane_double(s, kPartB);
-}
-
 // ---------------------------------------------------------------------------------------------------- Fortran order
 // Two chains of 16 additions at a time (their additions alternate: each hides the other's latency).
 __device__ __forceinline__ void add16x2(double& s, double v, double& t, double w) {
@@ -125,59 +105,108 @@ __device__ __forceinline__ void add16x2(double& s, double v, double& t, double w
 // The strictly sequential sums ((0 + v[0]) + v[1]) + ... of NS staged arrays of kN * kN values, bitwise.
 //
 // A chain of 8,100 dependent additions is bound by the latency of an FP64 addition (8.5 cycles: 29 us a sum; 12-16
-// cycles with operands from LDS, 45 us). So the chain is cut into chunks that run at the same time, two to a wave: a
-// chunk needs the running sum it starts from, which is only known approximately (the tree sums of the chunks before
-// it), up to the rounding of the chain so far, a few units in the last place. Its 64 lanes therefore run the chunk from
-// the 64 consecutive doubles around that estimate; then the chunks are put together by looking up, chunk after chunk,
-// the lane that started from the true running sum. Where no lane did, the chunks from there on run again around better
-// estimates: the first of them around its true start, the others moved by the same distance. Every pass settles at
-// least one chunk, so the result is always the chain's, whatever the data; it rarely takes more than two passes.
+// cycles with operands from LDS, 45 us). So the chain is cut into chunks that run at the same time, one to the 16 lanes of
+// a row, two instruction streams a wave: a chunk needs the running sum it starts from, which is only known approximately.
+// Its 16 lanes therefore run the chunk from the 16 consecutive doubles around an estimate, and the chunks are put together
+// by following, chunk after chunk, which of the next one's starts an end is: a walk over small integers, by lane reads.
+// Where an end is none of them, the chunks from there on run again around better estimates: the first of them around its
+// true start, the others moved by the same distance. Every pass settles at least one chunk, so the result is always the
+// chain's, whatever the data.
+//
+// The estimates have to know the rounding of the chain so far (some tens of units in the last place at its end), not only
+// its sum: each thread runs a link of 17 values from the scan of the links' sums before it, and the scan of what the links
+// add, rounded as they round, is within a few units of the running sum. (An addition rounds s + v alike from starts that
+// lie some units apart, but for ties and where the sum passes a power of two.)
+//
+// The pass is bound by the issue of the additions. 64 starts around the tree sums, in 16 chunks (8 a sum for two) with the
+// ends looked up one after the other in LDS, took 8.2 us a sum and 13.4 us for
+// two; 5.1 and 7.4 us now, of which the estimates are 1.7 and 3.1, the pass 1.3 and 2.2.
 // All threads call it; sum[q] is valid in every thread.
+constexpr int kStarts = 16, kChunks = 8 * kWaves, kLink = 17, kLinks = (kN * kN + kLink - 1) / kLink;
+static_assert(kLinks <= kThreads && kLink % 2 == 1, "a link a thread, no two lanes of a bank group in one bank");
 struct ChainLds {
-    double ends[2 * kWaves][64], center[2 * kWaves], sum[2];
-    int from[2];  // first chunk of a sum that has to run (again); all of them: done
+    double ends[kChunks * kStarts], center[kChunks], part[2][2][kWaves], sum[2];
+    // which start of the next chunk c the end is, plus 16 (c % 4): a lane number, if the start is one of those run
+    int next[kChunks * kStarts];
+    int from[2];                  // first chunk of a sum that has to run (again); all of them: done
 };
+// The sum of the lanes before this one; all: of all lanes. DPP: shifts within the rows of 16, then the last lane of a row
+// and of a half to what follows.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_or_zero(double v) {
+    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, ROWS, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, ROWS, 0xf, false);
+    return __hiloint2double(hi, lo);
+}
+__device__ __forceinline__ double wave_scan(double v, double& all) {
+    double s = v;
+    s = s + dpp_or_zero<0x111, 0xf>(s);
+    s = s + dpp_or_zero<0x112, 0xf>(s);
+    s = s + dpp_or_zero<0x114, 0xf>(s);
+    s = s + dpp_or_zero<0x118, 0xf>(s);
+    s = s + dpp_or_zero<0x142, 0xa>(s);
+    s = s + dpp_or_zero<0x143, 0xc>(s);
+    all = lane_double(s, 63);
+    return dpp_or_zero<0x138, 0xf>(s);
+}
 template <int NS>
 __device__ __forceinline__ void tile_chain(const double* st0, const double* st1, ChainLds& C) {
-    constexpr int NC = 2 * kWaves / NS, n = kN * kN;  // chunks of a sum
-    constexpr int len = (n + NC - 1) / NC, steps = (len + 15) / 16;
+    constexpr int NC = kChunks / NS, n = kN * kN;  // chunks of a sum
+    constexpr int links = (kLinks + NC - 1) / NC, len = links * kLink, steps = (len + 15) / 16;
+    constexpr int mid = kStarts / 2, kNone = 1 << 28;
+    static_assert(kStarts == 16 && NC % 4 == 0 && NC * links <= kThreads, "a chunk a row of lanes (the last may be empty)");
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15;
-    const int q = NS == 2 && wave >= kWaves / 2 ? 1 : 0, c = 2 * wave - q * NC;  // this wave's chunks: c, c + 1
-    const double* const v = (q ? st1 : st0) + c * len;
-    const int n1 = min(len, n - (c + 1) * len);  // values of chunk c + 1 (chunk c has len)
-    auto val = [&](int h, int k) { return k < (h ? n1 : len) ? v[h * len + k] : -0.0; };  // s + -0.0 is s
+    auto bits = [](double x) { return __double_as_longlong(x); };
+    // ---- the estimates
     {
-        double t0 = 0.0, t1 = 0.0;
-        for (int k = lane; k < len; k += 64) {
-            t0 = t0 + val(0, k);
-            t1 = t1 + val(1, k);
-        }
-        t0 = wave_tree(t0, 0.0, false);
-        t1 = wave_tree(t1, 0.0, false);
-        if (lane == 0) {
-            C.center[2 * wave] = t0;
-            C.center[2 * wave + 1] = t1;
-        }
-    }
-    if (tid < NS) C.from[tid] = 0;
-    __syncthreads();
-    if (tid < NS) {
-        double g = 0.0, d[NC];
+        auto link = [&](int w, double s) {
+            const int base = min(tid * kLink, n - kLink);  // the last link is short, some threads have none
+            const double* const p = (w ? st1 : st0) + base;
+            const int skip = tid < kLinks ? tid * kLink - base : kLink;
 #pragma unroll
-        for (int k = 0; k < NC; ++k) d[k] = C.center[tid * NC + k];
+            for (int k = 0; k < kLink; ++k) {
+                const double x = p[k];
+                s = s + (k >= skip ? x : -0.0);  // s + -0.0 is s
+            }
+            return s;
+        };
+        double start[NS], add[NS];
 #pragma unroll
-        for (int k = 0; k < NC; ++k) {
-            C.center[tid * NC + k] = g;
-            g = g + d[k];
+        for (int w = 0; w < NS; ++w) add[w] = link(w, 0.0);
+#pragma unroll
+        for (int round = 0; round < 2; ++round) {
+#pragma unroll
+            for (int w = 0; w < NS; ++w) {
+                double all;
+                start[w] = wave_scan(add[w], all);
+                if (lane == 0) C.part[round][w][wave] = all;
+            }
+            __syncthreads();
+#pragma unroll
+            for (int w = 0; w < NS; ++w) {
+                double g = 0.0;
+#pragma unroll
+                for (int k = 0; k < kWaves; ++k) g = k < wave ? g + C.part[round][w][k] : g;
+                start[w] = g + start[w];
+                if (round == 0) add[w] = link(w, start[w]) - start[w];
+            }
         }
+#pragma unroll
+        for (int w = 0; w < NS; ++w)
+            if (tid % links == 0 && tid / links < NC) C.center[w * NC + tid / links] = start[w];
+        if (tid < NS) C.from[tid] = 0;
     }
     __syncthreads();
+    const int q = NS == 2 && wave >= kWaves / 2 ? 1 : 0;
+    const int g0 = 8 * wave + (lane >> 4), g1 = g0 + 4, c0 = g0 - q * NC, c1 = c0 + 4;  // this lane's chunks
+    const double* const v = (q ? st1 : st0) + c0 * len;
+    const int n0 = min(len, n - c0 * len), n1 = min(len, n - c1 * len);
+    auto val = [&](int h, int k) { return k < (h ? n1 : n0) ? v[4 * h * len + k] : -0.0; };
     for (;;) {
-        const int from = C.from[q];
-        if (c + 1 >= from) {
-            double s = __longlong_as_double(__double_as_longlong(C.center[2 * wave]) + (lane - 32));
-            double t = __longlong_as_double(__double_as_longlong(C.center[2 * wave + 1]) + (lane - 32));
-            if (c == 0) s = 0.0;
+        if (8 * wave + 7 - q * NC >= C.from[q]) {
+            double s = __longlong_as_double(bits(C.center[g0]) + (l16 - mid));
+            double t = __longlong_as_double(bits(C.center[g1]) + (l16 - mid));
+            if (c0 == 0) s = 0.0;
             double v0 = val(0, l16), v1 = val(1, l16);
             for (int k = 0; k < steps; ++k) {
                 const double a = v0, b = v1;
@@ -185,31 +214,54 @@ __device__ __forceinline__ void tile_chain(const double* st0, const double* st1,
                 v1 = val(1, 16 * (k + 1) + l16);
                 add16x2(s, a, t, b);
             }
-            C.ends[2 * wave][lane] = s;
-            C.ends[2 * wave + 1][lane] = t;
+            auto put = [&](int g, int c, double end) {
+                C.ends[g * kStarts + l16] = end;
+                const long long d = c + 1 < NC ? bits(end) - bits(C.center[g + 1]) : 0;
+                C.next[g * kStarts + l16] = mid + (int)(d < -kNone ? -kNone : d > kNone ? kNone : d) + ((c + 1) & 3) * 16;
+            };
+            put(g0, c0, s);
+            put(g1, c1, t);
         }
         __syncthreads();
-        const int w = NS == 2 && tid >= 64 ? 1 : 0;  // the sum that this thread puts together
-        if (tid == 0 || (NS == 2 && tid == 64)) {
-            int k = C.from[w];
-            double s = k < NC ? C.center[w * NC + k] : 0.0;  // the true start of the first chunk that ran
-            while (k < NC) {
-                const long long at = __double_as_longlong(s) - __double_as_longlong(C.center[w * NC + k]) + 32;
-                if (at < 0 || at > 63) break;
-                s = C.ends[w * NC + k][at];
-                ++k;
+        const int w = wave;  // the sum that this wave puts together
+        const int f0 = w < NS ? __builtin_amdgcn_readfirstlane(C.from[w]) : NC;
+        if (f0 < NC) {
+            int off = ~0, last = 0;  // off: bits that are not those of a lane of the next chunk's, of any step
+            if (f0 == 0) {
+                int nx[NC / 4];  // chunk 4 k + j in the lanes 16 j .. 16 j + 15
+#pragma unroll
+                for (int k = 0; k < NC / 4; ++k) nx[k] = C.next[(w * NC + 4 * k) * kStarts + lane];
+                int at = mid;
+                off = 0;
+#pragma unroll
+                for (int c = 0; c < NC; ++c) {
+                    off |= at ^ (c & 3) * 16;
+                    last = at;
+                    at = __builtin_amdgcn_readlane(nx[c / 4], at);
+                }
             }
-            if (k < NC) {  // chunk k starts from s: move its estimate there and the later ones along
+            if ((off & ~(kStarts - 1)) == 0) {
+                if (lane == 0) {
+                    C.sum[w] = C.ends[(w * NC + NC - 1) * kStarts + (last & (kStarts - 1))];
+                    C.from[w] = NC;
+                }
+            } else if (lane == 0) {
+                int c = f0, run = mid;
+                double s = 0.0;
+                while (c < NC && run >= 0 && run < kStarts) {
+                    s = C.ends[(w * NC + c) * kStarts + run];
+                    run = C.next[(w * NC + c) * kStarts + run] - ((c + 1) & 3) * 16;
+                    ++c;
+                }
+                if (c == NC) C.sum[w] = s;
+                C.from[w] = c;
+                // chunk c starts from s: move its estimate there and the later ones along
                 double g = s;
-                for (int i = k; i < NC; ++i) {
-                    const double old = C.center[w * NC + i], e = C.ends[w * NC + i][32];
-                    C.center[w * NC + i] = g;
+                for (int k = c; k < NC; ++k) {
+                    const double old = C.center[w * NC + k], e = C.ends[(w * NC + k) * kStarts + mid];
+                    C.center[w * NC + k] = g;
                     g = e + (g - old);
                 }
-                C.from[w] = k;
-            } else if (C.from[w] < NC) {
-                C.from[w] = NC;
-                C.sum[w] = s;
             }
         }
         __syncthreads();

@@ -58,6 +58,36 @@ def test_resident_equals_phases(problem, B, order, tol, iters):
         assert torch.equal(d[k], dr[k]), k
 
 
+def test_resident_fortran_sums_of_hard_data(problem):
+    """The Fortran-order sums are chains cut into chunks that start from estimates; whatever the data, the bits are the
+    chain's: ties in every addition, sums that cancel to little or nothing, magnitudes over 300 decades, sums of a few
+    values among zeros, sums that pass a power of two again and again, denormal ones."""
+    from mit_jax_amd import cg2d
+    ex, cls, slots = problem
+    wet = np.where(np.abs(cls[0][0].maskC[:, 0]) > 0, 1.0, 0.0)
+    rng = np.random.default_rng(31)
+    shape = wet.shape
+    sign = np.where(rng.random(shape) < 0.5, -1.0, 1.0)
+    data = [rng.integers(-4, 5, shape) * 0.5, sign * (1.0 + 1e-15 * rng.normal(size=shape)),
+            sign * 10.0 ** rng.uniform(-150, 150, shape), np.where(rng.random(shape) < 1e-3, rng.normal(size=shape), 0.0),
+            1.0 + 0.0 * sign, np.where(np.arange(shape[2]) % 2, 1.0, -1.0) * np.ones(shape), 1e-160 * rng.normal(size=shape)]
+    b = torch.as_tensor(np.stack(data) * wet, device="cuda")
+    B = len(data)
+    norm = torch.full((B,), cls[0][2], dtype=torch.float64, device="cuda")
+    index = np.zeros(B, np.int32)
+    kw = dict(cg2dNorm=norm, tolerance=1e-7, max_iters=12, sum_order="fortran", op_index=index)
+    print("resident: Fortran order, hard sums", flush=True)
+    x, d = cg2d.cg2d_fortran(ex, slots, b, torch.zeros_like(b), **kw)
+    torch.cuda.synchronize()
+    xr, dr = cg2d.cg2d_fortran(ex, slots, b, torch.zeros_like(b), launch="phases", **kw)
+    torch.cuda.synchronize()
+    assert int(d["launches"].max()) == 0 and int(dr["launches"].max()) > 0
+    bits = lambda a: a.contiguous().view(torch.int64) if a.dtype == torch.float64 else a  # noqa: E731
+    assert torch.equal(bits(x), bits(xr))
+    for k in FIELDS:
+        assert torch.equal(bits(d[k]), bits(dr[k])), k
+
+
 @pytest.mark.parametrize("B,kw", [
     (1, {}), (1, dict(tolerance=1e6)), (3, dict(max_iters=1)), (19, dict(max_iters=37)), (20, dict(max_outer=2)),
     (49, dict(inner_tolerance=1e-2)), (50, dict(max_iters=0)), (50, dict(inner_max_iters=20)), (61, {})])
