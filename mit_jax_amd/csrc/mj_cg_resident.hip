@@ -339,18 +339,22 @@ __global__ void __launch_bounds__(kThreads, 2) cg2d_resident_kernel(ResDev a) {
     unsigned members = 0;
 
     if (tid == 0) s_bad = 0;
-    // the last exchange's words: ring value (lanes below kRingLanes) and partial sums A, B of every tile
-    auto receive = [&](bool ring, bool A, bool B, double& v, double& part) {
+    // the last exchange: ring value (lanes below kRingLanes) and the sums of the partials A, B of every tile
+    auto receive = [&](bool ring, bool A, bool B, double& v, double& sA, double& sB, bool largest = false) {
         double w[1] = {0.0};
-        part = -0.0;
         const unsigned odd = seq & 1;
         const uint64_t* const p[1] = {words + (ring_src + odd * (ring_words >> 1))};
         const bool need[1] = {ring && rneed};
+        double part = -0.0;
         if (!wait_words<2, 1>(a.y, p, need, w, words + (part_src + odd * 4u * (unsigned)T), (A && pA) || (B && pB),
                               part, seq) &&
             lane == 0)
             s_bad = 1;
         v = w[0];
+        if (largest)
+            sA = part_max(part, T);
+        else
+            part_sums(part, sA, sB);
     };
     auto publish_part = [&](int q, double v) {
         put_double(words + (ring_words + ((seq & 1) * (unsigned)T + (unsigned)t) * 4 + 2 * q), v, seq);
@@ -552,9 +556,8 @@ __global__ void __launch_bounds__(kThreads, 2) cg2d_resident_kernel(ResDev a) {
             if (lane == 0) publish_part(0, mx);
         }
         // ---- I1: x = the normalised first guess with its exchanged halo, r = b - A x
-        double rhsMax = 0.0, v, part;
-        receive(false, true, false, v, part);
-        for (int k = 0; k < T; ++k) rhsMax = fmax(rhsMax, lane_double(part, kPartA + k));
+        double rhsMax, v, unused;
+        receive(false, true, false, v, rhsMax, unused, true);
         const double rhsNorm = rhsMax != 0.0 ? 1.0 / rhsMax : 1.0;
         First f = first_row(A, aW, aS, aC);
         {
@@ -592,8 +595,7 @@ __global__ void __launch_bounds__(kThreads, 2) cg2d_resident_kernel(ResDev a) {
         // ---- I2: z = M r, eta(1)
         double err, eta, sumRHS, etaP = 1.0;
         f = first_row(M, pW, pS, pC);
-        receive(true, true, true, rring, part);
-        part_sums(part, err, sumRHS);
+        receive(true, true, true, rring, err, sumRHS);
         put_tile(r, rring);
         __syncthreads();
         if (s_bad) break;
@@ -614,10 +616,9 @@ __global__ void __launch_bounds__(kThreads, 2) cg2d_resident_kernel(ResDev a) {
         for (;; ++n) {
             // ---- B(n): stopping rule on err(n-1); s = z + beta s, q = A s, sigma
             f = first_row(A, aW, aS, aC);
-            receive(true, n > 1, true, v, part);
             {
                 double e;
-                part_sums(part, e, eta);
+                receive(true, n > 1, true, v, e, eta);
                 if (n > 1) err = e;
             }
             if (!(n - 1 < a.max_iters) || err < a.tol_sq) break;
@@ -633,9 +634,8 @@ __global__ void __launch_bounds__(kThreads, 2) cg2d_resident_kernel(ResDev a) {
             send_sum(zq, 0, [&](int k) { return s[k] * zq[k]; });
             // ---- C(n): x += alpha s, r -= alpha q, z = M r, err, eta
             f = first_row(M, pW, pS, pC);
-            receive(true, true, false, v, part);
-            double sigma, unused;
-            part_sums(part, sigma, unused);
+            double sigma;
+            receive(true, true, false, v, sigma, unused);
             const double alpha = eta / sigma;
 #pragma unroll
             for (int k = 0; k < kPts; ++k) {

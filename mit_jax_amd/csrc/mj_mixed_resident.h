@@ -95,7 +95,10 @@ __global__ void __launch_bounds__(64 * F::kWaves, F::kPerEu) mx_resident_kernel(
     float4* const ldsD = reinterpret_cast<float4*>(tile + kMrTile);  // MrTwo: d
     __shared__ float edge[2 * kMrN];
     __shared__ int s_bad, s_next;
+    __shared__ PartBox box;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, T = q.y.T;
+    // the last wave has no ring points
+    const bool part_wave = __builtin_amdgcn_readfirstlane(wave) == kMrWaves - 1;
     int g, t;
     resident_unit(q.y.G, g, t);
     // this thread's ring points: slot of the source, LDS offset and sign; and its points of the tile's edge: slot
@@ -116,25 +119,26 @@ __global__ void __launch_bounds__(64 * F::kWaves, F::kPerEu) mx_resident_kernel(
     const bool pA = lane >= kPartA && lane < kPartA + T, pB = lane >= kPartB && lane < kPartB + T;
     const unsigned part_src = ring_words + (pB ? 4u * (unsigned)(lane - kPartB) + 2u : pA ? 4u * (unsigned)(lane - kPartA) : 0u);
     unsigned seq = 0, members = 0;
-    if (tid == 0) s_bad = 0;
+    if (tid == 0) {
+        s_bad = 0;
+        box.tag = 0;
+    }
 
     // the last exchange: ring values (RW words: 0 none, 1 FP32, 2 FP64) and the partial sums A, B of every tile. Every
     // exchange waits for a sum of every tile, so that no word is overwritten before all have read it.
-    auto receive = [&](auto rw, bool B, double (&v)[kRing], double& sA, double& sB) {
-        double part = -0.0;
+    auto receive = [&](auto rw, bool B, double (&v)[kRing], double& sA, double& sB, bool largest = false) {
+        constexpr int W = decltype(rw)::value;
         const unsigned odd = seq & 1;
         const uint64_t* p[kRing];
 #pragma unroll
         for (int i = 0; i < kRing; ++i) {
             v[i] = 0.0;
-            p[i] = words + (2u * (unsigned)rslot[i] + odd * (ring_words >> 1));
+            p[i] = words + ((W > 1 ? 2u : 1u) * (unsigned)rslot[i] + odd * (ring_words >> 1));
         }
-        if (!wait_words<decltype(rw)::value, kRing>(q.y, p, rneed, v, words + (part_src + odd * 4u * (unsigned)T),
-                                                    pA || (B && pB), part, seq) &&
+        if (!wait_exchange<W, kRing>(q.y, box, part_wave, lane, p, rneed, v, words + (part_src + odd * 4u * (unsigned)T),
+                                     pA || (B && pB), largest, sA, sB, seq) &&
             lane == 0)
             s_bad = 1;
-        part_sums(part, sA, sB);  // uniform
-        return part;
     };
     const std::integral_constant<int, 0> kNoRing{};
     const std::integral_constant<int, 1> kRing32{};
@@ -160,7 +164,7 @@ __global__ void __launch_bounds__(64 * F::kWaves, F::kPerEu) mx_resident_kernel(
             const int e = anew(tid) + i * kMrThreads;
             const float* p = e < 2 * kMrN ? edge + e
                                           : tile + (e % kMrN + 1) * kMrW + (e < 3 * kMrN ? 0 : 1);
-            if (eslot[i] >= 0) put_float(words + (2u * (unsigned)eslot[i] + (seq & 1) * (ring_words >> 1)), *p, seq);
+            if (eslot[i] >= 0) put_float(words + ((unsigned)eslot[i] + (seq & 1) * (ring_words >> 1)), *p, seq);
         }
     };
     // where the slots are, and which are a row's first or last (2 columns and padding)
@@ -357,11 +361,8 @@ __global__ void __launch_bounds__(64 * F::kWaves, F::kPerEu) mx_resident_kernel(
         unit_I0(a, m, t);
         ++seq;
         if (tid == 0) publish_part(0, a.pmax[m * a.T + t]);
-        double rhsMax = 0.0;
-        {
-            const double part = receive(kNoRing, false, v, sA, sB);
-            for (int k = 0; k < T; ++k) rhsMax = fmax(rhsMax, lane_double(part, kPartA + k));
-        }
+        double rhsMax;
+        receive(kNoRing, false, v, rhsMax, sB, true);
         if (t == 0 && tid == 0) a.diag[m].rhsMax = rhsMax;
         const double rhsNorm = uniform(rhsMax != 0.0 ? 1.0 / rhsMax : 1.0);
         mx_first_rows(a, m, t, rhsNorm);

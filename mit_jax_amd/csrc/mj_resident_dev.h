@@ -17,10 +17,22 @@ __device__ __forceinline__ void put_word(uint64_t* p, uint64_t v) {
 __device__ __forceinline__ uint64_t get_word(const uint64_t* p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
+// A double is two neighbouring words, 16-byte aligned, stored and loaded as one access with the cache policy of the words
+// (agent scope): each half carries its tag, so it does not matter whether the access is one. The words of an exchange are
+// what bounds it (they go past the L2s): with two accesses a double 64 members to 1e-12 took 20.3 ms and 128 members of the
+// mixed solve 8.9; 17.4 and 7.6 with one. Polling more often than a poll takes (two in flight) made 22.7 and 12.8 of it.
+typedef unsigned ResPair __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ void put_double(uint64_t* p, double v, unsigned tag) {
-    const uint64_t hi = (uint64_t)tag << 32;
-    put_word(p, hi | (unsigned)__double2loint(v));
-    put_word(p + 1, hi | (unsigned)__double2hiint(v));
+    const ResPair w = {(unsigned)__double2loint(v), tag, (unsigned)__double2hiint(v), tag};
+    // a store of more than 8 bytes must not be followed at once by a write of its data registers (the compiler sees to
+    // that for its own stores only)
+    asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" : : "v"(p), "v"(w) : "memory");
+}
+__device__ __forceinline__ void get_pair(const uint64_t* p, uint64_t& a, uint64_t& b) {
+    ResPair w;
+    asm volatile("global_load_dwordx4 %0, %1, off sc1\n\ts_waitcnt vmcnt(0)" : "=&v"(w) : "v"(p) : "memory");
+    a = (uint64_t)w.y << 32 | w.x;
+    b = (uint64_t)w.w << 32 | w.z;
 }
 // Whether a wait that began at t0 (0: now) is to end: it took too long, or another workgroup gave up.
 __device__ __forceinline__ bool gave_up(const ResSync& a, unsigned long long& t0) {
@@ -52,13 +64,12 @@ __device__ __forceinline__ bool wait_words(const ResSync& a, const uint64_t* con
 #pragma unroll
         for (int i = 0; i < N; ++i)
             if (wp[i]) {
-                p0[i] = get_word(p[i]);
-                if (PW > 1) p1[i] = get_word(p[i] + 1);
+                if (PW > 1)
+                    get_pair(p[i], p0[i], p1[i]);
+                else
+                    p0[i] = get_word(p[i]);
             }
-        if (wq) {
-            q0 = get_word(q);
-            q1 = get_word(q + 1);
-        }
+        if (wq) get_pair(q, q0, q1);
         bool wait = false;
 #pragma unroll
         for (int i = 0; i < N; ++i) {
@@ -146,6 +157,50 @@ __device__ __forceinline__ void part_sums(double v, double& A, double& B) {
     const double s = add16(0.0, v);
     A = lane_double(s, kPartA);
     B = lane_double(s, kPartB);
+}
+
+// The largest of the partials A >= 0 of T tiles.
+__device__ __forceinline__ double part_max(double v, int T) {
+    double A = 0.0;
+    for (int k = 0; k < T; ++k) A = fmax(A, lane_double(v, kPartA + k));
+    return A;
+}
+// An exchange of the mixed solve: the words at p for the lanes with need_p; and the sums of the partials A, B (at q, in the
+// lanes with need_q), or with `largest` the largest A >= 0, uniform in every wave. One wave of the workgroup (mine) polls
+// the partials and tells the others through LDS: with every wave polling them, the few lines that hold a member's sums were
+// read by all its waves, and 128 members took 7.6 ms; 6.7 with one. (In the FP64 solve every wave polls them beside its
+// ring values: there the wait for the one costs more, 18.0 ms against 17.4 for 64 members to 1e-12.) A barrier has to lie
+// between two calls.
+struct PartBox {
+    double a, b;
+    unsigned tag;
+};
+template <int PW, int N>
+__device__ __forceinline__ bool wait_exchange(const ResSync& a, PartBox& box, bool mine, int lane,
+                                              const uint64_t* const (&p)[N], const bool (&need_p)[N], double (&vp)[N],
+                                              const uint64_t* q, bool need_q, bool largest, double& sA, double& sB,
+                                              unsigned tag) {
+    double part = -0.0;
+    const bool ok = wait_words<PW, N>(a, p, need_p, vp, q, mine && need_q, part, tag);
+    if (mine) {
+        sB = 0.0;
+        if (largest)
+            sA = part_max(part, a.T);
+        else
+            part_sums(part, sA, sB);
+        if (lane == 0) {
+            box.a = sA;
+            box.b = sB;
+        }
+        // after a wait that timed out, too: the others go on to the barrier behind which they look at the error
+        __hip_atomic_store(&box.tag, tag, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+    } else {
+        while (__hip_atomic_load(&box.tag, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) != tag)
+            __builtin_amdgcn_s_sleep(1);
+        sA = uniform(box.a);
+        sB = uniform(box.b);
+    }
+    return ok;
 }
 
 }  // namespace mj
