@@ -1010,10 +1010,10 @@ extern "C" int mj_cg2d_solve_mixed(const mj_halo_plan* plan_T, const mj_cg2d_ops
         resident_fits(P, cfg)) {
         bool capturing = false, done = false;
         if ((rc = stream_capturing(st, &capturing))) return rc;
-        // MrOne up to 2.5 members per place (19 on 256 CUs), MrTwo beyond: on 256 CUs, 13 tiles, mixed level counts, one
-        // / two workgroups per CU take 2.50 / 2.77 ms for 20 members, 3.88 / 3.99 for 39, 5.37 / 4.67 for 57, 10.9 /
-        // 9.2 for 128 (the step launches 6.8, 7.9, 10.0, 18.7)
-        auto* const solve = 2 * (int64_t)a.B * a.T <= 5 * (int64_t)ncu ? mx_resident_solve<MrOne> : mx_resident_solve<MrTwo>;
+        // MrOne up to 16/7 members per place (45 of 19 places on 256 CUs with 13 tiles), MrTwo beyond: with mixed level
+        // counts one / two workgroups per CU take 2.07 / 2.72 ms for 20 members, 3.14 / 3.23 for 39, 3.16 / 3.29 for 45,
+        // 3.51 / 3.29 for 49, 3.85 / 3.30 for 57, 8.5 / 7.0 for 128 (the step launches 6.8, 7.9, -, -, 10.0, 18.7)
+        auto* const solve = 7 * (int64_t)a.B * a.T <= 16 * (int64_t)ncu ? mx_resident_solve<MrOne> : mx_resident_solve<MrTwo>;
         if (!capturing && (rc = solve(a, P, ops, cfg, nslots, w + L.r0, L.coef - L.r0, st, &done))) return rc;
         if (done) return MJ_OK;
     }

@@ -90,9 +90,9 @@ def test_resident_fortran_sums_of_hard_data(problem):
 
 @pytest.mark.parametrize("B,kw", [
     (1, {}), (1, dict(tolerance=1e6)), (3, dict(max_iters=1)), (19, dict(max_iters=37)), (20, dict(max_outer=2)),
-    (49, dict(inner_tolerance=1e-2)), (50, dict(max_iters=0)), (50, dict(inner_max_iters=20)), (61, {})])
+    (45, dict(inner_tolerance=1e-2)), (46, dict(max_iters=0)), (46, dict(inner_max_iters=20)), (61, {})])
 def test_mixed_resident_equals_steps(problem, B, kw):
-    """The mixed solve's resident launches (one workgroup per CU up to 49 members on 256 CUs, two beyond) against its
+    """The mixed solve's resident launches (one workgroup per CU up to 45 members on 256 CUs, two beyond) against its
     step launches."""
     from mit_jax_amd import mixed
     ex, cls, slots = problem
