@@ -61,6 +61,10 @@ int mj_version(void);
 /* Copies the last error message of the calling thread into buf (NUL-terminated); returns its full length. */
 int mj_last_error(char* buf, size_t n);
 
+/* Puts n doubles of host memory (read before the call returns) at dst on the device, in launches that carry them as
+ * arguments: no copy, so nothing waits for the work queued before. Meant for a call's level vectors. */
+int mj_put_doubles(const double* host, int64_t n, double* dst, void* stream);
+
 /* ======================================================================================= exch2 halo exchange
  * Replaces Exchanger.scalar / vector / exch_xy / exch_uv_xy (parallel/exchange.py:136-142, :170-186): for each
  * written point d of the output component, out[d] = sign[d] * in_comp[d][src[d]], comp 1 = the u-like input,

@@ -125,6 +125,7 @@ SIGNATURES = {
     "mj_gad_implicit_r": (I32, [ctypes.POINTER(ImprGrid), ctypes.POINTER(ImprConfig), P, P, P, P, P, P]),
     "mj_gad_implicit_r_adjoint": (I32, [ctypes.POINTER(ImprGrid), ctypes.POINTER(ImprConfig), P, P, P, P, P, P, P,
                                         P, P]),
+    "mj_put_doubles": (I32, [P, I64, P, P]),
     "mj_gad_plan_create": (I32, [I32, P, P, I32, I32, I32, I32, ctypes.POINTER(P)]),
     "mj_gad_plan_destroy": (I32, [P]),
     "mj_gad_plan_describe": (I32, [P, P, P]),
@@ -179,18 +180,18 @@ def ptr(t):
 
 
 def to_device_f64(arrays, device):
-    """Copies of host vectors (numpy, float64) on the device, for the current stream: one asynchronous copy out of pinned
-    memory for all of them. A copy each, out of pageable memory, waits for all work queued before it (some 15 us each, and
-    the queue is empty behind it): five of them in a DST3 call held up one member's 200 us of kernels by 90 us."""
-    arrays = [np.ascontiguousarray(a, dtype=np.float64).reshape(-1) for a in arrays]
-    if not arrays:
-        return []
-    if torch.cuda.is_current_stream_capturing():  # a host copy has no place in a graph: the plain copy says so
-        return [torch.as_tensor(a, device=device) for a in arrays]
-    n = [a.size for a in arrays]
-    host = torch.empty(sum(n), dtype=torch.float64, device="cpu", pin_memory=True)
-    np.concatenate(arrays, out=host.numpy())
-    return list(host.to(device, non_blocking=True).split(n))
+    """Copies of host vectors (numpy, float64) on the device, for the current stream, by launches that carry them as
+    arguments (mj_put_doubles). A copy each, out of pageable memory, waits for all work queued before it (some 15 us each,
+    and the queue is empty behind it): five of them in a DST3 call held up one member's 200 us of kernels by 90 us. One
+    copy out of pinned memory does not wait, but takes 60 us more than this on a queue that is empty."""
+    index = torch.device(device).index
+    if not arrays or torch.cuda.is_current_stream_capturing() or \
+            (index is not None and index != torch.cuda.current_device()):
+        return [torch.as_tensor(np.asarray(a, dtype=np.float64).reshape(-1), device=device) for a in arrays]
+    host = np.concatenate(arrays, axis=None, dtype=np.float64)
+    out = torch.empty(host.size, dtype=torch.float64, device=device)
+    check(lib().mj_put_doubles(host.ctypes.data, host.size, out.data_ptr(), stream_ptr()), "mj_put_doubles")
+    return out.split([np.size(a) for a in arrays])
 
 
 def stream_ptr(stream=None):

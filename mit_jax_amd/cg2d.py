@@ -112,8 +112,11 @@ def _ops_struct(ops, B, L, device, op_index=None):
 def _norm_tensor(cg2dNorm, B, device):
     if isinstance(cg2dNorm, torch.Tensor):
         n = cg2dNorm.to(device=device, dtype=torch.float64).reshape(-1)
+    elif np.size(cg2dNorm) == 1 and not torch.cuda.is_current_stream_capturing():
+        # a fill, not a copy: that would wait for all work queued before it
+        return torch.full((B,), float(np.reshape(cg2dNorm, ())), dtype=torch.float64, device=device)
     else:
-        n = _lib.to_device_f64([cg2dNorm], device)[0]
+        n = torch.as_tensor(np.asarray(cg2dNorm, dtype=np.float64).reshape(-1), device=device)
     if n.numel() == 1 and B > 1:
         n = n.expand(B)
     if n.numel() != B:

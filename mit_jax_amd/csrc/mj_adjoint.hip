@@ -8,6 +8,9 @@
 //   gaS[q] = -(lambda[q] xe[q-nx] + lambda[q-nx] xe[q]) / cg2dNorm
 //   gaC[q] = -(lambda[q] xe[q]) / cg2dNorm
 // with xe = exch(where(inner, x, 0)) and lambda zero off the interior. Entries that no interior stencil reads get 0.
+#include <algorithm>
+#include <cstring>
+
 #include "mj_common.h"
 #include "mj_internal.h"
 
@@ -43,9 +46,31 @@ __global__ void zero_halo_copy_adj_kernel(const double* v, double* w, int64_t ms
     w[m * ms + q] = inner ? v[m * ms + q] : 0.0;
 }
 
+// A launch's arguments hold kPutMax doubles (they may take 4 KB).
+constexpr int kPutMax = 480;
+struct PutArgs {
+    double v[kPutMax];
+};
+__global__ void __launch_bounds__(kPutMax) put_doubles_kernel(PutArgs a, double* dst, int n) {
+    const int i = threadIdx.x;
+    if (i < n) dst[i] = a.v[i];
+}
+
 }  // namespace mj
 
 using namespace mj;
+
+extern "C" int mj_put_doubles(const double* host, int64_t n, double* dst, void* stream) {
+    MJ_REQUIRE(n >= 0 && (n == 0 || (host && dst)), "mj_put_doubles: null array or negative length");
+    for (int64_t k = 0; k < n; k += kPutMax) {
+        PutArgs a;
+        const int c = (int)std::min<int64_t>(kPutMax, n - k);
+        std::memcpy(a.v, host + k, c * sizeof(double));
+        hipLaunchKernelGGL(put_doubles_kernel, dim3(1), dim3(kPutMax), 0, as_stream(stream), a, dst + k, c);
+        MJ_HIP(hipGetLastError());
+    }
+    return MJ_OK;
+}
 
 extern "C" int mj_cg2d_coeff_grad(const mj_halo_plan* plan_T, const double* x, const double* lam,
                                   const double* cg2dNorm, double* gaW, double* gaS, double* gaC,
