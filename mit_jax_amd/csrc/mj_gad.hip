@@ -44,14 +44,22 @@ struct GadDev {
 
 // Mask slot of member m: members of one level class share their grid masks.
 __device__ __forceinline__ int64_t mask_slot(const GadDev& a, int m) { return a.mask_index ? a.mask_index[m] : m; }
-// A bit plane: four words a row, bit i of a row in its word i / 32 (one column has the same shift in all rows).
-constexpr int kRowWords = 4, kMaskWords = GNY * kRowWords;
-static_assert(GNX <= 32 * kRowWords && GNX > 64, "two wavefronts' ballots a row");
-// The bit planes of member m's masks at (tile t, level k): maskLocW's kMaskWords words, then maskLocS's.
+// A bit plane in LDS: four words a row, bit i of a row in its word i / 32 (one column has the same shift in all rows). In
+// memory its points follow one another (kPlaneBits words; a plane in rows would take 30 % more).
+constexpr int kRowWords = 4, kMaskWords = GNY * kRowWords, kPlaneBits = 2 * ((GPLANE + 63) / 64);
+static_assert(GNX > 96 && GNX < 32 * kRowWords, "words of a row");
+// The bit planes of member m's masks at (tile t, level k): maskLocW's kPlaneBits words, then maskLocS's.
 __device__ __forceinline__ const unsigned* unit_bits(const GadDev& a, int m, int t, int k) {
     const int64_t s = a.mms ? mask_slot(a, m) : 0;
-    return a.mbits + ((s * a.T + t) * a.K + k) * 2 * kMaskWords;
+    return a.mbits + ((s * a.T + t) * a.K + k) * 2 * kPlaneBits;
 }
+// Word i of a plane's rows, from the plane in memory.
+__device__ __forceinline__ unsigned row_word(const unsigned* plane, int i) {
+    const int w = i % kRowWords, bit = i / kRowWords * GNX + 32 * w;
+    const unsigned v = __builtin_amdgcn_alignbit(plane[(bit >> 5) + 1], plane[bit >> 5], bit & 31);
+    return w == kRowWords - 1 ? v & ((1u << (GNX - 96)) - 1) : v;
+}
+static_assert(((GNY - 1) * GNX + 96) / 32 + 1 < kPlaneBits, "the last row's words");
 
 // maskLocW / maskLocS: maskW / maskS with FILL_CS_CORNER_UV_RS(.FALSE.) applied (gad.py:263-281, :489-490).
 // (ia, ja) array indices; returns the corner-filled mask value at that point.
@@ -236,8 +244,18 @@ __global__ void __launch_bounds__(kPreThreads) gad_pre_kernel(GadDev a, int npla
         }
     }
     __syncthreads();
-    unsigned* o = a.mbits + (int64_t)blockIdx.x * kMaskWords;
-    for (int i = tid; i < kMaskWords; i += kPreThreads) o[i] = b[i];
+    unsigned* o = a.mbits + (int64_t)blockIdx.x * kPlaneBits;
+    static_assert(kPlaneBits <= kPreThreads, "a word a thread");
+    if (tid < kPlaneBits) {
+        const int j = 32 * tid / GNX, c = 32 * tid % GNX, w = c >> 5;
+        unsigned v = 0;
+        if (j < GNY) {
+            const unsigned* const row = b + j * kRowWords;
+            v = __builtin_amdgcn_alignbit(w + 1 < kRowWords ? row[w + 1] : 0, row[w], c & 31);
+            if (c > GNX - 32 && j + 1 < GNY) v |= row[kRowWords] << (GNX - c);
+        }
+        o[tid] = v;
+    }
 }
 
 // Box point idx (row-major, width bw) of box B: array index.
@@ -412,7 +430,8 @@ __device__ __forceinline__ void hz_plane(const GadDev& a, int t, int m, int k, H
         const int pw = tid < kPlanWords ? ((const int*)&a.tiles[t])[tid] : 0;
         static_assert(kMaskWords <= kHzThreads, "a word of each plane per thread");
         const unsigned* gb = unit_bits(a, m, t, k);
-        const unsigned w0 = tid < kMaskWords ? gb[tid] : 0, w1 = tid < kMaskWords ? gb[kMaskWords + tid] : 0;
+        const int wi = min(tid, kMaskWords - 1);
+        const unsigned w0 = row_word(gb, wi), w1 = row_word(gb + kPlaneBits, wi);
 #pragma unroll
         for (int r = 0; r < R; ++r) {
             tv[r] = at8(tr, r);
@@ -604,6 +623,7 @@ __global__ void __launch_bounds__(kHzThreads, 3) gad_hz_kernel(GadDev a) {
 // ------------------------------------------------------------------------------------------------ reverse mode
 constexpr int kAdjChunk = 1024;  // (member, tile, level)s per reverse launch, in whole columns (at least one)
 constexpr int kAdjSnaps = 5;     // snapshots of one: six sweeps, the first from the tracer itself
+constexpr int kAdjPlanes = 7;    // planes of one that the workspace allows for
 // Partial derivatives of one DST3 interface value f = A (t_m1 + d0 Rj + d1 Rjm) + Bm (t_0 - d0 Rj - d1 Rjp)
 // (A = (tr + |tr|)/2, Bm = (tr - |tr|)/2, d0 = (2-c)(1-c)/6, d1 = (1-c^2)/6): w[0..3] = df/dt_m2, df/dt_m1,
 // df/dt_0, df/dt_p1 (independent of the tracer), dtr = df/dtr, dc = df/dcfl. The derivative of |x| at 0 is taken
@@ -736,8 +756,8 @@ __global__ void __launch_bounds__(kAdjThreads, 3)
         const unsigned* gb = unit_bits(a, m, t, k);
         static_assert(kMaskWords <= kAdjThreads, "a word of each plane per thread");
         if (tid < kMaskWords) {
-            S.mlw[tid] = gb[tid];
-            S.mls[tid] = gb[kMaskWords + tid];
+            S.mlw[tid] = row_word(gb, tid);
+            S.mls[tid] = row_word(gb + kPlaneBits, tid);
         }
         if (tid < kPlanWords) ((int*)&S.plan)[tid] = ((const int*)&a.tiles[t])[tid];
     }
@@ -1345,7 +1365,7 @@ int mask_slots_of(const mj_gad_config* c) {
 }
 // The bit planes of every (mask slot, tile, level), then the packed 2-D metrics.
 size_t mask_bits_bytes(const mj_gad_config* c, int ntiles) {
-    return (size_t)mask_slots_of(c) * ntiles * c->nr * 2 * kMaskWords * sizeof(unsigned);
+    return (size_t)mask_slots_of(c) * ntiles * c->nr * 2 * kPlaneBits * sizeof(unsigned);
 }
 size_t pre_bytes(const mj_gad_config* c, int ntiles) {
     return al256(mask_bits_bytes(c, ntiles)) + al256((size_t)3 * ntiles * GPLANE * sizeof(double2));
@@ -1359,13 +1379,14 @@ size_t batch3_bytes(const mj_gad_config* c, int ntiles) {
 int adjoint_columns(const mj_gad_config* c, int ntiles) {
     return (int)std::min<int64_t>((int64_t)c->batch * ntiles, std::max(1, kAdjChunk / c->nr));
 }
-// The reverse mode's part of its workspace (before the bit planes): the snapshots, and with the R flux localTij and its
-// cotangent.
+// The reverse mode's part of its workspace (before the bit planes): the snapshots of a launch (more than kAdjChunk units
+// if one column is more), and with the R flux localTij and its cotangent, from adjoint_snap_bytes on.
 size_t adjoint_snap_bytes(const mj_gad_config* c, int ntiles) {
-    return al256((size_t)adjoint_columns(c, ntiles) * c->nr * kAdjSnaps * GPLANE * sizeof(double));
+    const size_t unit = (size_t)GPLANE * sizeof(double);
+    return std::max((size_t)kAdjChunk * kAdjPlanes * unit, (size_t)adjoint_columns(c, ntiles) * c->nr * kAdjSnaps * unit);
 }
 size_t adjoint_scratch_bytes(const mj_gad_config* c, int ntiles, int with_w) {
-    return adjoint_snap_bytes(c, ntiles) + (with_w ? 2 * al256(batch3_bytes(c, ntiles)) : 0);
+    return al256(adjoint_snap_bytes(c, ntiles) + (with_w ? 2 * batch3_bytes(c, ntiles) : 0));
 }
 // The per-call tables at `pre` (pre_bytes): the bit planes of maskLocW / maskLocS for every (mask slot, tile,
 // level) and the packed 2-D metrics; sets a.mbits and a.g2.
@@ -1527,7 +1548,7 @@ extern "C" int mj_gad_dst3_adjoint(const mj_gad_plan* P, const mj_gad_grid* g, c
     double* lbar = nullptr;
     if (wFld) {
         f.out = (double*)((char*)work + adjoint_snap_bytes(c, P->ntiles));
-        lbar = (double*)((char*)f.out + al256(batch3_bytes(c, P->ntiles)));
+        lbar = (double*)((char*)f.out + batch3_bytes(c, P->ntiles));
     }
     const int ncol = c->batch * P->ntiles, step = adjoint_columns(c, P->ntiles);
     for (int c0 = 0; c0 < ncol; c0 += step) {
