@@ -374,7 +374,10 @@ __device__ __forceinline__ double level_value(const double* p, int k) {
 // Bound by HBM: a unit moves seven planes (540 KB, 28 us of a CU's share) and takes 37 us, of which some 4 are phases
 // without loads; one member of 50 levels is 650 units on 256 CUs. Evaluating both faces at each of ten points a thread, all
 // loads of a point behind one another, took 136 us for it (122 now) and 1700 us for 24 members of mixed level counts (1615
-// now). One row ahead instead of two measured 3 % more for both, four 8 % more for the members.
+// now). One row ahead instead of two measured 3 % more for both, four 8 % more for the members. recip_rA and maskInC are
+// read from their own planes, where half of a pair would be thrown away: a row's loads are 40 bytes instead of 48 (the whole
+// step 152 -> 146 us and 3.05 -> 2.95 ms). maskInC as bits, 32 bytes, gave nothing more, nor did loading a sweep's first rows
+// before the barriers in front of it (149 us).
 constexpr int kHzRows = 14, kHzSegs = GNY / kHzRows, kHzThreads = 704, kHzSmall = 1024;
 constexpr int kHzAhead = 2;
 static_assert(kHzSegs * kHzRows == GNY && kHzSegs * GNX <= kHzThreads, "a thread per column and segment");
@@ -396,6 +399,7 @@ __device__ __forceinline__ void hz_plane(const GadDev& a, int t, int m, int k, H
     const int64_t b2 = (int64_t)t * GPLANE;
     const double* const rhC = a.recip_hFacC + b3;
     const double2* const am = a.g2 + 2 * (int64_t)a.T * GPLANE + b2;  // {recip_rA, maskInC}
+    const double *const rrA = a.recip_rA + b2, *const mIn = a.maskInC + b2;
     const double dt = level_value(a.dTlev, k), deepFacC = level_value(a.deepFacC, k), rdeepC = level_value(a.recip_deepFacC, k);
     const double rdeep2C = level_value(a.recip_deepFac2C, k), rhoFacC = level_value(a.rhoFacC, k);
     const double rrhoFacC = level_value(a.recip_rhoFacC, k), drF = level_value(a.drF, k), rdrF = level_value(a.recip_drF, k);
@@ -404,7 +408,6 @@ __device__ __forceinline__ void hz_plane(const GadDev& a, int t, int m, int k, H
     const int seg = own ? tid / GNX : 0;
     int col = own ? tid - seg * GNX : 0, j0 = seg * R, q0 = j0 * GNX + col;
     auto at8 = [&](const double* p, int r) { return plane8(p, q0, r); };
-    auto at16 = [&](const double2* p, int r) { return plane16(p, q0, r); };
     // X: lane r has row r of the point behind the wave's last lane
     int qe;
     {
@@ -436,7 +439,7 @@ __device__ __forceinline__ void hz_plane(const GadDev& a, int t, int m, int k, H
         for (int r = 0; r < R; ++r) {
             tv[r] = at8(tr, r);
             rh[r] = at8(rhC, r);
-            ra[r] = at16(am, r).x;
+            ra[r] = at8(rrA, r);
         }
         if (tid < kPlanWords) ((int*)&S.plan)[tid] = pw;
         if (tid < kMaskWords) S.mlw[tid] = w0, S.mls[tid] = w1;
@@ -510,7 +513,7 @@ __device__ __forceinline__ void hz_plane(const GadDev& a, int t, int m, int k, H
             double inc[R];
             if (dir == 0) {
                 auto load = [&](int r) {
-                    if (r < R) in[r % N] = RowIn{at8(vel, r), at8(hf, r), at16(am, r).y, at16(gr, r)};
+                    if (r < R) in[r % N] = RowIn{at8(vel, r), at8(hf, r), at8(mIn, r), plane16(gr, q0, r)};
                 };
                 const double Ve = ld(vel, qe), He = ld(hf, qe);
                 const double2 Ge = ld(gr, qe);
@@ -543,7 +546,7 @@ __device__ __forceinline__ void hz_plane(const GadDev& a, int t, int m, int k, H
                 auto lds = [&](int r) { return r >= 0 && r < R ? loc[q0 + r * GNX] : loc[beside(r)]; };
                 auto load = [&](int r) {
                     if (r < R)
-                        in[r % N] = RowIn{at8(vel, r), at8(hf, r), at16(am, r).y, at16(gr, r)};
+                        in[r % N] = RowIn{at8(vel, r), at8(hf, r), at8(mIn, r), plane16(gr, q0, r)};
                     else if (r == R)
                         in[r % N] = RowIn{ld(vel, beside(r)), ld(hf, beside(r)), 0.0, ld(gr, beside(r))};
                 };
