@@ -181,8 +181,9 @@ def single_member(E, reps=5):
     return out
 
 
-TRAFFIC_FILE = ROOT / "profiles" / "mx_step_kernel_ensemble128_traffic.md"
-TRAFFIC_FILES = (TRAFFIC_FILE, ROOT / "profiles" / "sfp_impr_kernels_ensemble128_traffic.md")
+TRAFFIC_FILES = tuple(ROOT / "profiles" / n for n in (
+    "resident_solves_gad_kernels_ensemble128.md", "mx_step_kernel_ensemble128_traffic.md",
+    "sfp_impr_kernels_ensemble128_traffic.md"))
 
 
 def measured_traffic(kernel, members):
@@ -198,6 +199,12 @@ def measured_traffic(kernel, members):
             if len(f) == 3 and f[0] == "traffic_bytes_per_launch" and f[1] == kernel:
                 return float(f[2])
     return None
+
+
+def traffic_source(kernel):
+    """The profile that measured_traffic's figure for `kernel` is from."""
+    return next((p.name for p in TRAFFIC_FILES if p.exists() and f"traffic_bytes_per_launch {kernel} " in p.read_text()),
+                None)
 
 
 def profile_solves(B):
@@ -456,11 +463,13 @@ def roofline_of(precision, cg_ms, d, op_index, members, launch):
     achieved = alg / (cg_ms * 1e-3) / 1e9
     tr = measured_traffic(kernel, members)
     return {"bound": "hbm", "kernel": kernel, "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
-            "frac": achieved / HBM_PEAK_GBS, "traffic": tr, "traffic_source": TRAFFIC_FILE.name if tr else None,
+            "frac": achieved / HBM_PEAK_GBS, "traffic": tr, "traffic_source": traffic_source(kernel) if tr else None,
             "launches": launches, "avg_launch_us": cg_ms * 1e3 / launches if launches else None,
             "algorithmic_bytes_per_launch": alg / launches if launches else None, "algorithmic_bytes": alg,
-            "operator_slot_iterations": slot_iters, "implementation_bytes": impl,
-            "implementation_GBs": impl / (cg_ms * 1e-3) / 1e9, "solve_ms": cg_ms}
+            "operator_slot_iterations": slot_iters, "solve_ms": cg_ms,
+            # of the per-phase and step launches: the resident ones keep the vectors on the chip
+            "implementation_bytes": impl if launches else None,
+            "implementation_GBs": impl / (cg_ms * 1e-3) / 1e9 if launches else None}
 
 
 def make_step(E, params, precision, args):
