@@ -13,9 +13,9 @@ The headline (default) is the mixed-precision solve (FP32 PCG + FP64 residual re
 FP64 solve (mj_cg2d_solve) is timed on the same step for `mixed_over_fp64`, and the two solutions are compared
 member by member (`error_vs_fp64`). Prints one JSON line.
 
-`roofline` is the solve's step kernel (the dominant kernel), from the solve alone on its stream (eager, not
-overlapped), timed with HIP events: achieved = algorithmic bytes per launch / average launch duration (= the solve's
-algorithmic bytes / its time; the average includes the few setup kernels and the launch gaps, so it is an upper bound
+`roofline` is the solve's kernel, from the solve alone on its stream (eager, not overlapped), timed with HIP events (a
+resident launch keeps the vectors on chip: its `achieved` exceeds the bytes it moves): achieved = algorithmic bytes per launch /
+average launch duration (= the solve's algorithmic bytes / its time; the average includes the few setup kernels and the launch gaps, so it is an upper bound
 of the profiler's per-kernel average). Algorithmic bytes are what the recurrence itself must move, per interior
 point (N2 = 105,300 per member): per member-iteration the vectors r, s, x read and written (6 streams of s_v bytes);
 per operator slot and iteration in which any member of the slot iterates, the six operator and preconditioner arrays
@@ -26,8 +26,8 @@ once; FP64: 11 FP64 streams per iteration, 48 B per point once; coefficients ser
 DST3 (`dst3`): per (member, tile, level) the padded 3-D planes the step reads (tracer, u, v, hFacW, hFacS,
 recip_hFacC, maskW, maskS; with the R flux also w) and the tendency it writes, 8 B each, plus the 2-D metrics
 (6 planes per tile) once. `traffic` = measured HBM bytes per launch from the committed FETCH_SIZE / WRITE_SIZE
-profile of this workload. `cpu_baseline` is the FP64 C oracle (OpenMP, all host cores) on a bounded sample of the
-same member-steps. `producers` times the operator builder (UPDATE_CG2D) and the rhs builder (cg2d_rhs) on the same
+profile of this workload; `implementation_bytes` is null for a resident launch. `cpu_baseline` is the
+FP64 C oracle (OpenMP, all host cores) on a bounded sample of the same member-steps. `producers` times the operator builder (UPDATE_CG2D) and the rhs builder (cg2d_rhs) on the same
 ensemble, each alone (not part of the headline step, whose operators and rhs are inputs); `implicit_r` likewise
 times GAD_IMPLICIT_R (the implicit vertical advection/diffusion solve) on the ensemble's tracer; `dst3_xyr` the DST3
 step with the vertical (R) flux. `single_member` gives B = 1, which is latency-bound and so has no roofline
