@@ -4,14 +4,14 @@
 // three passes, each an X and a Y block whose action per tile comes from the facet pass table (which direction
 // sweeps, overlap-only / interior-only update regions, FILL_CS_CORNER_TR_RL corner fills before/after the flux).
 // Everything is tile-local, so one workgroup owns one (member, tile, level): the 98x98 FP64 working tracer
-// (localTij) and the input tracer live in LDS (2 x 76.8 KB, gfx950's 160 KB LDS); each point evaluates the
-// interfaces on both its faces, velocities and metrics are read once per sweep that needs them, and only the
+// (localTij) and the input tracer live in LDS (2 x 76.8 KB, gfx950's 160 KB LDS); each interface is evaluated once
+// (twice in the small overlap sweeps), velocities and metrics are read once per sweep that needs them, and only the
 // tendency is written. The reference evaluates all six flux arrays on every tile and
 // masks; here each tile evaluates only the sweeps its table runs (2-3 of 6).
 //
 // Vertical part (R, only when wFld is given): a DST3 flux through the level interfaces applied after the
 // horizontal passes, with the same non-divergent update form. It is not in the reference (which runs the vertical
-// implicitly); its definition is written out at vert_kernel.
+// implicitly); its definition is written out at gad_vert_kernel.
 #include <string.h>
 
 #include <algorithm>
