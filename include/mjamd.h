@@ -81,6 +81,10 @@ int mj_halo_plan_create(int nmaps, const int32_t* npts, const int32_t* const* ds
 int mj_halo_plan_destroy(mj_halo_plan* plan);
 /* 1 when no written point is the source of a written point (T, 3D, UVs, UVn, UV3s): in-place fills are exact. */
 int mj_halo_plan_inplace_ok(const mj_halo_plan* plan);
+/* How long a workgroup of a resident CG2D solve with this (T) plan may wait for another one, in seconds (kept to about
+ * a millisecond): 20 unless set, 0 for a wait that is not served at its first look. The launch of a solve in which one waits longer ends early. Takes
+ * effect with the next solve; not to be called while another thread enqueues one with the same plan. */
+int mj_halo_plan_set_wait_limit(mj_halo_plan* plan, double seconds);
 
 /* Geometry of the arrays one halo call covers: element (outer o, tile t, inner n, j, i) lives at
  * o*outer_stride + t*tile_stride + n*inner_stride + j*nx + i. [T, ny, nx]: nouter = ninner = 1;

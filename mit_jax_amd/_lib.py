@@ -100,6 +100,7 @@ SIGNATURES = {
     "mj_halo_plan_create": (I32, [I32, P, P, P, P, P, I32, I32, I32, ctypes.POINTER(P)]),
     "mj_halo_plan_destroy": (I32, [P]),
     "mj_halo_plan_inplace_ok": (I32, [P]),
+    "mj_halo_plan_set_wait_limit": (I32, [P, ctypes.c_double]),
     "mj_halo_exchange": (I32, [P, P, P, ctypes.POINTER(HaloGeom), P]),
     "mj_halo_exchange_uv": (I32, [P, P, P, P, P, ctypes.POINTER(HaloGeom), P]),
     "mj_halo_exchange_adjoint": (I32, [P, P, P, P, P, ctypes.POINTER(HaloGeom), P]),

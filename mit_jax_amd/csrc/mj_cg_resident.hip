@@ -614,14 +614,14 @@ __global__ void __launch_bounds__(kThreads, 2) cg2d_resident_kernel(ResDev a) {
         bool bad = false;
         int n = 1;
         for (;; ++n) {
-            // ---- B(n): stopping rule on err(n-1); s = z + beta s, q = A s, sigma
+            // ---- B(n): stopping rule on err(n-1); s = z + beta s, q = A s, sigma. The rule comes behind the barrier and
+            // the look at s_bad: a wave whose wait failed has no err, and all waves must take the same way.
             f = first_row(A, aW, aS, aC);
             {
                 double e;
                 receive(true, n > 1, true, v, e, eta);
                 if (n > 1) err = e;
             }
-            if (!(n - 1 < a.max_iters) || err < a.tol_sq) break;
             const double beta = eta / etaP;
 #pragma unroll
             for (int k = 0; k < kPts; ++k) s[k] = zq[k] + beta * s[k];
@@ -629,6 +629,7 @@ __global__ void __launch_bounds__(kThreads, 2) cg2d_resident_kernel(ResDev a) {
             put_tile(s, sring);
             __syncthreads();
             if ((bad = s_bad)) break;
+            if (!(n - 1 < a.max_iters) || err < a.tol_sq) break;
             ++seq;
             stencil(A, aW, aS, aC, f, s, zq);
             send_sum(zq, 0, [&](int k) { return s[k] * zq[k]; });
@@ -663,6 +664,7 @@ __global__ void __launch_bounds__(kThreads, 2) cg2d_resident_kernel(ResDev a) {
             a.diag[m].numIters = n - 1;
             a.diag[m].converged = err < a.tol_sq ? 1 : 0;
         }
+        __syncthreads();  // every wave has looked at s_bad; the next member's first wait may set it
     }
     // a wait timed out: every member's record says so
     for (int m = blockIdx.x * kThreads + tid; m < a.B; m += gridDim.x * kThreads) a.diag[m].converged = -2;
@@ -752,7 +754,7 @@ int resident_prepare(const mj_halo_plan* P, const mj_cg2d_ops* ops, const mj_cg2
     y->next = w + next;
     y->queue = (int*)(w + misc);
     y->error = (int*)(w + misc + 8);
-    y->limit = (unsigned long long)(clk_khz > 0 ? clk_khz : 100000) * 1000ull * 20ull;  // 20 s
+    y->limit = (unsigned long long)((clk_khz > 0 ? clk_khz : 100000) * 1000.0 * P->res_wait_s);
     hipLaunchKernelGGL(res_init_kernel, dim3(64), dim3(256), 0, st, w, misc, y->queue, y->error);
     MJ_HIP(hipGetLastError());
     y->order = nullptr;

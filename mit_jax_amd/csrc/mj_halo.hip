@@ -227,6 +227,12 @@ extern "C" int mj_halo_plan_destroy(mj_halo_plan* plan) {
     return MJ_OK;
 }
 
+extern "C" int mj_halo_plan_set_wait_limit(mj_halo_plan* plan, double seconds) {
+    MJ_REQUIRE(plan && seconds >= 0.0 && seconds <= 1e6, "mj_halo_plan_set_wait_limit: a plan and 0..1e6 s expected");
+    plan->res_wait_s = seconds;
+    return MJ_OK;
+}
+
 extern "C" int mj_halo_plan_inplace_ok(const mj_halo_plan* plan) { return plan ? plan->inplace_ok : 0; }
 
 static int check_geom(const mj_halo_plan* plan, const mj_halo_geom* g) {

@@ -35,6 +35,7 @@ struct mj_halo_plan {
     int4* res_ring = nullptr;
     int32_t* res_pub = nullptr;
     int res_nslots = 0, res_ok = 0;
+    double res_wait_s = 20.0;  // longest wait of a resident solve (mj_halo_plan_set_wait_limit)
 
     // Transpose tables (built once, on first use): per input component c (0 = u-like, 1 = v-like) and padded
     // point q, the written points that read q (tr_off[c][q] .. tr_off[c][q+1] into tr_dst/tr_map/tr_sign, sorted by

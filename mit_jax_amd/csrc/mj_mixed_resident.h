@@ -367,7 +367,9 @@ __global__ void __launch_bounds__(64 * F::kWaves, F::kPerEu) mx_resident_kernel(
         const double rhsNorm = uniform(rhsMax != 0.0 ? 1.0 / rhsMax : 1.0);
         mx_first_rows(a, m, t, rhsNorm);
         __syncthreads();
-        if (s_bad) break;
+        const int failed = s_bad;
+        __syncthreads();  // every wave has looked at s_bad; RST's wait may set it
+        if (failed) break;
         ++seq;
         send_edges64(r64);
         send_rows(0);

@@ -19,7 +19,7 @@ struct ResSync {
     uint64_t* next;      // [G] the group's current member
     int* queue;          // members taken so far
     int* error;          // a wait timed out
-    unsigned long long limit;  // ticks a wait may take
+    unsigned long long limit;  // ticks a wait may take; it looks at the clock every 1024 polls, 0: at every one
     const int* order;    // [B] the order in which members are taken, or NULL (as they come)
     int G, T, nslots, B;
 };

@@ -34,11 +34,13 @@ __device__ __forceinline__ void get_pair(const uint64_t* p, uint64_t& a, uint64_
     a = (uint64_t)w.y << 32 | w.x;
     b = (uint64_t)w.w << 32 | w.z;
 }
-// Whether a wait that began at t0 (0: now) is to end: it took too long, or another workgroup gave up.
+// Whether a wait that began at t0 (0: now) is to end: it took too long, or another workgroup gave up. The same answer in
+// every lane (one lane's look at the error).
 __device__ __forceinline__ bool gave_up(const ResSync& a, unsigned long long& t0) {
     const unsigned long long now = wall_clock64();
     if (t0 == 0) t0 = now;
-    if (__hip_atomic_load(a.error, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0 && now - t0 <= a.limit) return false;
+    const int error = __hip_atomic_load(a.error, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (__builtin_amdgcn_readfirstlane(error) == 0 && now - t0 < a.limit) return false;
     __hip_atomic_store(a.error, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     return true;
 }
@@ -78,7 +80,7 @@ __device__ __forceinline__ bool wait_words(const ResSync& a, const uint64_t* con
         }
         if (wq) wq = (unsigned)(q0 >> 32) != tag || (unsigned)(q1 >> 32) != tag;
         if (!__any(wait || wq)) break;
-        if ((++spins & 1023u) == 0 && gave_up(a, t0)) return false;
+        if (((++spins & 1023u) == 0 || a.limit == 0) && gave_up(a, t0)) return false;
     }
 #pragma unroll
     for (int i = 0; i < N; ++i)
@@ -104,7 +106,7 @@ __device__ __forceinline__ int next_member(const ResSync& a, int g, int t, unsig
     for (;;) {
         const uint64_t v = get_word(w);
         if ((unsigned)(v >> 32) == members) return (int)(unsigned)v;
-        if ((++spins & 1023u) == 0 && gave_up(a, t0)) return -1;
+        if (((++spins & 1023u) == 0 || a.limit == 0) && gave_up(a, t0)) return -1;
     }
 }
 // Unit of this block: group g, tile t. The blocks of an XCD (b % 8) take consecutive units, tile-major, so that few

@@ -169,3 +169,45 @@ def test_resident_concurrent_streams(problem):
     for k, (x, d) in enumerate(out):
         d.check()
         assert torch.equal(x, runs[k % 3][3]), k
+
+
+GIVING_UP = [("tile", 1), ("fortran", 2), ("tile", 41), ("mixed", 3), ("mixed", 61)]
+
+
+def _giving_up(problem, solve, B):
+    """The call and a switch for how long its waits may take, on an exchanger (and a T plan) of its own."""
+    from mit_jax_amd import _lib, cg2d, mixed
+    from mit_jax_amd.exchange import Exchanger, ExchangeMaps
+    _, cls, slots = problem
+    ex = Exchanger(ExchangeMaps.load())
+    index = np.arange(B, dtype=np.int32) % len(cls)
+    b, x0, norm = _inputs(ex, cls, B, index)
+    kw = dict(cg2dNorm=norm, tolerance=1e-9, max_iters=400, op_index=index)
+    if solve == "mixed":
+        run = lambda **o: mixed.cg2d_mixed(ex, slots, b, x0, **kw, **o)  # noqa: E731
+    else:
+        run = lambda **o: cg2d.cg2d_fortran(ex, slots, b, x0, sum_order=solve, **kw, **o)  # noqa: E731
+
+    def limit(seconds):
+        _lib.check(_lib.lib().mj_halo_plan_set_wait_limit(ex.plan("T", b.device).handle, seconds), "wait limit")
+    return run, limit
+
+
+@pytest.mark.parametrize("solve,B", GIVING_UP)
+def test_resident_ends_when_its_waits_fail(problem, solve, B):
+    """With a limit of 0 the first wait that is not served at once fails, in each workgroup wherever it happens to be: the
+    launch ends all the same (no wave is left at a barrier that the others have passed), and the next solve with the plan
+    is right."""
+    run, limit = _giving_up(problem, solve, B)
+    xr, _ = run(block_threads=512)
+    torch.cuda.synchronize()
+    for _ in range(3):
+        limit(0.0)
+        print(f"resident: {solve} B={B}, waits fail", flush=True)
+        run()
+        torch.cuda.synchronize()
+        limit(20.0)
+        x, d = run()
+        torch.cuda.synchronize()
+        assert int(d["launches"].max()) == 0
+        assert torch.equal(x, xr)

@@ -213,3 +213,15 @@ def test_synthetic_inputs_shape_the_configs():
     assert g.depth.max() <= 6000.0 and g.drF.sum() >= 6000.0
     wet = g.maskC[:, 0, J, I] > 0
     assert abs(tr[:, 0, J, I][wet].mean() - (2 + 25 * np.exp(-(-g.rC[0]) / 800.0))) < 0.01
+
+
+def test_wait_limit_is_checked():
+    """mj_halo_plan_set_wait_limit refuses a missing plan and what is not a time, before it looks at the plan."""
+    import ctypes
+    from mit_jax_amd import _lib
+    L = _lib.lib()
+    plan = ctypes.create_string_buffer(8192)  # stands for a plan: refused calls do not touch it
+    assert L.mj_halo_plan_set_wait_limit(None, 1.0) != 0
+    for s in (-1.0, float("nan"), float("inf"), 1e7):
+        assert L.mj_halo_plan_set_wait_limit(ctypes.cast(plan, ctypes.c_void_p), s) != 0, s
+    assert plan.raw == bytes(8192)
