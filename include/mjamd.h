@@ -82,8 +82,9 @@ int mj_halo_plan_destroy(mj_halo_plan* plan);
 /* 1 when no written point is the source of a written point (T, 3D, UVs, UVn, UV3s): in-place fills are exact. */
 int mj_halo_plan_inplace_ok(const mj_halo_plan* plan);
 /* How long a workgroup of a resident CG2D solve with this (T) plan may wait for another one, in seconds (kept to about
- * a millisecond): 20 unless set, 0 for a wait that is not served at its first look. The launch of a solve in which one waits longer ends early. Takes
- * effect with the next solve; not to be called while another thread enqueues one with the same plan. */
+ * a millisecond): 20 unless set, 0 for a wait that is not served at its first look. The launch of a solve in which one
+ * waits longer ends early, with converged = -2 in every member's record. Takes effect with the next solve; not to be
+ * called while another thread enqueues one with the same plan. */
 int mj_halo_plan_set_wait_limit(mj_halo_plan* plan, double seconds);
 
 /* Geometry of the arrays one halo call covers: element (outer o, tile t, inner n, j, i) lives at
@@ -119,7 +120,7 @@ typedef struct {
     double sumRHS;         /* global sum of the normalised rhs */
     double rhsMax;         /* max |cg2d_b * cg2dNorm| */
     int32_t numIters;      /* iterations done */
-    int32_t converged;     /* 1 if err_sq < tol^2 at exit */
+    int32_t converged;     /* 1 if err_sq < tol^2 at exit; -2 (every member's) if a wait between workgroups failed */
     int32_t outerIters;    /* FP64 residual replacements (mixed precision), 0 for the plain solve */
     int32_t launches;      /* kernel launches of the iteration loop (PHASES modes; the same value in every member's
                               record, written when the loop ends); 0 for the persistent and resident launches */

@@ -46,8 +46,8 @@ class Cg2dParams:
 
 class Cg2dDiag(dict):
     """Per-member diagnostics of a solve (tensors on the device; the reference returns firstResidual,
-    lastResidual, numIters, sumRHS, rhsMax, core/cg2d.py:267-268), plus `converged` (1 / 0; -2 when a device
-    barrier timed out), `outerIters` (FP64 residual replacements of the mixed-precision solve) and `launches` (kernel launches
+    lastResidual, numIters, sumRHS, rhsMax, core/cg2d.py:267-268), plus `converged` (1 / 0; -2 in every
+    record when a wait between workgroups timed out), `outerIters` (FP64 residual replacements of the mixed-precision solve) and `launches` (kernel launches
     of the solve's iteration loop in the per-phase launch modes, the same in every member's record)."""
 
     def __init__(self, raw, batched):
@@ -60,9 +60,9 @@ class Cg2dDiag(dict):
         self.raw = raw
 
     def check(self):
-        """Raise if a device barrier timed out (the launch was abandoned; results are invalid)."""
+        """Raise if a wait between workgroups timed out (the launch was abandoned; results are invalid)."""
         if bool((self["converged"] == -2).any()):
-            raise _lib.MjError("cg2d: a device grid barrier timed out")
+            raise _lib.MjError("cg2d: a wait between workgroups timed out")
         return self
 
 

@@ -666,8 +666,6 @@ __global__ void __launch_bounds__(kThreads, 2) cg2d_resident_kernel(ResDev a) {
         }
         __syncthreads();  // every wave has looked at s_bad; the next member's first wait may set it
     }
-    // a wait timed out: every member's record says so
-    for (int m = blockIdx.x * kThreads + tid; m < a.B; m += gridDim.x * kThreads) a.diag[m].converged = -2;
 }
 
 __global__ void res_init_kernel(uint64_t* words, size_t n, int* queue, int* error) {
@@ -677,6 +675,13 @@ __global__ void res_init_kernel(uint64_t* words, size_t n, int* queue, int* erro
         *queue = 0;
         *error = 0;
     }
+}
+
+// After a launch in which a wait failed, every member's record says so. Not the launch's own business: its workgroups end
+// one by one, and one that was served in time may still write a record after the others have left.
+__global__ void __launch_bounds__(256) res_failed_kernel(const int* error, mj_cg2d_diag* diag, int B) {
+    if (*error == 0) return;
+    for (int m = threadIdx.x; m < B; m += 256) diag[m].converged = -2;
 }
 
 // The order in which a batch with several operators is taken: the members that need most iterations first, so that the
@@ -772,6 +777,14 @@ int resident_prepare(const mj_halo_plan* P, const mj_cg2d_ops* ops, const mj_cg2
     return MJ_OK;
 }
 
+int resident_launch(const void* kfn, int threads, void** args, size_t lds, const ResSync& y, mj_cg2d_diag* diag,
+                    hipStream_t st) {
+    MJ_HIP(hipLaunchCooperativeKernel(kfn, dim3(y.G * y.T), dim3(threads), args, (unsigned)lds, st));
+    hipLaunchKernelGGL(res_failed_kernel, dim3(1), dim3(256), 0, st, y.error, diag, y.B);
+    MJ_HIP(hipGetLastError());
+    return MJ_OK;
+}
+
 int stream_capturing(hipStream_t st, bool* capturing) {
     hipStreamCaptureStatus s = hipStreamCaptureStatusNone;
     MJ_HIP(hipStreamIsCapturing(st, &s));
@@ -792,7 +805,7 @@ int resident_solve(mj_halo_plan* P, const mj_cg2d_ops* ops, const double* b, con
     const size_t lds = (cfg->sum_order == MJ_SUM_FORTRAN ? kLdsFort : kLdsTree) * sizeof(double);
     ResDev a{};
     bool ok = false;
-    const int rc = resident_prepare(P, ops, cfg, kfn, kThreads, lds, workspace, workspace_bytes, st, &a.y, &ok);
+    int rc = resident_prepare(P, ops, cfg, kfn, kThreads, lds, workspace, workspace_bytes, st, &a.y, &ok);
     if (rc || !ok) return rc;
     a.B = cfg->batch;
     a.ms = cfg->member_stride;
@@ -818,7 +831,7 @@ int resident_solve(mj_halo_plan* P, const mj_cg2d_ops* ops, const double* b, con
     a.pub = P->res_pub;
     a.diag = diag;
     void* args[] = {(void*)&a};
-    MJ_HIP(hipLaunchCooperativeKernel(kfn, dim3(a.y.G * a.y.T), dim3(kThreads), args, (unsigned)lds, st));
+    if ((rc = resident_launch(kfn, kThreads, args, lds, a.y, diag, st))) return rc;
     *done = true;
     return MJ_OK;
 }

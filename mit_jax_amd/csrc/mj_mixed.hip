@@ -898,8 +898,7 @@ int mx_resident_solve(const MxDev& a, const mj_halo_plan* P, const mj_cg2d_ops* 
     if ((rc = mx_convert(a, ops, nslots, st))) return rc;
     MxDev d = a;
     void* args[] = {(void*)&d, (void*)&q};
-    MJ_HIP(hipLaunchCooperativeKernel(kfn, dim3(q.y.G * q.y.T), dim3(64 * F::kWaves), args, (unsigned)lds, st));
-    return MJ_OK;
+    return resident_launch(kfn, 64 * F::kWaves, args, lds, q.y, a.diag, st);
 }
 
 }  // namespace

@@ -24,10 +24,13 @@ struct ResSync {
     int G, T, nslots, B;
 };
 // Fills y for a cooperative launch of kfn (threads, dynamic LDS) over cfg's batch and clears its words on the stream;
-// *ok false (and nothing enqueued) when the device or the workspace does not allow it. The launch has y->G * T blocks.
+// *ok false (and nothing enqueued) when the device or the workspace does not allow it.
 int resident_prepare(const mj_halo_plan* P, const mj_cg2d_ops* ops, const mj_cg2d_config* cfg, const void* kfn,
                      int threads, size_t lds, void* workspace, size_t workspace_bytes, hipStream_t st, ResSync* y,
                      bool* ok);
+// The launch of kfn (y.G * y.T blocks); diag's records say -2 if a wait in it failed.
+int resident_launch(const void* kfn, int threads, void** args, size_t lds, const ResSync& y, mj_cg2d_diag* diag,
+                    hipStream_t st);
 // Whether a stream is being captured into a graph (the resident launches are not for that).
 int stream_capturing(hipStream_t st, bool* capturing);
 

@@ -211,3 +211,23 @@ def test_resident_ends_when_its_waits_fail(problem, solve, B):
         torch.cuda.synchronize()
         assert int(d["launches"].max()) == 0
         assert torch.equal(x, xr)
+
+
+@pytest.mark.parametrize("solve,B", GIVING_UP)
+def test_resident_failed_waits_are_reported(problem, solve, B):
+    """A solve whose waits failed says so in every member's record (the sums that it did not get read as 0, which must not
+    pass for a residual), whatever the buffer held before, and the next solve does not."""
+    from mit_jax_amd import _lib
+    run, limit = _giving_up(problem, solve, B)
+    for _ in range(3):
+        limit(0.0)
+        print(f"resident: {solve} B={B}, waits fail", flush=True)
+        _, d = run()
+        torch.cuda.synchronize()
+        assert bool((d["converged"] == -2).all()), d["converged"]
+        with pytest.raises(_lib.MjError, match="timed out"):
+            d.check()
+        limit(20.0)
+        _, d = run()
+        torch.cuda.synchronize()
+        assert bool((d.check()["converged"] >= 0).all())
