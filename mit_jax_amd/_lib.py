@@ -181,15 +181,15 @@ def ptr(t):
 
 
 def to_device_f64(arrays, device):
-    """Copies of host vectors (numpy, float64) on the device, for the current stream, by launches that carry them as
-    arguments (mj_put_doubles). A copy each, out of pageable memory, waits for all work queued before it (some 15 us each,
-    and the queue is empty behind it): five of them in a DST3 call held up one member's 200 us of kernels by 90 us. One
-    copy out of pinned memory does not wait, but takes 60 us more than this on a queue that is empty."""
+    """Copies of host vectors (float64, or what numpy converts to it) on the device, for the current stream, by launches
+    that carry them as arguments (mj_put_doubles). A copy each, out of pageable memory, waits for all work queued before it
+    (some 15 us each, and the queue is empty behind it): five of them in a DST3 call held up one member's 200 us of kernels
+    by 90 us. One copy out of pinned memory does not wait, but takes 60 us more than this on a queue that is empty."""
     index = torch.device(device).index
     if not arrays or torch.cuda.is_current_stream_capturing() or \
             (index is not None and index != torch.cuda.current_device()):
         return [torch.as_tensor(np.asarray(a, dtype=np.float64).reshape(-1), device=device) for a in arrays]
-    host = np.concatenate(arrays, axis=None, dtype=np.float64)
+    host = np.concatenate(arrays, axis=None, dtype=np.float64, casting="unsafe")  # as np.asarray converts
     out = torch.empty(host.size, dtype=torch.float64, device=device)
     check(lib().mj_put_doubles(host.ctypes.data, host.size, out.data_ptr(), stream_ptr()), "mj_put_doubles")
     return out.split([np.size(a) for a in arrays])

@@ -144,3 +144,14 @@ def test_host_vectors_to_device(dev, monkeypatch):
     monkeypatch.setattr(torch, "empty", None)
     for a, r in zip(_lib.to_device_f64(src, dev), [np.array(a, dtype=np.float64).reshape(-1) for a in src]):
         assert np.array_equal(a.cpu().numpy(), r)
+
+
+@pytest.mark.parametrize("vector", [np.array([1, 2.5, 3.25], dtype=object), ["1", "2.5", "3.25"],
+                                    np.array([1.0, 2.5, 3.25], dtype=np.longdouble), [np.float32(1.0), 2.5, 3.25]])
+def test_host_vectors_that_numpy_converts(dev, vector):
+    """_lib.to_device_f64 takes every vector that np.asarray(v, float64) does (objects and texts among them), as the level
+    vectors' arguments always did."""
+    from mit_jax_amd import _lib
+    got = _lib.to_device_f64([vector, np.arange(2.0)], dev)
+    assert np.array_equal(got[0].cpu().numpy(), [1.0, 2.5, 3.25])
+    assert np.array_equal(got[1].cpu().numpy(), [0.0, 1.0])
