@@ -13,10 +13,12 @@ The headline (default) is the mixed-precision solve (FP32 PCG + FP64 residual re
 FP64 solve (mj_cg2d_solve) is timed on the same step for `mixed_over_fp64`, and the two solutions are compared
 member by member (`error_vs_fp64`). Prints one JSON line.
 
-`roofline` is the solve's kernel, from the solve alone on its stream (eager, not overlapped), timed with HIP events (a
-resident launch keeps the vectors on chip: its `achieved` exceeds the bytes it moves): achieved = algorithmic bytes per launch /
-average launch duration (= the solve's algorithmic bytes / its time; the average includes the few setup kernels and the launch gaps, so it is an upper bound
-of the profiler's per-kernel average). Algorithmic bytes are what the recurrence itself must move, per interior
+`roofline` is the solve's kernel, from the solve alone on its stream (eager, not overlapped), timed with HIP events.
+Launches that stream the vectors are bound by HBM: achieved = algorithmic bytes per launch / average launch duration
+(= the solve's algorithmic bytes / its time; the average includes the few setup kernels and the launch gaps, so it is an
+upper bound of the profiler's per-kernel average). A resident launch keeps the vectors on chip and is bound by the latency
+of its exchanges ("bound": "latency"): achieved and frac are those of the bytes it moves (`traffic`; null where that is not
+measured), and `algorithmic_GBs`, the recurrence's bytes over the time, is no bandwidth. Algorithmic bytes are what the recurrence itself must move, per interior
 point (N2 = 105,300 per member): per member-iteration the vectors r, s, x read and written (6 streams of s_v bytes);
 per operator slot and iteration in which any member of the slot iterates, the six operator and preconditioner arrays
 (6 x s_c); per FP64 residual replacement of the mixed solve 64 B (the FP64 true residual and solution update); s_v = s_c = 4 for
@@ -452,7 +454,8 @@ def kernel_times(st, reps=3):
 
 
 def roofline_of(precision, cg_ms, d, op_index, members, launch):
-    """The `roofline` object of a solve timed alone (cg_ms) with diagnostics d."""
+    """The `roofline` object of a solve timed alone (cg_ms) with diagnostics d. A resident launch does not move the
+    recurrence's bytes: what it achieves is counted from the measured ones."""
     alg, impl, slot_iters = solve_bytes(precision, d, op_index)
     launches = int(d["launches"].max())  # 0: one launch, persistent or resident
     if precision == "fp64":
@@ -460,10 +463,14 @@ def roofline_of(precision, cg_ms, d, op_index, members, launch):
             "cg2d_persistent_kernel" if launch == "persistent" else "cg2d_resident_kernel"
     else:
         kernel = "mx_step_kernel" if launches else "mx_resident_kernel"
-    achieved = alg / (cg_ms * 1e-3) / 1e9
+    resident = kernel in ("cg2d_resident_kernel", "mx_resident_kernel")
     tr = measured_traffic(kernel, members)
-    return {"bound": "hbm", "kernel": kernel, "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
-            "frac": achieved / HBM_PEAK_GBS, "traffic": tr, "traffic_source": traffic_source(kernel) if tr else None,
+    moved = tr if resident else alg
+    achieved = moved / (cg_ms * 1e-3) / 1e9 if moved else None
+    return {"bound": "latency" if resident else "hbm", "kernel": kernel, "achieved": achieved, "peak": HBM_PEAK_GBS,
+            "unit": "GB/s", "frac": achieved / HBM_PEAK_GBS if moved else None,
+            "algorithmic_GBs": alg / (cg_ms * 1e-3) / 1e9,
+            "traffic": tr, "traffic_source": traffic_source(kernel) if tr else None,
             "launches": launches, "avg_launch_us": cg_ms * 1e3 / launches if launches else None,
             "algorithmic_bytes_per_launch": alg / launches if launches else None, "algorithmic_bytes": alg,
             "operator_slot_iterations": slot_iters, "solve_ms": cg_ms,
