@@ -373,8 +373,8 @@ __device__ __forceinline__ double level_value(const double* p, int k) {
 //
 // Bound by HBM: a unit moves seven planes (540 KB, 28 us of a CU's share) and takes 37 us, of which some 4 are phases
 // without loads; one member of 50 levels is 650 units on 256 CUs. Evaluating both faces at each of ten points a thread, all
-// loads of a point behind one another, took 136 us for it (122 now) and 1700 us for 24 members of mixed level counts (1615
-// now). One row ahead instead of two measured 3 % more for both, four 8 % more for the members. recip_rA and maskInC are
+// loads of a point behind one another, took 136 us for it (120 now) and 1700 us for 24 members of mixed level counts (1510
+// now, 3.7 TB/s). One row ahead instead of two measured 3 % more for both, four 8 % more for the members. recip_rA and maskInC are
 // read from their own planes, where half of a pair would be thrown away: a row's loads are 40 bytes instead of 48 (the whole
 // step 152 -> 146 us and 3.05 -> 2.95 ms). maskInC as bits, 32 bytes, gave nothing more, nor did loading a sweep's first rows
 // before the barriers in front of it (149 us).
@@ -626,7 +626,7 @@ __global__ void __launch_bounds__(kHzThreads, 3) gad_hz_kernel(GadDev a) {
 // ------------------------------------------------------------------------------------------------ reverse mode
 constexpr int kAdjChunk = 1024;  // (member, tile, level)s per reverse launch, in whole columns (at least one)
 constexpr int kAdjSnaps = 5;     // snapshots of one: six sweeps, the first from the tracer itself
-constexpr int kAdjPlanes = 7;    // planes of one that the workspace allows for
+constexpr int kAdjPlanes = 7;    // planes of one in the workspace query's answer, which callers know; kAdjSnaps are used
 // Partial derivatives of one DST3 interface value f = A (t_m1 + d0 Rj + d1 Rjm) + Bm (t_0 - d0 Rj - d1 Rjp)
 // (A = (tr + |tr|)/2, Bm = (tr - |tr|)/2, d0 = (2-c)(1-c)/6, d1 = (1-c^2)/6): w[0..3] = df/dt_m2, df/dt_m1,
 // df/dt_0, df/dt_p1 (independent of the tracer), dtr = df/dtr, dc = df/dcfl. The derivative of |x| at 0 is taken
@@ -687,19 +687,20 @@ __global__ void __launch_bounds__(kHzThreads, 3) gad_hz_snap_kernel(GadDev a, in
 // With lbar (the R flux's reverse mode) the sweeps start from lbar, the cotangent of localTij after the horizontal passes,
 // instead of from gbar, and the tracer cotangent already holds the vertical part (added to, not set).
 //
-// Thread (seg, col) = (tid / 98, tid % 98) owns the rows 14 seg .. 14 seg + 13 of column col. Every face's partials are evaluated once, by its owner: in X the four points that they go to take them from
-// the lanes beside (DPP shifts; the three faces beside a wave's 64 points are evaluated by lanes 3 r + 0 .. 2 for row r),
-// in Y a thread walks up its column and evaluates the faces of three rows more. The update's cotangents are formed from
-// localTij's cotangent before a barrier, which is then updated in place behind it. LDS: the tile and that cotangent,
-// 154 KB, one workgroup of 11 waves a CU.
+// Thread (seg, col) = (tid / 98, tid % 98) owns the rows 14 seg .. 14 seg + 13 of column col. Every face's partials are
+// evaluated once, by its owner: in X the four points that they go to take them from the lanes beside (DPP shifts; the three
+// faces beside a wave's 64 points are evaluated by lanes 3 r + 0 .. 2 for row r), in Y a thread walks up its column and
+// evaluates the faces of three rows more. The update's cotangents are formed from localTij's cotangent before a barrier,
+// which is then updated in place behind it. LDS: the tile and that cotangent, 154 KB, one workgroup of 11 waves a CU.
 //
 // What a row reads from memory is loaded a row ahead, and no row has a branch: the loads of all rows issued together spill,
-// and a load issued behind a row's stores waits for them too (both count in order). Bound by HBM (15 planes of 77 KB a unit,
-// 59 us of a CU's share for two sweeps) and the rounds of 650 units on 256 CUs; it reaches 85 us a unit.
+// and a load issued behind a row's stores waits for them too (both count in order). Bound by HBM (one
+// member of 50 levels moves 1.13 GB, 22 planes of 77 KB a unit of two or three sweeps, at 3.9 TB/s) and the rounds of its
+// 650 units on 256 CUs, the last one half empty.
 //
 // Evaluating all five partials that a point needs, with a second flux plane and no more than a point's loads in flight,
 // took 958 us for one member of 50 levels together with the replay of the forward sweeps (two of three, each with a
-// snapshot); 291 us now, and 152 us for the replay, whose launch with the R flux also makes the localTij that took another
+// snapshot); 291 us now, and 128 us for the replay, whose launch with the R flux also makes the localTij that took another
 // 136 us. Ten rows a thread (1024 threads, 128 VGPRs) and twenty (512, 256) measured 540 to 560 us in the form without the
 // loads ahead, as did fourteen; two rows ahead spill (400 us).
 constexpr int kAdjRows = 14, kAdjSegs = GNY / kAdjRows, kAdjThreads = 704;
@@ -997,8 +998,7 @@ __global__ void __launch_bounds__(kAdjThreads, 3)
 //
 // Bound by HBM: one walk down the column, step k takes level k in, evaluates interface k - 1 and completes level k - 2; the
 // level data are loaded kVertAhead steps ahead. With one step's loads in flight one member of 50 levels (300 MB) took 98 us;
-// 75 us now, 4 TB/s. 24 members, which fill the card by themselves, take 1.01 ms either way (5.1 TB/s with the masks that
-// members share). One, two and four steps ahead measure the same, six 2 us more.
+// 75 us now, 4 TB/s. 24 members, which fill the card by themselves, take 1.01 ms either way (4.6 TB/s). One, two and four steps ahead measure the same, six 2 us more.
 constexpr int kVertAhead = 2;
 __global__ void __launch_bounds__(256) gad_vert_kernel(GadDev a, const double* __restrict__ loc_h) {
     const int q = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1076,7 +1076,7 @@ __global__ void __launch_bounds__(256) gad_vert_kernel(GadDev a, const double* _
 // One walk down the column: step k takes level k in, evaluates interface k - 1 (which reads the levels k - 3 .. k) and
 // writes what is complete, so each of the six arrays is read once and each of the three written once; the level data are
 // loaded kVertAhead steps ahead. Bound by HBM: reading them as needed, with locbar updated in memory, took 240 us for one
-// member of 50 levels; 82 us now (450 MB, 5.5 TB/s).
+// member of 50 levels; 84 us now (470 MB, 5.6 TB/s).
 __global__ void __launch_bounds__(256) gad_vert_adjoint_kernel(GadDev a, int col0, const double* __restrict__ loc_h,
                                                                const double* __restrict__ gbar,
                                                                double* __restrict__ locbar, double* __restrict__ trb,

@@ -416,16 +416,14 @@ extern "C" int mj_gad_implicit_r(const mj_impr_grid* g, const mj_impr_config* c,
 // cotangents), three written. Reading the level data as needed kept one or two loads in flight per lane (772 us for two
 // members of 50 levels, 1.7 TB/s of these twelve passes); now both walks run on register rings that load kPfA levels
 // ahead, in laps of kPfA rows without branches, and the parameter cotangents of interface m + 1 are formed as soon as
-// lam(m) is known, so that lam is not read back: 252 us, 4.8 TB/s, where a copy reaches 4.65 and reads alone 6. Six levels
+// lam(m) is known, so that lam is not read back: 250 us, 5.0 TB/s, where a copy reaches 4.65 and reads alone 6. Six levels
 // ahead: four and eight measured within the spread of the runs, and eight no longer fit the registers. For the LLC90 level
-// count the walks are unrolled and y' stays in registers (NR; else it makes a round trip through the output column).
+// count, as in the forward solve, the walks are unrolled and y' stays in registers (NR). Other counts send it through the
+// output column: 74, 167 and 320 us for 15, 30 and 49 levels, and 323 us for 50.
 namespace mj {
 namespace {
 
-#ifndef MJ_IMPR_PFA
-#define MJ_IMPR_PFA 6
-#endif
-constexpr int kPfA = MJ_IMPR_PFA;
+constexpr int kPfA = 6;
 static_assert(kPfA >= 4, "the rings must hold the levels of a row");
 
 struct Row {

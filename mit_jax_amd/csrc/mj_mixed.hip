@@ -1011,7 +1011,10 @@ extern "C" int mj_cg2d_solve_mixed(const mj_halo_plan* plan_T, const mj_cg2d_ops
         if ((rc = stream_capturing(st, &capturing))) return rc;
         // MrOne up to 16/7 members per place (45 of 19 places on 256 CUs with 13 tiles), MrTwo beyond: with mixed level
         // counts one / two workgroups per CU take 2.07 / 2.72 ms for 20 members, 3.14 / 3.23 for 39, 3.16 / 3.29 for 45,
-        // 3.51 / 3.29 for 49, 3.85 / 3.30 for 57, 8.5 / 7.0 for 128 (the step launches 6.8, 7.9, -, -, 10.0, 18.7)
+        // 3.51 / 3.29 for 49, 3.85 / 3.30 for 57, 8.5 / 7.0 for 128 (the step launches 6.8, 7.9, -, -, 10.0, 18.7).
+        // The line is that of mixed counts. Members of one level count end together and take whole rounds: 50 levels 3.56 /
+        // 2.95 ms for 20 members, 5.29 / 3.24 for 39, 5.39 / 6.15 for 45, 5.37 / 6.31 for 46, 7.10 / 6.40 for 58,
+        // 12.5 / 12.5 for 128, so there the line costs up to 1.6 times at 39 members and 1.2 times from 46 to 57.
         auto* const solve = 7 * (int64_t)a.B * a.T <= 16 * (int64_t)ncu ? mx_resident_solve<MrOne> : mx_resident_solve<MrTwo>;
         if (!capturing && (rc = solve(a, P, ops, cfg, nslots, w + L.r0, L.coef - L.r0, st, &done))) return rc;
         if (done) return MJ_OK;
